@@ -740,7 +740,6 @@ void solve_nr(Batch& bt, Context& ctx, const SolveOptions& opt, const double* b,
     ctx.sweep_mode = saved_mode;
     ctx.sync.waves_per_cu = saved_waves;
     ctx.sync.level_order = saved_order;
-    ctx.sync.cooperative = true;
   };
   try {
     ctx.sync.ensure(im.fwd.nsup, s);
@@ -790,7 +789,6 @@ void solve_nr(Batch& bt, Context& ctx, const SolveOptions& opt, const double* b,
       if (!valid) {
         bt.graph.reset(new BatchGraph());
         g = bt.graph.get();
-        ctx.sync.cooperative = false;
         CaptureGuard capture;  // no set-up HIP calls of other threads until instantiation
         BCM_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         try {
@@ -803,7 +801,6 @@ void solve_nr(Batch& bt, Context& ctx, const SolveOptions& opt, const double* b,
         }
         BCM_HIP(hipStreamEndCapture(s, &g->g));
         BCM_HIP(hipGraphInstantiate(&g->exec, g->g, nullptr, nullptr, 0));
-        ctx.sync.cooperative = true;
         g->nrhs = NR; g->prec = opt.prec; g->iters = every; g->sweep_mode = tu.sweep_mode;
         g->waves = tu.waves_per_cu; g->order = tu.level_order; g->flex = flex; g->niter = opt.niter; g->ittype = opt.ittype; g->eps = opt.eps;
         g->key = key;
@@ -876,8 +873,7 @@ void batch_solve(Batch& bt, Context& ctx, const SolveOptions& opt, int nrhs, con
     }
     BCM_HIP(hipStreamSynchronize(ctx.stream));
   };
-  // Sync-free sweeps rely on every wave being resident; a dependency wait
-  // that reaches its bound (part of the GPU held by another process) leaves
+  // A dependency wait of a sync-free sweep that reaches its bound leaves
   // its sweep unfinished and raises the error flag. The solve is then
   // repeated from x0 with level-scheduled sweeps, which never wait.
   const bool syncfree = bt.tune.sweep_mode != 0;
@@ -911,7 +907,7 @@ void batch_solve(Batch& bt, Context& ctx, const SolveOptions& opt, int nrhs, con
 
 BatchTune batch_tune(Batch& bt, Context& ctx, const SolveOptions& opt, int nrhs, const double* b, bool allow_graph) {
   // Two stages: the sweep schedule (level-scheduled, or sync-free with a row
-  // order and a launch shape) with eager launches, then graph replay and the
+  // order) with eager launches, then graph replay and the
   // polling interval for the winner. Every candidate runs the same fixed
   // number of iterations (tolerance 0) from x0 = 0.
   const size_t vb = (size_t)bt.n * nrhs * 8;
@@ -941,12 +937,10 @@ BatchTune batch_tune(Batch& bt, Context& ctx, const SolveOptions& opt, int nrhs,
     t.sweep_mode = 0;
     stage1.push_back(t);
     t.sweep_mode = 1;
-    for (int order = 0; order <= 1; ++order)
-      for (int waves : {4, 8, 16}) {
-        t.level_order = order;
-        t.waves_per_cu = waves;
-        stage1.push_back(t);
-      }
+    for (int order = 0; order <= 1; ++order) {
+      t.level_order = order;
+      stage1.push_back(t);
+    }
   }
   BatchTune best = keep;
   best.ms_per_iter = 1e300;

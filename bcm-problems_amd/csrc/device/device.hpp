@@ -152,16 +152,14 @@ void dev_tri_forward_parts(const std::vector<const BlockCsr*>& f, int prec, DevT
 void dev_tri_backward_parts(const std::vector<const BlockCsr*>& f, int prec, DevTri& t);
 
 // State of the sync-free sweeps on one stream: ctl[2] is the error flag (a
-// dependency wait reached its bound). Launch shape: at most waves_per_cu resident waves
-// per CU (never more than the occupancy limit), launched cooperatively
-// (residency guaranteed by the runtime) or, for stream capture into a graph,
-// as an ordinary launch of a grid that fits the device at once.
+// dependency wait reached its bound), ctl[4] the ticket counter of the running
+// sweep. Sweeps are ordinary launches: workgroups draw their rows in
+// topological order, so they need no co-residency.
 struct SweepSync {
   DevBuf ctl;
   int* ext_ctl = nullptr;  // caller-provided control words (at least 16 ints, zeroed) used instead of ctl
   int nsup = 0;
-  int waves_per_cu = 8;
-  bool cooperative = true;
+  int waves_per_cu = 8;     // accepted bound on the resident waves per CU
   bool level_order = true;  // process rows sorted by dependency level (false: natural sweep order)
   void ensure(int nsup, hipStream_t s);
   int error(hipStream_t s);
@@ -217,6 +215,14 @@ void launch_spmv(const DevBsr& A, const double* x, double* y, const double* bsub
 // launch using `sync`. x and y must not alias.
 void launch_sweep(const DevTri& T, const void* x, void* y, int vec_prec, int nrhs, hipStream_t s,
                   const int* skip = nullptr, SweepSync* sync = nullptr, RowGate gate = RowGate());
+
+// Both sweeps of a preconditioner, z = T2^-1 T1^-1 r on FP64 vectors r and z,
+// with the factors' precision and vectors of vec_prec in between. w0 (and w1,
+// for FP32 vectors) hold n * nrhs values of vec_prec. Sync-free sweeps over
+// one block size take one launch for both, which also converts; else as
+// launch_sweep twice. r and z may be the same vector.
+void launch_sweep_pair(const DevTri& T1, const DevTri& T2, const double* r, double* z, void* w0, void* w1,
+                       int vec_prec, int nrhs, hipStream_t s, const int* skip = nullptr, SweepSync* sync = nullptr);
 
 // out[k] = sum_i x_k[i] * y_k[i] for K pairs (K <= kMaxDots), one pass plus a
 // finalize launch; with out == kDeferred the partials stay pending in rw.

@@ -656,29 +656,39 @@ __global__ __launch_bounds__(256) void k_sweep_level(int nrows, const int* __res
 }
 
 // ---------------------------------------------------------------------------
-// Sync-free triangular sweep (one cooperative launch per sweep). Wave w owns
-// positions w, w+W, w+2W, ... of a topological order of the rows -- the
-// natural sweep order, or the rows sorted by dependency level, which
-// interleaves independent chains (e.g. the cells of a block-diagonal union)
-// -- and processes them in that order; every wave of the grid is resident
-// (cooperative launch), so the smallest unfinished position always belongs
-// to a wave whose dependencies are complete and the sweep cannot deadlock.
+// Sync-free triangular sweeps: one launch for a sweep, or for the forward and
+// the backward sweep of a preconditioner together. The rows form a sequence of
+// positions in a topological order -- the natural sweep order, or the rows
+// sorted by dependency level, which interleaves independent chains (e.g. the
+// cells of a block-diagonal union); the positions of the second sweep follow
+// those of the first. A workgroup draws one ticket when it starts and its
+// kSweepWaves waves process kSweepWaves consecutive positions, one each.
+// Tickets are drawn in position order by workgroups that already run, so the
+// smallest unfinished position always belongs to a running wave whose
+// dependencies are complete: the sweep ends whatever else occupies the GPU and
+// needs no co-residency (a cooperative launch costs 22 us per sweep in queue
+// hand-overs). One ticket for 8 rows because same-address atomics across the
+// XCDs serialise at 11 ns each.
 //
-// The output vector is its own completion record: before the sweep it is
-// filled with a sentinel NaN pattern that no arithmetic produces (a signaling
-// NaN with a fixed payload); a row's values are final once they differ from
-// it. A wave puts its row's factor columns in flight, stages the values of
-// the rows it depends on through LDS (each value loaded once; the ones still
-// holding the sentinel re-polled, bounded, until a wave vote finds none),
-// computes, and stores its row. Values cross XCDs through
+// The output vectors are their own completion record: before the launch they
+// are filled with a sentinel NaN pattern that no arithmetic produces (a
+// signaling NaN with a fixed payload); a row's values are final once they
+// differ from it. A wave puts its row's factor columns in flight, stages the
+// values of the rows it depends on (and, in the second sweep, its right-hand
+// side, which is the first sweep's output) through LDS -- each value loaded
+// once; the ones still holding the sentinel re-polled, bounded, until a wave
+// vote finds none -- computes, and stores its row. Values cross XCDs through
 // device-scope relaxed atomic loads/stores (coherent across the 8 L2s, the
 // protocol rocPRIM's look-back scan uses on gfx942/gfx950); there is no
 // separate flag and no fence on the critical path. A wait that exceeds its
 // bound raises ctl[2], which stops every other wait; the host reports it.
 //
-// The row loop is wave-uniform (blockIdx/gridDim scalars) and every wait
-// ends on a wave vote; lane-divergent code inside holds no cross-lane
-// operation.
+// What bounds it: a single system's sweep is a chain of dependency levels,
+// each one hand-over (0.4-0.6 us between two waves through the coherent
+// stores and polls) plus the row's arithmetic on one wave. So every
+// load that does not depend on the wait is issued before it, all of a row's
+// dependencies (up to two chunks) are polled together, and the multiply runs
+// without branches on zero-padded chunks.
 template <class T> struct Sentinel;
 template <> struct Sentinel<double> {
   using Bits = unsigned long long;
@@ -695,53 +705,107 @@ __device__ __forceinline__ bool is_sentinel(TX v) {
   return __builtin_bit_cast(Bits, v) == Sentinel<TX>::bits;
 }
 
+constexpr int kSweepWaves = 8;    // waves (rows) per workgroup
+constexpr int kSweepTicket = 4;   // ctl word of the ticket counter (its own use: ctl[2] is the error flag)
+
+// Sentinel into the output vectors of the sweeps to come, ticket counter to 0.
 template <class TX>
-__global__ void k_sweep_fill(int64_t n, TX* __restrict__ y, const int* skip) {
+__global__ void k_sweep_fill(int64_t n, TX* __restrict__ y0, TX* __restrict__ y1, int* ctl, const int* skip) {
   if (skip && *skip) return;
   using Bits = typename Sentinel<TX>::Bits;
-  Bits* yb = reinterpret_cast<Bits*>(y);
+  Bits* b0 = reinterpret_cast<Bits*>(y0);
+  Bits* b1 = reinterpret_cast<Bits*>(y1);
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) yb[i] = Sentinel<TX>::bits;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    b0[i] = Sentinel<TX>::bits;
+    if (b1) b1[i] = Sentinel<TX>::bits;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) ctl[kSweepTicket] = 0;
 }
 
-// Stages the values of dependency blocks kb0 .. kb0+nb-1 of a row (block
-// columns ja[jb + k], every right-hand side) into ys[((k - kb0) * NR + q) * B
-// + c]. Each value is loaded once, by one of the 64 lanes (the columns a lane
-// multiplies are shared by the B lanes of its column group, so loading them
-// per lane would repeat every load B times), and the lanes re-poll the values
-// still holding the sentinel until a wave vote finds none: one coherent round
-// trip once the dependency rows are done, and a waiting wave polls only the
-// values it still lacks. The loop exit is a wave vote (uniform); a wait past
-// its bound raises ctl[2], which ends every other wait.
-template <int B, int NR, int KD, class TX>
-__device__ __forceinline__ void stage_deps(int kb0, int nb, int jb, const int* __restrict__ ja, TX* y, int n,
-                                           TX* ys, int* ctl) {
-  constexpr int SV = KD * B * NR, SJ = (SV + 63) / 64;
-  const int lane = threadIdx.x;
-  const int nv = nb * B * NR;
-  int64_t src[SJ];  // element offsets in y (-1: beyond the chunk)
+// One direction of a sweep launch: the factor image and the row order.
+struct SweepDir {
+  const int* order;  // rows by level, or null: the natural order of the direction
+  const int* ia;
+  const int* ja;
+  const void* off;
+  const void* diag;
+  int forward;
+};
+
+// A sweep launch: `phases` sweeps (1 or 2) over npos = nsup * ng positions
+// each; position p is block row p / ng (in the order of its direction) and
+// column group p % ng of NR columns. Phase 0 reads x (doubles if x64, else
+// vector values) and writes y0; phase 1 reads y0 and writes y1, and out (as
+// doubles) if given.
+template <class TX>
+struct SweepJob {
+  int nsup, n, ng, npos, phases, x64;
+  int fixed;  // 1: positions by workgroup index (every dependency is complete before the launch)
+  SweepDir d0, d1;
+  const void* x;
+  TX* y0;
+  TX* y1;
+  double* out;
+  int* ctl;
+  const int* skip;
+};
+
+// Draws the workgroup's ticket; returns this wave's position (-1: past the end).
+template <class TX>
+__device__ __forceinline__ int sweep_position(const SweepJob<TX>& jb) {
+  __shared__ int ticket;
+  if (threadIdx.x == 0)
+    ticket = jb.fixed ? (int)blockIdx.x
+                      : __hip_atomic_fetch_add(&jb.ctl[kSweepTicket], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const int pos = __builtin_amdgcn_readfirstlane(ticket * kSweepWaves + (int)(threadIdx.x >> 6));
+  return pos < jb.npos * jb.phases ? pos : -1;
+}
+
+// Stages nd (<= KM) dependency blocks of a row (block rows cols[0..nd) of y,
+// NR columns of leading dimension n) into s[((1 + k) * B + c) * NR + q], and
+// with row >= 0 the row's right-hand side into block 0 of s: x (already a
+// complete vector; doubles if x64) or, when xw is given, the row of xw, waited
+// for like a dependency. Blocks nd .. npad-1 are zero-filled. Each value is
+// loaded once, by one of the 64 lanes, and the lanes re-poll the values still
+// holding the sentinel until a wave vote finds none. The loop exit is a wave
+// vote (uniform); a wait past its bound raises ctl[2], which ends every other
+// wait.
+template <int B, int NR, int KM, class TX>
+__device__ __forceinline__ void stage_deps(int nd, int npad, const int* __restrict__ cols, TX* y, int n, int row,
+                                           const void* x, int x64, TX* xw, TX* s, int* ctl) {
+  constexpr int M = B * NR, SJ = ((1 + KM) * M + 63) / 64;
+  const int lane = threadIdx.x & 63;
+  const TX* src[SJ];  // polled values (null: not polled)
   TX val[SJ];
   bool ok = true;
 #pragma unroll
   for (int j = 0; j < SJ; ++j) {
-    const int e = lane + 64 * j;
-    src[j] = -1;
+    const int e = lane + 64 * j, kk = e / M, rem = e - kk * M, q = rem / B, c = rem - q * B;
+    src[j] = nullptr;
     val[j] = TX(0);
-    if (e < nv) {
-      const int k = e / (B * NR), rem = e - k * (B * NR), q = rem / B, c = rem - q * B;
-      src[j] = (int64_t)q * n + (int64_t)ja[jb + kb0 + k] * B + c;
-      val[j] = ld_coherent(y + src[j]);
-      ok = ok && !is_sentinel(val[j]);
+    if (kk == 0 && row >= 0) {
+      const size_t xo = (size_t)q * n + (size_t)row * B + c;
+      if (xw) src[j] = xw + xo;
+      else val[j] = x64 ? (TX) static_cast<const double*>(x)[xo] : static_cast<const TX*>(x)[xo];
+    } else if (kk > 0 && kk <= nd) {
+      src[j] = y + (size_t)q * n + (size_t)cols[kk - 1] * B + c;
     }
   }
+#pragma unroll
+  for (int j = 0; j < SJ; ++j)
+    if (src[j]) {
+      val[j] = ld_coherent(src[j]);
+      ok = ok && !is_sentinel(val[j]);
+    }
   int spins = 0;
   while (!__all(ok)) {
-    __builtin_amdgcn_s_sleep(1);
     ok = true;
 #pragma unroll
     for (int j = 0; j < SJ; ++j)
-      if (src[j] >= 0 && is_sentinel(val[j])) {
-        val[j] = ld_coherent(y + src[j]);
+      if (src[j] && is_sentinel(val[j])) {
+        val[j] = ld_coherent(src[j]);
         ok = ok && !is_sentinel(val[j]);
       }
     ++spins;
@@ -750,9 +814,13 @@ __device__ __forceinline__ void stage_deps(int kb0, int nb, int jb, const int* _
       break;
     }
   }
+  const int e1 = (1 + npad) * M;
 #pragma unroll
-  for (int j = 0; j < SJ; ++j)
-    if (src[j] >= 0) ys[lane + 64 * j] = val[j];
+  for (int j = 0; j < SJ; ++j) {
+    const int e = lane + 64 * j, kk = e / M, rem = e - kk * M, q = rem / B, c = rem - q * B;
+    if (e < e1 && (kk > 0 || row >= 0)) s[(kk * B + c) * NR + q] = val[j];
+  }
+  wave_lds_sync();
 }
 
 // Rows per lane of the sync-free sweep: two (one 16-byte load per factor
@@ -764,262 +832,285 @@ constexpr int sweep_free_width() {
   return (B % 2 == 0 && B >= 12) ? 2 : 1;
 }
 
+// Entry k of a raw vector load.
+template <int V, class TA>
+__device__ __forceinline__ auto raw_elem(const typename VecOf<TA, V>::T& v, int k) {
+  if constexpr (V == 1) {
+    return ldv(&v);
+  } else {
+    const TA e = v[k];
+    return ldv(&e);
+  }
+}
+
 template <int B, int NR, class TA, class TX>
-__global__ __launch_bounds__(64) void k_sweep_free(int nsup, int n, int forward, const int* __restrict__ order,
-                                                   const int* __restrict__ ia,
-                                                   const int* __restrict__ ja, const TA* __restrict__ off,
-                                                   const TA* __restrict__ diag, const TX* __restrict__ x, TX* y,
-                                                   int* ctl, const int* skip) {
-  if (skip && *skip) return;
+__global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free(SweepJob<TX> jb) {
+  if (jb.skip && *jb.skip) return;
   using Acc = typename AccOf<TX>::type;
   constexpr int V = sweep_free_width<B>();  // consecutive rows per lane (one vector load per column)
+  using VT = typename VecOf<TA, V>::T;
   constexpr int L = B / V;                  // lanes per column
   constexpr int G = 64 / L;                 // column groups
-  constexpr int KD = 3;                     // dependency blocks per staged chunk (one round trip for most rows)
+  constexpr int KD = 3;                     // dependency blocks per chunk
   constexpr int CK = (KD * B + G - 1) / G;  // columns of a chunk per lane
   constexpr int PD = (B + G - 1) / G;       // diagonal-block columns per lane
-  __shared__ Acc v[NR][B];
-  __shared__ TX ys[KD * B * NR];
-  const int lane = threadIdx.x;
-  const int lr = lane % L, g = lane / L;
-  const bool act = g < G;
-  for (int t = blockIdx.x; t < nsup; t += gridDim.x) {
-    const int row = order ? order[t] : (forward ? t : nsup - 1 - t);
-    const int jb = ia[row], ndep = ia[row + 1] - jb;
-    const TA* blk0 = off + (size_t)jb * B * B + lr * V;
+  // chunks whose factor values are in flight during the wait: two where they
+  // take up to 240 bytes of registers a lane each, and 64 KB of LDS hold the values
+  constexpr int NC = CK * V * (int)sizeof(TA) <= 240 && B * NR <= 144 ? 2 : 1;
+  __shared__ __align__(16) TX lds[kSweepWaves][(1 + NC * KD) * B * NR];
+  const int pos = sweep_position(jb);
+  if (pos < 0) return;  // wave-uniform; no workgroup-level synchronisation below
+  const int lane = threadIdx.x & 63;
+  TX* s = lds[threadIdx.x >> 6];
+  const bool second = pos >= jb.npos;
+  const int tp = second ? pos - jb.npos : pos, t = tp / jb.ng;
+  const size_t q0 = (size_t)(tp - t * jb.ng) * NR * jb.n;  // first value of the column group
+  const int* order = second ? jb.d1.order : jb.d0.order;
+  const int fwd = second ? jb.d1.forward : jb.d0.forward;
+  const int* __restrict__ ia = second ? jb.d1.ia : jb.d0.ia;
+  const int* __restrict__ ja = second ? jb.d1.ja : jb.d0.ja;
+  const TA* off = static_cast<const TA*>(second ? jb.d1.off : jb.d0.off);
+  const TA* diag = static_cast<const TA*>(second ? jb.d1.diag : jb.d0.diag);
+  TX* y = (second ? jb.y1 : jb.y0) + q0;
+  TX* xw = second ? jb.y0 + q0 : nullptr;
+  const char* x = static_cast<const char*>(jb.x) + q0 * (jb.x64 ? sizeof(double) : sizeof(TX));
+  const int lr = lane % L, g = lane / L < G ? lane / L : 0;
+  const bool act = lane < G * L;
+  const int row = order ? order[t] : (fwd ? t : jb.nsup - 1 - t);
+  const int j0 = ia[row], ndep = ia[row + 1] - j0;
+  const VT zero = {};
+  // the diagonal block does not depend on the wait
+  VT pd[PD];
+  {
     const TA* d = diag + (size_t)row * B * B + lr * V;
-    // the diagonal block and the right-hand side do not depend on the wait
-    Acc pd[PD][V];
 #pragma unroll
     for (int i = 0; i < PD; ++i) {
-      if (act && g + i * G < B) {
-        load_vec<V>(d + (g + i * G) * B, pd[i]);
-      } else {
-#pragma unroll
-        for (int k = 0; k < V; ++k) pd[i][k] = Acc(0);
-      }
+      pd[i] = zero;
+      if (act && g + i * G < B) pd[i] = __builtin_nontemporal_load(reinterpret_cast<const VT*>(d + (g + i * G) * B));
     }
-    Acc xv[NR][V];
-#pragma unroll
-    for (int q = 0; q < NR; ++q)
-#pragma unroll
-      for (int k = 0; k < V; ++k)
-        xv[q][k] = lane < L ? (Acc)x[(size_t)q * n + (size_t)row * B + lr * V + k] : Acc(0);
-    Acc acc[NR][V];
-#pragma unroll
-    for (int q = 0; q < NR; ++q)
-#pragma unroll
-      for (int k = 0; k < V; ++k) acc[q][k] = Acc(0);
-    // Chunks of KD dependency blocks. Column tt of the row's block stream
-    // (block tt / B, column tt % B) starts at blk0 + tt * B; the lane group g
-    // multiplies the columns tt = g (mod G), in ascending order.
-    for (int kb0 = 0; kb0 < ndep; kb0 += KD) {
-      const int nb = min(KD, ndep - kb0);
-      const int c0 = kb0 * B, c1 = (kb0 + nb) * B;
-      const int tf = c0 + ((g - c0 % G) % G + G) % G;
-      // the chunk's factor values do not depend on the wait: in flight first
-      Acc av[CK][V];
-#pragma unroll
-      for (int i = 0; i < CK; ++i) {
-        const int tt = tf + i * G;
-        if (act && tt < c1) {
-          load_vec<V>(blk0 + (size_t)tt * B, av[i]);
-        } else {
-#pragma unroll
-          for (int k = 0; k < V; ++k) av[i][k] = Acc(0);
-        }
-      }
-      stage_deps<B, NR, KD>(kb0, nb, jb, ja, y, n, ys, ctl);
-      __syncthreads();
-      if (act) {
-#pragma unroll
-        for (int i = 0; i < CK; ++i) {
-          const int tt = tf + i * G;
-          if (tt < c1) {
-            const int k = tt / B - kb0, c = tt % B;
-#pragma unroll
-            for (int q = 0; q < NR; ++q) {
-              const Acc yv = (Acc)ys[(k * NR + q) * B + c];
-#pragma unroll
-              for (int e = 0; e < V; ++e) acc[q][e] += av[i][e] * yv;
-            }
-          }
-        }
-      }
-      __syncthreads();
-    }
-#pragma unroll
-    for (int q = 0; q < NR; ++q)
-#pragma unroll
-      for (int k = 0; k < V; ++k) {
-        Acc s = acc[q][k];
-#pragma unroll
-        for (int h = 1; h < G; ++h) s += __shfl(acc[q][k], lane + h * L);
-        if (lane < L) v[q][lr * V + k] = xv[q][k] - s;
-      }
-    __syncthreads();
-    Acc z[NR][V];
-#pragma unroll
-    for (int q = 0; q < NR; ++q)
-#pragma unroll
-      for (int k = 0; k < V; ++k) z[q][k] = Acc(0);
-    if (act) {
-#pragma unroll
-      for (int i = 0; i < PD; ++i) {
-        const int c = g + i * G;
-        if (c < B) {
-#pragma unroll
-          for (int q = 0; q < NR; ++q) {
-            const Acc vc = v[q][c];
-#pragma unroll
-            for (int k = 0; k < V; ++k) z[q][k] += pd[i][k] * vc;
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < NR; ++q)
-#pragma unroll
-      for (int k = 0; k < V; ++k) {
-        Acc s = z[q][k];
-#pragma unroll
-        for (int h = 1; h < G; ++h) s += __shfl(z[q][k], lane + h * L);
-        if (lane < L) st_coherent(&y[(size_t)q * n + (size_t)row * B + lr * V + k], (TX)s);
-      }
-    __syncthreads();
   }
+  Acc acc[NR][V];
+#pragma unroll
+  for (int q = 0; q < NR; ++q)
+#pragma unroll
+    for (int k = 0; k < V; ++k) acc[q][k] = Acc(0);
+  // Column tt of a chunk (block tt / B, column tt % B): lane group g takes tt
+  // = g (mod G); columns past the chunk's last block are zero in av and s.
+  VT av[NC][CK];
+  auto load_chunk = [&](int k0, int nb, VT(&a)[CK]) {
+    const TA* blk = off + (size_t)(j0 + k0) * B * B + lr * V;
+#pragma unroll
+    for (int i = 0; i < CK; ++i) {
+      const int tt = g + i * G;
+      a[i] = zero;
+      if (act && tt < nb * B) a[i] = __builtin_nontemporal_load(reinterpret_cast<const VT*>(blk + (size_t)tt * B));
+    }
+  };
+  auto multiply = [&](int c, const VT(&a)[CK]) {
+    const TX* sc = s + (1 + c * KD) * B * NR;
+#pragma unroll
+    for (int i = 0; i < CK; ++i) {
+      const int tt = g + i * G, tc = tt < KD * B ? tt : KD * B - 1;
+#pragma unroll
+      for (int q = 0; q < NR; ++q) {
+        const Acc yv = (i + 1) * G <= KD * B || tt < KD * B ? (Acc)sc[tc * NR + q] : Acc(0);
+#pragma unroll
+        for (int k = 0; k < V; ++k) acc[q][k] += (Acc)raw_elem<V, TA>(a[i], k) * yv;
+      }
+    }
+  };
+  // rows with more than NC chunks of dependencies: the leading ones first
+  int k0 = 0;
+  for (; ndep - k0 > NC * KD; k0 += KD) {
+    load_chunk(k0, KD, av[0]);
+    stage_deps<B, NR, KD>(KD, KD, ja + j0 + k0, y, jb.n, -1, x, jb.x64, xw, s, jb.ctl);
+    multiply(0, av[0]);
+    wave_lds_sync();
+  }
+  const int nd = ndep - k0;
+  if (nd > 0) load_chunk(k0, nd < KD ? nd : KD, av[0]);
+  if constexpr (NC == 2)
+    if (nd > KD) load_chunk(k0 + KD, nd - KD, av[1]);
+  stage_deps<B, NR, NC * KD>(nd, nd > KD ? NC * KD : (nd > 0 ? KD : 0), ja + j0 + k0, y, jb.n, row, x, jb.x64, xw, s,
+                             jb.ctl);
+  if (nd > 0) multiply(0, av[0]);
+  if constexpr (NC == 2)
+    if (nd > KD) multiply(1, av[1]);
+#pragma unroll
+  for (int q = 0; q < NR; ++q)
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      Acc sm = acc[q][k];
+#pragma unroll
+      for (int h = 1; h < G; ++h) sm += __shfl(acc[q][k], lane + h * L);
+      if (lane < L) s[(lr * V + k) * NR + q] = (TX)((Acc)s[(lr * V + k) * NR + q] - sm);
+    }
+  wave_lds_sync();
+#pragma unroll
+  for (int q = 0; q < NR; ++q)
+#pragma unroll
+    for (int k = 0; k < V; ++k) acc[q][k] = Acc(0);
+#pragma unroll
+  for (int i = 0; i < PD; ++i) {
+    const int c = g + i * G, cc = c < B ? c : B - 1;
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+      const Acc vc = (i + 1) * G <= B || c < B ? (Acc)s[cc * NR + q] : Acc(0);
+#pragma unroll
+      for (int k = 0; k < V; ++k) acc[q][k] += (Acc)raw_elem<V, TA>(pd[i], k) * vc;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < NR; ++q)
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      Acc sm = acc[q][k];
+#pragma unroll
+      for (int h = 1; h < G; ++h) sm += __shfl(acc[q][k], lane + h * L);
+      if (lane < L) {
+        const size_t e = (size_t)q * jb.n + (size_t)row * B + lr * V + k;
+        st_coherent(&y[e], (TX)sm);
+        if (second && jb.out) jb.out[q0 + e] = (double)(TX)sm;
+      }
+    }
 }
 
 // The sync-free sweep of a complex factor (DevTri::cplx): factor blocks are
 // complex BC x BC, (re, im) pairs column-major, vectors real-equivalent
-// ([Re z; Im z] per block row). The protocol -- row order, sentinel
+// ([Re z; Im z] per block row). The protocol -- positions, sentinel
 // completion, bounded waits, dependency staging -- is k_sweep_free's; lane
 // (r, g) multiplies complex row r of the columns g, g + G, ... of the
 // dependency stream (one 16-byte load each), then of the diagonal block:
 //   v = x_row - sum_k F_k y_k,  y_row = D v,  (P + iQ)(a + ib) = (Pa - Qb) + i(Qa + Pb).
-// With order given and every dependency complete before the launch (one
-// launch per level) no wait ever spins.
 __device__ __forceinline__ VecOf<double, 2>::T ldnt_c(const double* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const VecOf<double, 2>::T*>(p));
 }
 
 template <int BC, int NR>
-__global__ __launch_bounds__(64) void k_sweep_free_cx(int nsup, int n, int forward, const int* __restrict__ order,
-                                                      const int* __restrict__ ia, const int* __restrict__ ja,
-                                                      const double* __restrict__ off,
-                                                      const double* __restrict__ diag,
-                                                      const double* __restrict__ x, double* y, int* ctl,
-                                                      const int* skip) {
-  if (skip && *skip) return;
+__global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free_cx(SweepJob<double> jb) {
+  if (jb.skip && *jb.skip) return;
   using C2 = VecOf<double, 2>::T;
   constexpr int B = 2 * BC;                   // real rows of a block row
   constexpr int G = 64 / BC;
-  constexpr int KD = 3;                       // dependency blocks per staged chunk
+  constexpr int KD = 3;                       // dependency blocks per chunk
   constexpr int CK = (KD * BC + G - 1) / G;   // complex columns of a chunk per lane
   constexpr int PD = (BC + G - 1) / G;        // diagonal-block columns per lane
-  __shared__ double v[NR][B];
-  __shared__ double ys[KD * B * NR];
-  const int lane = threadIdx.x;
-  const int r = lane % BC, g = lane / BC;
-  const bool act = g < G;
-  const C2 zero2 = {0.0, 0.0};
-  for (int t = blockIdx.x; t < nsup; t += gridDim.x) {
-    const int row = order ? order[t] : (forward ? t : nsup - 1 - t);
-    const int jb = ia[row], ndep = ia[row + 1] - jb;
-    const double* blk0 = off + (size_t)jb * BC * BC * 2;
-    const double* d = diag + (size_t)row * BC * BC * 2;
-    C2 pd[PD];
+  constexpr int NC = CK * 16 <= 240 && B * NR <= 144 ? 2 : 1;  // chunks in flight, as in k_sweep_free
+  __shared__ __align__(16) double lds[kSweepWaves][(1 + NC * KD) * B * NR];
+  const int pos = sweep_position(jb);
+  if (pos < 0) return;  // wave-uniform; no workgroup-level synchronisation below
+  const int lane = threadIdx.x & 63;
+  double* s = lds[threadIdx.x >> 6];
+  const bool second = pos >= jb.npos;
+  const int tp = second ? pos - jb.npos : pos, t = tp / jb.ng;
+  const size_t q0 = (size_t)(tp - t * jb.ng) * NR * jb.n;
+  const int* order = second ? jb.d1.order : jb.d0.order;
+  const int fwd = second ? jb.d1.forward : jb.d0.forward;
+  const int* __restrict__ ia = second ? jb.d1.ia : jb.d0.ia;
+  const int* __restrict__ ja = second ? jb.d1.ja : jb.d0.ja;
+  const double* off = static_cast<const double*>(second ? jb.d1.off : jb.d0.off);
+  const double* diag = static_cast<const double*>(second ? jb.d1.diag : jb.d0.diag);
+  double* y = (second ? jb.y1 : jb.y0) + q0;
+  double* xw = second ? jb.y0 + q0 : nullptr;
+  const double* x = static_cast<const double*>(jb.x) + q0;
+  const int r = lane % BC, g = lane / BC < G ? lane / BC : 0;
+  const bool act = lane < G * BC;
+  const int row = order ? order[t] : (fwd ? t : jb.nsup - 1 - t);
+  const int j0 = ia[row], ndep = ia[row + 1] - j0;
+  const C2 zero = {0.0, 0.0};
+  C2 pd[PD];
+  const double* d = diag + (size_t)row * BC * BC * 2;
 #pragma unroll
-    for (int i = 0; i < PD; ++i) pd[i] = (act && g + i * G < BC) ? ldnt_c(d + ((g + i * G) * BC + r) * 2) : zero2;
-    double xr[NR], xi[NR];
+  for (int i = 0; i < PD; ++i) {
+    pd[i] = zero;
+    if (act && g + i * G < BC) pd[i] = ldnt_c(d + ((g + i * G) * BC + r) * 2);
+  }
+  double ar[NR], ai[NR];
+#pragma unroll
+  for (int q = 0; q < NR; ++q) {
+    ar[q] = 0.0;
+    ai[q] = 0.0;
+  }
+  C2 av[NC][CK];
+  auto load_chunk = [&](int k0, int nb, C2(&a)[CK]) {
+    const double* blk = off + (size_t)(j0 + k0) * BC * BC * 2 + r * 2;
+#pragma unroll
+    for (int i = 0; i < CK; ++i) {
+      const int tt = g + i * G;
+      a[i] = zero;
+      if (act && tt < nb * BC) a[i] = ldnt_c(blk + (size_t)tt * BC * 2);
+    }
+  };
+  auto multiply = [&](int c, const C2(&a)[CK]) {
+    const double* sc = s + (1 + c * KD) * B * NR;
+#pragma unroll
+    for (int i = 0; i < CK; ++i) {
+      const int tt = g + i * G, tc = tt < KD * BC ? tt : KD * BC - 1;
+      const int k = tc / BC, cc = tc - k * BC;
+      const bool in = (i + 1) * G <= KD * BC || tt < KD * BC;
+#pragma unroll
+      for (int q = 0; q < NR; ++q) {
+        const double yr = in ? sc[(k * B + cc) * NR + q] : 0.0, yi = in ? sc[(k * B + BC + cc) * NR + q] : 0.0;
+        ar[q] += a[i].x * yr - a[i].y * yi;
+        ai[q] += a[i].y * yr + a[i].x * yi;
+      }
+    }
+  };
+  int k0 = 0;
+  for (; ndep - k0 > NC * KD; k0 += KD) {
+    load_chunk(k0, KD, av[0]);
+    stage_deps<B, NR, KD>(KD, KD, ja + j0 + k0, y, jb.n, -1, x, 0, xw, s, jb.ctl);
+    multiply(0, av[0]);
+    wave_lds_sync();
+  }
+  const int nd = ndep - k0;
+  if (nd > 0) load_chunk(k0, nd < KD ? nd : KD, av[0]);
+  if constexpr (NC == 2)
+    if (nd > KD) load_chunk(k0 + KD, nd - KD, av[1]);
+  stage_deps<B, NR, NC * KD>(nd, nd > KD ? NC * KD : (nd > 0 ? KD : 0), ja + j0 + k0, y, jb.n, row, x, 0, xw, s,
+                             jb.ctl);
+  if (nd > 0) multiply(0, av[0]);
+  if constexpr (NC == 2)
+    if (nd > KD) multiply(1, av[1]);
+#pragma unroll
+  for (int q = 0; q < NR; ++q) {
+    double sr = ar[q], si = ai[q];
+#pragma unroll
+    for (int h = 1; h < G; ++h) {
+      sr += __shfl(ar[q], lane + h * BC);
+      si += __shfl(ai[q], lane + h * BC);
+    }
+    if (lane < BC) {
+      s[lane * NR + q] -= sr;
+      s[(BC + lane) * NR + q] -= si;
+    }
+    ar[q] = 0.0;
+    ai[q] = 0.0;
+  }
+  wave_lds_sync();
+#pragma unroll
+  for (int i = 0; i < PD; ++i) {
+    const int c = g + i * G, cc = c < BC ? c : BC - 1;
+    const bool in = (i + 1) * G <= BC || c < BC;
 #pragma unroll
     for (int q = 0; q < NR; ++q) {
-      xr[q] = lane < BC ? x[(size_t)q * n + (size_t)row * B + lane] : 0.0;
-      xi[q] = lane < BC ? x[(size_t)q * n + (size_t)row * B + BC + lane] : 0.0;
+      const double vr = in ? s[cc * NR + q] : 0.0, vi = in ? s[(BC + cc) * NR + q] : 0.0;
+      ar[q] += pd[i].x * vr - pd[i].y * vi;
+      ai[q] += pd[i].y * vr + pd[i].x * vi;
     }
-    double ar[NR], ai[NR];
+  }
 #pragma unroll
-    for (int q = 0; q < NR; ++q) {
-      ar[q] = 0.0;
-      ai[q] = 0.0;
+  for (int q = 0; q < NR; ++q) {
+    double sr = ar[q], si = ai[q];
+#pragma unroll
+    for (int h = 1; h < G; ++h) {
+      sr += __shfl(ar[q], lane + h * BC);
+      si += __shfl(ai[q], lane + h * BC);
     }
-    for (int kb0 = 0; kb0 < ndep; kb0 += KD) {
-      const int nb = min(KD, ndep - kb0);
-      const int c0 = kb0 * BC, c1 = (kb0 + nb) * BC;
-      const int tf = c0 + ((g - c0 % G) % G + G) % G;
-      C2 av[CK];
-#pragma unroll
-      for (int i = 0; i < CK; ++i) {
-        const int tt = tf + i * G;
-        av[i] = (act && tt < c1) ? ldnt_c(blk0 + ((size_t)tt * BC + r) * 2) : zero2;
-      }
-      stage_deps<B, NR, KD>(kb0, nb, jb, ja, y, n, ys, ctl);
-      __syncthreads();
-      if (act) {
-#pragma unroll
-        for (int i = 0; i < CK; ++i) {
-          const int tt = tf + i * G;
-          if (tt < c1) {
-            const int k = tt / BC - kb0, c = tt % BC;
-#pragma unroll
-            for (int q = 0; q < NR; ++q) {
-              const double yr = ys[(k * NR + q) * B + c], yi = ys[(k * NR + q) * B + BC + c];
-              ar[q] += av[i].x * yr - av[i].y * yi;
-              ai[q] += av[i].y * yr + av[i].x * yi;
-            }
-          }
-        }
-      }
-      __syncthreads();
+    if (lane < BC) {
+      st_coherent(&y[(size_t)q * jb.n + (size_t)row * B + lane], sr);
+      st_coherent(&y[(size_t)q * jb.n + (size_t)row * B + BC + lane], si);
     }
-#pragma unroll
-    for (int q = 0; q < NR; ++q) {
-      double sr = ar[q], si = ai[q];
-#pragma unroll
-      for (int h = 1; h < G; ++h) {
-        sr += __shfl(ar[q], lane + h * BC);
-        si += __shfl(ai[q], lane + h * BC);
-      }
-      if (lane < BC) {
-        v[q][lane] = xr[q] - sr;
-        v[q][BC + lane] = xi[q] - si;
-      }
-    }
-    __syncthreads();
-    double zr[NR], zi[NR];
-#pragma unroll
-    for (int q = 0; q < NR; ++q) {
-      zr[q] = 0.0;
-      zi[q] = 0.0;
-    }
-    if (act) {
-#pragma unroll
-      for (int i = 0; i < PD; ++i) {
-        const int c = g + i * G;
-        if (c < BC) {
-#pragma unroll
-          for (int q = 0; q < NR; ++q) {
-            const double vr = v[q][c], vi = v[q][BC + c];
-            zr[q] += pd[i].x * vr - pd[i].y * vi;
-            zi[q] += pd[i].y * vr + pd[i].x * vi;
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < NR; ++q) {
-      double sr = zr[q], si = zi[q];
-#pragma unroll
-      for (int h = 1; h < G; ++h) {
-        sr += __shfl(zr[q], lane + h * BC);
-        si += __shfl(zi[q], lane + h * BC);
-      }
-      if (lane < BC) {
-        st_coherent(&y[(size_t)q * n + (size_t)row * B + lane], sr);
-        st_coherent(&y[(size_t)q * n + (size_t)row * B + BC + lane], si);
-      }
-    }
-    __syncthreads();
   }
 }
 
@@ -2088,38 +2179,107 @@ void launch_spmv(const DevBsr& A, const double* x, double* y, const double* bsub
   }
 }
 
-template <int B, int NR, class TA, class TX>
-static void sweep_b(const DevTri& T, const void* x, void* y, hipStream_t s, const int* skip, SweepSync* sync,
-                    RowGate gate) {
-  if (sync) {
-    // every wave must be resident: cooperative launch of at most the occupancy limit
-    auto kern = k_sweep_free<B, NR, TA, TX>;
-    // resident one-wave blocks per CU of this instantiation (queried once)
-    static const int per_cu = [&] {
-      int v = 0;
-      BCM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, kern, 64, 0));
-      return v;
-    }();
-    const int waves = std::max(1, std::min(T.nsup, std::min(per_cu, sync->waves_per_cu) * device_cu_count()));
-    const int64_t ny = (int64_t)T.n * NR;
-    TX* yy = static_cast<TX*>(y);
-    hipLaunchKernelGGL((k_sweep_fill<TX>), dim3(std::max<int64_t>(1, std::min<int64_t>((ny + 255) / 256, 2048))),
-                       dim3(256), 0, s, ny, yy, skip);
-    int nsup = T.nsup, n = T.n, fwd = T.forward ? 1 : 0;
-    const int* ia = T.ia.as<int>();
-    const int* ja = T.ja.as<int>();
-    const TA* off = T.off.as<TA>();
-    const TA* dg = T.diag.as<TA>();
-    const TX* xx = static_cast<const TX*>(x);
-    int* ct = sync->ext_ctl ? sync->ext_ctl : sync->ctl.as<int>();
-    const int* ord = sync->level_order ? T.level_rows.as<int>() : nullptr;
-    void* args[] = {&nsup, &n, &fwd, &ord, &ia, &ja, &off, &dg, &xx, &yy, &ct, (void*)&skip};
-    if (sync->cooperative)
-      BCM_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kern), dim3(waves), dim3(64), args, 0, s));
-    else
-      BCM_HIP(hipLaunchKernel(reinterpret_cast<const void*>(kern), dim3(waves), dim3(64), args, 0, s));
+// Columns per wave and column groups of a sync-free sweep over nrhs columns.
+// A wave that carries all columns reads every factor value once; one wave per
+// column reads them nrhs times (from L2 mostly) but its row takes a fraction
+// of the time, and that is on the dependency chain. So columns are split while
+// the waves of an average level stay within a quarter of the chip's wave slots
+// (16 a CU at these registers): such a sweep is bound by its chain, not by its
+// loads.
+static bool sweep_split_columns(const DevTri& T, int nrhs) {
+  const int64_t level_rows = T.levels > 0 ? (T.nsup + T.levels - 1) / T.levels : 1;
+  return level_rows * nrhs <= 4LL * device_cu_count();
+}
+
+// A set of sweeps of one launch: the first over T1, the second (if T2) over T2.
+struct SweepLaunch {
+  const DevTri* T1;
+  const DevTri* T2;
+  const void* x;
+  int x_prec;
+  void* y0;
+  void* y1;
+  double* out;
+  hipStream_t s;
+  const int* skip;
+  SweepSync* sync;
+};
+
+static SweepDir sweep_dir(const DevTri& T, const SweepSync& sync) {
+  SweepDir d;
+  d.order = sync.level_order ? T.level_rows.as<int>() : nullptr;
+  d.ia = T.ia.as<int>();
+  d.ja = T.ja.as<int>();
+  d.off = T.off.p;
+  d.diag = T.diag.p;
+  d.forward = T.forward ? 1 : 0;
+  return d;
+}
+
+// Fills the outputs and launches `kern` (8 block rows per workgroup) over
+// columns c0 .. c0 + nr * ng - 1.
+template <class TX>
+static void sweep_launch(void (*kern)(SweepJob<TX>), const SweepLaunch& l, int c0, int nr, int ng) {
+  const DevTri& T = *l.T1;
+  const size_t o = (size_t)c0 * T.n;
+  SweepJob<TX> jb{};
+  jb.nsup = T.nsup;
+  jb.n = T.n;
+  jb.ng = ng;
+  if ((int64_t)T.nsup * ng * 2 > INT32_MAX - kSweepWaves) throw Error(kErrArg, "device sweep exceeds 32-bit indexing");
+  jb.npos = T.nsup * ng;
+  jb.phases = l.T2 ? 2 : 1;
+  jb.x64 = l.x_prec == kF64 ? 1 : 0;
+  jb.d0 = sweep_dir(T, *l.sync);
+  if (l.T2) jb.d1 = sweep_dir(*l.T2, *l.sync);
+  jb.x = static_cast<const char*>(l.x) + o * (jb.x64 ? 8 : 4);
+  jb.y0 = static_cast<TX*>(l.y0) + o;
+  jb.y1 = l.T2 ? static_cast<TX*>(l.y1) + o : nullptr;
+  jb.out = l.out ? l.out + o : nullptr;
+  jb.ctl = l.sync->ext_ctl ? l.sync->ext_ctl : l.sync->ctl.as<int>();
+  jb.skip = l.skip;
+  const int64_t ny = (int64_t)T.n * nr * ng;
+  hipLaunchKernelGGL((k_sweep_fill<TX>), dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((ny + 255) / 256, 2048))),
+                     dim3(256), 0, l.s, ny, jb.y0, jb.y1, jb.ctl, l.skip);
+  const int grid = (jb.npos * jb.phases + kSweepWaves - 1) / kSweepWaves;
+  hipLaunchKernelGGL(kern, dim3(std::max(1, grid)), dim3(64 * kSweepWaves), 0, l.s, jb);
+  BCM_HIP(hipGetLastError());
+}
+
+template <int B, class TA, class TX>
+static void sweep_free(const SweepLaunch& l, int nrhs) {
+  if (sweep_split_columns(*l.T1, nrhs)) {
+    sweep_launch<TX>(k_sweep_free<B, 1, TA, TX>, l, 0, 1, nrhs);
     return;
   }
+  int done = 0;
+  while (done < nrhs) {
+    const int left = nrhs - done;
+    if (left >= 6) { sweep_launch<TX>(k_sweep_free<B, 6, TA, TX>, l, done, 6, 1); done += 6; }
+    else if (left >= 3) { sweep_launch<TX>(k_sweep_free<B, 3, TA, TX>, l, done, 3, 1); done += 3; }
+    else if (left == 2) { sweep_launch<TX>(k_sweep_free<B, 2, TA, TX>, l, done, 2, 1); done += 2; }
+    else { sweep_launch<TX>(k_sweep_free<B, 1, TA, TX>, l, done, 1, 1); done += 1; }
+  }
+}
+
+template <int BC>
+static void sweep_free_cx(const SweepLaunch& l, int nrhs) {
+  if (sweep_split_columns(*l.T1, nrhs)) {
+    sweep_launch<double>(k_sweep_free_cx<BC, 1>, l, 0, 1, nrhs);
+    return;
+  }
+  int done = 0;
+  while (done < nrhs) {
+    const int left = nrhs - done;
+    if (left >= 6) { sweep_launch<double>(k_sweep_free_cx<BC, 6>, l, done, 6, 1); done += 6; }
+    else if (left >= 3) { sweep_launch<double>(k_sweep_free_cx<BC, 3>, l, done, 3, 1); done += 3; }
+    else if (left == 2) { sweep_launch<double>(k_sweep_free_cx<BC, 2>, l, done, 2, 1); done += 2; }
+    else { sweep_launch<double>(k_sweep_free_cx<BC, 1>, l, done, 1, 1); done += 1; }
+  }
+}
+
+template <int B, int NR, class TA, class TX>
+static void sweep_b(const DevTri& T, const void* x, void* y, hipStream_t s, const int* skip, RowGate gate) {
   const int* rows = T.level_rows.as<int>();
   for (int l = 0; l < T.levels; ++l) {
     const int r0 = T.level_ptr[l], nr = T.level_ptr[l + 1] - r0;
@@ -2131,121 +2291,144 @@ static void sweep_b(const DevTri& T, const void* x, void* y, hipStream_t s, cons
   BCM_HIP(hipGetLastError());
 }
 
-template <int B, int NR>
-static void sweep_prec(const DevTri& T, const void* x, void* y, int vec_prec, hipStream_t s, const int* skip,
-                       SweepSync* sync, RowGate gate) {
-  if (T.prec == kF64 && vec_prec == kF64) sweep_b<B, NR, double, double>(T, x, y, s, skip, sync, gate);
-  else if (T.prec == kF32 && vec_prec == kF32) sweep_b<B, NR, float, float>(T, x, y, s, skip, sync, gate);
-  else if (T.prec == kBF16 && vec_prec == kF32) sweep_b<B, NR, uint16_t, float>(T, x, y, s, skip, sync, gate);
-  else throw Error(kErrArg, "unsupported factor/vector precision pair (fp64/fp64, fp32/fp32, bf16/fp32)");
-}
-
-template <int B>
-static void sweep_nr(const DevTri& T, const void* x, void* y, int vec_prec, int nrhs, hipStream_t s,
-                     const int* skip, SweepSync* sync, RowGate gate) {
-  const size_t es = prec_bytes(vec_prec);
+template <int B, class TA, class TX>
+static void sweep_nr(const DevTri& T, const void* x, void* y, int nrhs, hipStream_t s, const int* skip,
+                     RowGate gate) {
   int done = 0;
   while (done < nrhs) {
     const int left = nrhs - done;
-    const char* xs = static_cast<const char*>(x) + (size_t)done * T.n * es;
-    char* ys = static_cast<char*>(y) + (size_t)done * T.n * es;
-    if (left >= 6) { sweep_prec<B, 6>(T, xs, ys, vec_prec, s, skip, sync, gate); done += 6; }
-    else if (left >= 3) { sweep_prec<B, 3>(T, xs, ys, vec_prec, s, skip, sync, gate); done += 3; }
-    else if (left == 2) { sweep_prec<B, 2>(T, xs, ys, vec_prec, s, skip, sync, gate); done += 2; }
-    else { sweep_prec<B, 1>(T, xs, ys, vec_prec, s, skip, sync, gate); done += 1; }
+    const TX* xs = static_cast<const TX*>(x) + (size_t)done * T.n;
+    TX* ys = static_cast<TX*>(y) + (size_t)done * T.n;
+    if (left >= 6) { sweep_b<B, 6, TA, TX>(T, xs, ys, s, skip, gate); done += 6; }
+    else if (left >= 3) { sweep_b<B, 3, TA, TX>(T, xs, ys, s, skip, gate); done += 3; }
+    else if (left == 2) { sweep_b<B, 2, TA, TX>(T, xs, ys, s, skip, gate); done += 2; }
+    else { sweep_b<B, 1, TA, TX>(T, xs, ys, s, skip, gate); done += 1; }
+  }
+}
+
+template <int B>
+static void sweep_prec(const SweepLaunch& l, int vec_prec, int nrhs, RowGate gate) {
+  const DevTri& T = *l.T1;
+  if (T.prec == kF64 && vec_prec == kF64) {
+    if (l.sync) sweep_free<B, double, double>(l, nrhs);
+    else sweep_nr<B, double, double>(T, l.x, l.y0, nrhs, l.s, l.skip, gate);
+  } else if (T.prec == kF32 && vec_prec == kF32) {
+    if (l.sync) sweep_free<B, float, float>(l, nrhs);
+    else sweep_nr<B, float, float>(T, l.x, l.y0, nrhs, l.s, l.skip, gate);
+  } else if (T.prec == kBF16 && vec_prec == kF32) {
+    if (l.sync) sweep_free<B, uint16_t, float>(l, nrhs);
+    else sweep_nr<B, uint16_t, float>(T, l.x, l.y0, nrhs, l.s, l.skip, gate);
+  } else {
+    throw Error(kErrArg, "unsupported factor/vector precision pair (fp64/fp64, fp32/fp32, bf16/fp32)");
   }
 }
 
 template <int BC, int NR>
-static void sweep_cx_b(const DevTri& T, const double* x, double* y, hipStream_t s, const int* skip,
-                       SweepSync* sync) {
-  auto kern = k_sweep_free_cx<BC, NR>;
-  int n = T.n, fwd = T.forward ? 1 : 0;
-  const int* ia = T.ia.as<int>();
-  const int* ja = T.ja.as<int>();
-  const double* off = T.off.as<double>();
-  const double* dg = T.diag.as<double>();
-  if (sync) {  // as the real sync-free sweep: every wave resident, y filled with the sentinel first
-    static const int per_cu = [&] {
-      int v = 0;
-      BCM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, kern, 64, 0));
-      return v;
-    }();
-    const int waves = std::max(1, std::min(T.nsup, std::min(per_cu, sync->waves_per_cu) * device_cu_count()));
-    const int64_t ny = (int64_t)T.n * NR;
-    hipLaunchKernelGGL((k_sweep_fill<double>), dim3(std::max<int64_t>(1, std::min<int64_t>((ny + 255) / 256, 2048))),
-                       dim3(256), 0, s, ny, y, skip);
-    int nsup = T.nsup;
-    int* ct = sync->ext_ctl ? sync->ext_ctl : sync->ctl.as<int>();
-    const int* ord = sync->level_order ? T.level_rows.as<int>() : nullptr;
-    void* args[] = {&nsup, &n, &fwd, &ord, &ia, &ja, &off, &dg, &x, &y, &ct, (void*)&skip};
-    if (sync->cooperative)
-      BCM_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kern), dim3(waves), dim3(64), args, 0, s));
-    else
-      BCM_HIP(hipLaunchKernel(reinterpret_cast<const void*>(kern), dim3(waves), dim3(64), args, 0, s));
-    return;
-  }
+static void sweep_cx_level(const DevTri& T, const double* x, double* y, hipStream_t s, const int* skip) {
   // level by level: a launch's rows depend only on rows of earlier launches, so its waits never spin
-  const int* rows = T.level_rows.as<int>();
-  int* ct = T.lctl.as<int>();
+  SweepJob<double> jb{};
+  jb.n = T.n;
+  jb.ng = 1;
+  jb.phases = 1;
+  jb.x64 = 1;
+  jb.fixed = 1;
+  jb.d0 = SweepDir{nullptr, T.ia.as<int>(), T.ja.as<int>(), T.off.p, T.diag.p, T.forward ? 1 : 0};
+  jb.x = x;
+  jb.y0 = y;
+  jb.ctl = T.lctl.as<int>();
+  jb.skip = skip;
   for (int l = 0; l < T.levels; ++l) {
-    const int r0 = T.level_ptr[l], nr = T.level_ptr[l + 1] - r0;
-    hipLaunchKernelGGL(kern, dim3(nr), dim3(64), 0, s, nr, n, fwd, rows + r0, ia, ja, off, dg, x, y, ct, skip);
+    jb.nsup = jb.npos = T.level_ptr[l + 1] - T.level_ptr[l];
+    jb.d0.order = T.level_rows.as<int>() + T.level_ptr[l];
+    hipLaunchKernelGGL((k_sweep_free_cx<BC, NR>), dim3((jb.npos + kSweepWaves - 1) / kSweepWaves),
+                       dim3(64 * kSweepWaves), 0, s, jb);
   }
   BCM_HIP(hipGetLastError());
 }
 
 template <int BC>
-static void sweep_cx_nr(const DevTri& T, const double* x, double* y, int nrhs, hipStream_t s, const int* skip,
-                        SweepSync* sync) {
+static void sweep_cx(const SweepLaunch& l, int nrhs) {
+  if (l.sync) {
+    sweep_free_cx<BC>(l, nrhs);
+    return;
+  }
+  const DevTri& T = *l.T1;
   int done = 0;
   while (done < nrhs) {
     const int left = nrhs - done;
-    const size_t o = (size_t)done * T.n;
-    if (left >= 6) { sweep_cx_b<BC, 6>(T, x + o, y + o, s, skip, sync); done += 6; }
-    else if (left >= 3) { sweep_cx_b<BC, 3>(T, x + o, y + o, s, skip, sync); done += 3; }
-    else if (left == 2) { sweep_cx_b<BC, 2>(T, x + o, y + o, s, skip, sync); done += 2; }
-    else { sweep_cx_b<BC, 1>(T, x + o, y + o, s, skip, sync); done += 1; }
+    const double* x = static_cast<const double*>(l.x) + (size_t)done * T.n;
+    double* y = static_cast<double*>(l.y0) + (size_t)done * T.n;
+    if (left >= 6) { sweep_cx_level<BC, 6>(T, x, y, l.s, l.skip); done += 6; }
+    else if (left >= 3) { sweep_cx_level<BC, 3>(T, x, y, l.s, l.skip); done += 3; }
+    else if (left == 2) { sweep_cx_level<BC, 2>(T, x, y, l.s, l.skip); done += 2; }
+    else { sweep_cx_level<BC, 1>(T, x, y, l.s, l.skip); done += 1; }
+  }
+}
+
+static void sweep_dispatch(const SweepLaunch& l, int vec_prec, int nrhs, RowGate gate) {
+  const DevTri& T = *l.T1;
+  if (l.sync) l.sync->ensure(T.nsup, l.s);
+  if (T.cplx) {
+    if (gate.active) throw Error(kErrArg, "row-gated sweeps are not defined for complex factors");
+    if (vec_prec != kF64) throw Error(kErrArg, "complex factors sweep FP64 vectors");
+    switch (T.b / 2) {
+      case 3: sweep_cx<3>(l, nrhs); break;
+      case 4: sweep_cx<4>(l, nrhs); break;
+      case 6: sweep_cx<6>(l, nrhs); break;
+      case 8: sweep_cx<8>(l, nrhs); break;
+      case 12: sweep_cx<12>(l, nrhs); break;
+      case 16: sweep_cx<16>(l, nrhs); break;
+      default: throw Error(kErrInternal, "complex sweep: unsupported block size");
+    }
+    return;
+  }
+  switch (T.b) {
+    case 3: sweep_prec<3>(l, vec_prec, nrhs, gate); break;
+    case 6: sweep_prec<6>(l, vec_prec, nrhs, gate); break;
+    case 8: sweep_prec<8>(l, vec_prec, nrhs, gate); break;
+    case 9: sweep_prec<9>(l, vec_prec, nrhs, gate); break;
+    case 12: sweep_prec<12>(l, vec_prec, nrhs, gate); break;
+    case 16: sweep_prec<16>(l, vec_prec, nrhs, gate); break;
+    case 24: sweep_prec<24>(l, vec_prec, nrhs, gate); break;
+    case 32: sweep_prec<32>(l, vec_prec, nrhs, gate); break;
+    default: throw Error(kErrArg, "unsupported block size for the device sweep (use 3,6,8,9,12,16,24,32)");
   }
 }
 
 void launch_sweep(const DevTri& T, const void* x, void* y, int vec_prec, int nrhs, hipStream_t s,
                   const int* skip, SweepSync* sync, RowGate gate) {
   if (x == y) throw Error(kErrArg, "triangular sweep: input and output must not alias");
-  if (T.cplx) {
-    if (gate.active) throw Error(kErrArg, "row-gated sweeps are not defined for complex factors");
-    if (vec_prec != kF64) throw Error(kErrArg, "complex factors sweep FP64 vectors");
-    if (sync) sync->ensure(T.nsup, s);
-    const double* xd = static_cast<const double*>(x);
-    double* yd = static_cast<double*>(y);
-    switch (T.b / 2) {
-      case 3: sweep_cx_nr<3>(T, xd, yd, nrhs, s, skip, sync); break;
-      case 4: sweep_cx_nr<4>(T, xd, yd, nrhs, s, skip, sync); break;
-      case 6: sweep_cx_nr<6>(T, xd, yd, nrhs, s, skip, sync); break;
-      case 8: sweep_cx_nr<8>(T, xd, yd, nrhs, s, skip, sync); break;
-      case 12: sweep_cx_nr<12>(T, xd, yd, nrhs, s, skip, sync); break;
-      case 16: sweep_cx_nr<16>(T, xd, yd, nrhs, s, skip, sync); break;
-      default: throw Error(kErrInternal, "complex sweep: unsupported block size");
-    }
-    return;
-  }
   if (T.b == 0) {  // variable blocks: level by level whatever the schedule
     if (gate.active) throw Error(kErrArg, "row-gated sweeps need a uniform tuned block size");
     launch_sweep_var(T, x, y, vec_prec, nrhs, s, skip);
     return;
   }
-  if (sync) sync->ensure(T.nsup, s);
-  switch (T.b) {
-    case 3: sweep_nr<3>(T, x, y, vec_prec, nrhs, s, skip, sync, gate); break;
-    case 6: sweep_nr<6>(T, x, y, vec_prec, nrhs, s, skip, sync, gate); break;
-    case 8: sweep_nr<8>(T, x, y, vec_prec, nrhs, s, skip, sync, gate); break;
-    case 9: sweep_nr<9>(T, x, y, vec_prec, nrhs, s, skip, sync, gate); break;
-    case 12: sweep_nr<12>(T, x, y, vec_prec, nrhs, s, skip, sync, gate); break;
-    case 16: sweep_nr<16>(T, x, y, vec_prec, nrhs, s, skip, sync, gate); break;
-    case 24: sweep_nr<24>(T, x, y, vec_prec, nrhs, s, skip, sync, gate); break;
-    case 32: sweep_nr<32>(T, x, y, vec_prec, nrhs, s, skip, sync, gate); break;
-    default: throw Error(kErrArg, "unsupported block size for the device sweep (use 3,6,8,9,12,16,24,32)");
+  sweep_dispatch({&T, nullptr, x, vec_prec, y, nullptr, nullptr, s, skip, sync}, vec_prec, nrhs, gate);
+}
+
+void launch_sweep_pair(const DevTri& T1, const DevTri& T2, const double* r, double* z, void* w0, void* w1,
+                       int vec_prec, int nrhs, hipStream_t s, const int* skip, SweepSync* sync) {
+  const size_t vb = (size_t)T1.n * nrhs * 8;
+  const char *rb = reinterpret_cast<const char*>(r), *zb = reinterpret_cast<const char*>(z);
+  const bool apart = rb + vb <= zb || zb + vb <= rb;
+  // In one launch z is filled before r is read and written while it still is.
+  if (sync && T1.b && T1.b == T2.b && T1.nsup == T2.nsup && T1.cplx == T2.cplx && T1.prec == T2.prec &&
+      apart) {
+    void* y1 = vec_prec == kF64 ? static_cast<void*>(z) : w1;
+    double* out = vec_prec == kF64 ? nullptr : z;
+    sweep_dispatch({&T1, &T2, r, kF64, w0, y1, out, s, skip, sync}, vec_prec, nrhs, RowGate());
+    return;
   }
+  if (vec_prec == kF64) {
+    launch_sweep(T1, r, w0, kF64, nrhs, s, skip, sync);
+    launch_sweep(T2, w0, z, kF64, nrhs, s, skip, sync);
+    return;
+  }
+  const int64_t ne = (int64_t)T1.n * nrhs;
+  launch_convert(ne, r, kF64, w1, kF32, s, skip);
+  launch_sweep(T1, w1, w0, kF32, nrhs, s, skip, sync);
+  launch_sweep(T2, w0, w1, kF32, nrhs, s, skip, sync);
+  launch_convert(ne, w1, kF32, z, kF64, s, skip);
 }
 
 void launch_multidot(int n, int k, const double* const* xs, const double* const* ys, double* out, RedWork& rw,

@@ -425,12 +425,12 @@ hipEvent_t Context::prof_begin() {
   return e;
 }
 
-void Context::prof_end(int kind, hipEvent_t e0, double bytes) {
+void Context::prof_end(int kind, hipEvent_t e0, double bytes, int launches) {
   hipEvent_t e1;
   if (ev_pool.empty()) BCM_HIP(hipEventCreate(&e1));
   else { e1 = ev_pool.back(); ev_pool.pop_back(); }
   BCM_HIP(hipEventRecord(e1, stream));
-  pending.push_back(Pending{kind, e0, e1, bytes});
+  pending.push_back(Pending{kind, launches, e0, e1, bytes});
   if (pending.size() > 4096) prof_flush();
 }
 
@@ -453,7 +453,7 @@ __global__ void k_gate_bytes(int np, const int* __restrict__ active, const doubl
 
 ProfScope::~ProfScope() {
   if (!(c.prof && e0)) return;
-  c.prof_end(kind, e0, bytes);
+  c.prof_end(kind, e0, bytes, launches);
   if (gate_active) {  // after the closing event: not part of the timed span
     hipLaunchKernelGGL(k_gate_bytes, dim3(1), dim3(256), 0, c.stream, nparts, gate_active, part_bytes,
                        c.prof_dev_bytes() + kind);
@@ -485,7 +485,7 @@ void Context::prof_flush() {
     float ms = 0.f;
     BCM_HIP(hipEventElapsedTime(&ms, p.e0, p.e1));
     prof_acc[p.kind].ms += ms;
-    prof_acc[p.kind].launches += 1;
+    prof_acc[p.kind].launches += p.launches;
     prof_acc[p.kind].bytes += p.bytes;
     ev_pool.push_back(p.e0);
     ev_pool.push_back(p.e1);
@@ -494,30 +494,14 @@ void Context::prof_flush() {
 }
 
 void precond_sweeps(const DevTri& t1, const DevTri& t2, Context& ctx, const double* r, double* z, int prec, int nrhs,
-                    const int* skip, RowGate gate) {
-  const int64_t n = t1.n;
-  if (prec == kF64) {
-    double* tmp = ctx.vec(12, (size_t)n * nrhs * 8);
-    {
-      ProfScope ps(ctx, kProfSweep, sweep_bytes(t1, nrhs));
-      launch_sweep(t1, r, tmp, kF64, nrhs, ctx.stream, skip, ctx.sweep_sync(), gate);
-    }
-    ProfScope ps(ctx, kProfSweep, sweep_bytes(t2, nrhs));
-    launch_sweep(t2, tmp, z, kF64, nrhs, ctx.stream, skip, ctx.sweep_sync(), gate);
-  } else {
-    float* r32 = reinterpret_cast<float*>(ctx.vec(13, (size_t)n * nrhs * 4));
-    float* t32 = reinterpret_cast<float*>(ctx.vec(14, (size_t)n * nrhs * 4));
-    launch_convert(n * nrhs, r, kF64, r32, kF32, ctx.stream, skip);
-    {
-      ProfScope ps(ctx, kProfSweep, sweep_bytes(t1, nrhs));
-      launch_sweep(t1, r32, t32, kF32, nrhs, ctx.stream, skip, ctx.sweep_sync(), gate);
-    }
-    {
-      ProfScope ps(ctx, kProfSweep, sweep_bytes(t2, nrhs));
-      launch_sweep(t2, t32, r32, kF32, nrhs, ctx.stream, skip, ctx.sweep_sync(), gate);
-    }
-    launch_convert(n * nrhs, r32, kF32, z, kF64, ctx.stream, skip);
-  }
+                    const int* skip) {
+  const size_t n = (size_t)t1.n * nrhs;
+  const int vp = prec == kF64 ? kF64 : kF32;
+  double* w0 = ctx.vec(prec == kF64 ? 12 : 14, n * prec_bytes(vp));
+  double* w1 = prec == kF64 ? nullptr : ctx.vec(13, n * 4);
+  ProfScope ps(ctx, kProfSweep, sweep_bytes(t1, nrhs) + sweep_bytes(t2, nrhs));
+  ps.launches = 2;
+  launch_sweep_pair(t1, t2, r, z, w0, w1, vp, nrhs, ctx.stream, skip, ctx.sweep_sync());
 }
 
 void precond_apply(Factor& F, Context& ctx, const double* r, double* z, int prec, bool transpose, int nrhs,
@@ -803,27 +787,16 @@ void solve(Matrix& A, Factor& F, Context& ctx, const SolveOptions& opt, const do
     }
     BCM_HIP(hipStreamSynchronize(ctx.stream));
   };
-  // Sync-free sweeps are first launched as ordinary kernels: the grid never
-  // exceeds what the device holds at once, so on an otherwise idle GPU every
-  // wave is resident, without the cooperative launch's cost. If a wait hit
-  // its bound (another process held part of the GPU), the solve is repeated
-  // from the same x0 with cooperative launches, which guarantee residency.
-  const bool saved = ctx.sync.cooperative;
-  const bool fast = ctx.sweep_mode == 1 && saved;
+  // If a wait of a sync-free sweep hit its bound (another process held the
+  // GPU for long), the solve is repeated from the same x0.
+  const bool fast = ctx.sweep_mode == 1;
   const int64_t n = A.d.n;
   double* x0 = nullptr;
   if (fast) {
     x0 = ctx.vec(87, (size_t)n * 8);
     launch_copy(n, x, x0, ctx.stream);
-    ctx.sync.cooperative = false;
   }
-  try {
-    run();
-  } catch (...) {
-    ctx.sync.cooperative = saved;
-    throw;
-  }
-  ctx.sync.cooperative = saved;
+  run();
   if (fast && ctx.sync.error(ctx.stream)) {
     ctx.sync.clear(ctx.stream);
     launch_copy(n, x0, x, ctx.stream);

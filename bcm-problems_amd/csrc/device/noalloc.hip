@@ -75,30 +75,19 @@ void precond_noalloc(Factor& F, Context& ctx, const double* r, double* z, int pr
   char* ctl = scratch_ptr();
   char* base = ctl + kCtlBytes;
   hipStream_t s = ctx.stream;
-  const int64_t ne = (int64_t)elems;
   SweepSync local;
   SweepSync* sync = nullptr;
   if (const SweepSync* cs = ctx.sweep_sync()) {
     local.waves_per_cu = cs->waves_per_cu;
-    local.cooperative = cs->cooperative;
     local.level_order = cs->level_order;
     local.ext_ctl = reinterpret_cast<int*>(ctl);
     hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, s, local.ext_ctl, (int)(kCtlBytes / 4));
     BCM_HIP(hipGetLastError());
     sync = &local;
   }
-  if (prec == kF64) {
-    double* tmp = reinterpret_cast<double*>(base);
-    launch_sweep(t1, r, tmp, kF64, nrhs, s, nullptr, sync);
-    launch_sweep(t2, tmp, z, kF64, nrhs, s, nullptr, sync);
-  } else {
-    float* r32 = reinterpret_cast<float*>(base);
-    float* t32 = reinterpret_cast<float*>(base + ((elems * 4 + 255) & ~size_t(255)));  // 256-byte aligned
-    launch_convert(ne, r, kF64, r32, kF32, s);
-    launch_sweep(t1, r32, t32, kF32, nrhs, s, nullptr, sync);
-    launch_sweep(t2, t32, r32, kF32, nrhs, s, nullptr, sync);
-    launch_convert(ne, r32, kF32, z, kF64, s);
-  }
+  char* second = base + ((elems * 4 + 255) & ~size_t(255));  // 256-byte aligned
+  const int vp = prec == kF64 ? kF64 : kF32;
+  launch_sweep_pair(t1, t2, r, z, base, prec == kF64 ? nullptr : second, vp, nrhs, s, nullptr, sync);
 }
 
 }  // namespace bcm

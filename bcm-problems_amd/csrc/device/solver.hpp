@@ -74,10 +74,10 @@ struct Context {
   bool prof = false;
   ProfAcc prof_acc[kProfKinds];
   std::vector<hipEvent_t> ev_pool;
-  struct Pending { int kind; hipEvent_t e0, e1; double bytes; };
+  struct Pending { int kind, launches; hipEvent_t e0, e1; double bytes; };
   std::vector<Pending> pending;
   hipEvent_t prof_begin();
-  void prof_end(int kind, hipEvent_t e0, double bytes);
+  void prof_end(int kind, hipEvent_t e0, double bytes, int launches = 1);
   void prof_flush();
   // Bytes of launches whose work is only known on the device (row-gated
   // products and sweeps): accumulated by device kernels per kind, added to
@@ -92,6 +92,7 @@ struct ProfScope {
   Context& c;
   int kind;
   double bytes;
+  int launches = 1;  // sweeps or products that the scope counts as
   hipEvent_t e0 = nullptr;
   // row-gated launch: bytes = sum over parts of active[c] * part_bytes[c] (device)
   const int* gate_active = nullptr;
@@ -173,7 +174,7 @@ size_t precond_noalloc_max_elems();
 // z = M^-1 r through the sweep pair (t1 then t2) in the given precision
 // (fp64 vectors, or fp32 vectors converted on the way in and out).
 void precond_sweeps(const DevTri& t1, const DevTri& t2, Context& ctx, const double* r, double* z, int prec, int nrhs,
-                    const int* skip = nullptr, RowGate gate = RowGate());
+                    const int* skip = nullptr);
 
 // FGMRES(m) driver (fgmres.hip).
 void solve_fgmres(Matrix& A, Factor& F, Context& ctx, const SolveOptions& opt, const double* b, double* x,

@@ -227,18 +227,17 @@ int bcm_context_create(bcm_context* out);
 int bcm_context_destroy(bcm_context c);
 int bcm_context_sync(bcm_context c);
 /* Triangular sweep schedule: 0 = one launch per dependency level;
- * 1 = one sync-free cooperative launch per sweep (default): resident waves
- * own positions of the rows sorted by dependency level round-robin and wait
- * (bounded) on the values of the rows they depend on; 2 = as 1 over the
- * natural sweep order. The schedules agree to rounding: per row they add
+ * 1 = one sync-free launch per sweep, or per pair of sweeps (default): waves
+ * take the rows in dependency-level order and wait (bounded) on the values of
+ * the rows they depend on; 2 = as 1 over the natural sweep order. The schedules agree to rounding: per row they add
  * the same products, grouped differently across lanes for some block sizes. */
 int bcm_context_set_sweep_mode(bcm_context c, int mode);
-/* Resident waves per CU of the sync-free sweeps (1..64, default 8; fewer
- * waves than block rows make each wave own several rows in turn). */
+/* Resident waves per CU asked of the sync-free sweeps (1..64, default 8).
+ * A hint without effect on results; the present kernels take what fits. */
 int bcm_context_set_sweep_waves(bcm_context c, int waves_per_cu);
 /* Test hook: marks the sync-free sweeps' dependency wait as having reached its
  * bound, so that every wait of the next solve exits at once and the solve
- * takes its recovery path (repeated from x0 with cooperative launches). No
+ * takes its recovery path (repeated from x0 after the flag is cleared). No
  * counterpart in the reference. */
 int bcm_context_raise_wait_flag(bcm_context c);
 
@@ -319,7 +318,7 @@ typedef struct bcm_batch_stats {
 } bcm_batch_stats;
 typedef struct bcm_batch_tune {
   int sweep_mode;    /* 0 level-scheduled sweeps, 1 sync-free sweeps */
-  int waves_per_cu;  /* sync-free sweeps: resident waves per CU */
+  int waves_per_cu;  /* sync-free sweeps: resident waves per CU (hint) */
   int level_order;   /* sync-free sweeps: 1 rows in dependency-level order, 0 natural order */
   int graph;         /* 1: replay check_every iterations as one captured hipGraph */
   int check_every;   /* iterations between host polls */

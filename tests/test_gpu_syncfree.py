@@ -75,3 +75,75 @@ def test_syncfree_solvers(B, O, fctx):
     st = fctx.solve(s["mo"], s["f"], db, dx, B.default_opts(kind=B.BICGSTAB, eps=1e-10))
     xo, r = O.bicgstab(s["A"], s["L"], s["U"], s["b"], eps=1e-10)
     assert st.converged and st.relres_true <= 1e-10 and rel(dx.host(), xo) < 1e-8
+
+
+def coupled_groups(B, size, ngroup, blocks, seed):
+    """Groups of `size` block rows, every row coupled to every other of its
+    group: `size` dependency levels of `ngroup` rows, up to size - 1 blocks a
+    row. `blocks` lists the block sizes, row after row (repeated)."""
+    rng = np.random.default_rng(seed)
+    ns = size * ngroup
+    bs = np.array([blocks[k % len(blocks)] for k in range(ns)])
+    vals, ja = [], []
+    for r in range(ns):
+        for c in range(r // size * size, r // size * size + size):
+            blk = 0.2 * rng.standard_normal((bs[c], bs[r]))
+            if c == r:
+                blk = blk + 8.0 * np.eye(bs[r])
+            vals.append(blk.ravel())
+            ja.append(c)
+    sp = np.concatenate([[0], np.cumsum(bs)]).astype(np.int32)
+    m = B.Matrix.from_arrays(sp, np.arange(ns + 1) * size, ja, np.concatenate(vals), False)
+    return m, B.Factor.ilu2(m, B.default_params(tau1=1e-9, tau2=1e-11))
+
+
+# 600 groups of 3: level of 600 rows, one wave carries 2, 3 or 6 columns; 12
+# groups of 9: narrow levels, one wave per column, and rows of 8 dependencies
+# (more than the chunks held in registers)
+GROUPS = [(3, 600, 2), (3, 600, 3), (3, 400, 7), (9, 12, 1), (9, 12, 6), (9, 200, 6)]
+
+
+@pytest.mark.parametrize("size,ngroup,nrhs", GROUPS)
+@pytest.mark.parametrize("b", [3, 6, 8, 9, 12, 16, 24, 32])
+def test_syncfree_pair_matches_level_schedule(B, fctx, b, size, ngroup, nrhs):
+    if b > 16 and size * ngroup * size > 6000:
+        size, ngroup = 3, 400  # bounded host factorization
+    m, f = coupled_groups(B, size, ngroup, [b], seed=b)
+    print(f"pair b={b} groups {ngroup} x {size} nrhs={nrhs}", flush=True)
+    r = np.random.default_rng(6).standard_normal((m.n, nrhs))
+    lctx = B.Context()
+    lctx.set_sweep_mode(0)
+    # the same products per row in another order: sums of up to 9 * 32 terms, FP32 factors and vectors for precision 1 and 2
+    for precision, tol in ((0, 1e-13), (1, 2e-5), (2, 2e-5)):
+        dr, dz, dl = dev(B, r), B.DeviceArray((m.n, nrhs)), B.DeviceArray((m.n, nrhs))
+        fctx.precond(f, dr, dz, nrhs, precision=precision)
+        lctx.precond(f, dr, dl, nrhs, precision=precision)
+        fctx.sync()
+        lctx.sync()
+        want = dl.host()
+        assert rel(dz.host(), want) < tol
+        fctx.precond(f, dr, dr, nrhs, precision=precision)  # in place
+        fctx.sync()
+        assert rel(dr.host(), want) < tol
+
+
+def test_syncfree_complex_wide_levels(B, fctx):
+    rng = np.random.default_rng(8)
+    for bc, nrhs in ((3, 2), (12, 3), (16, 6), (4, 6)):
+        ns = 1200  # 400 groups of 3
+        ia, ja = [0], []
+        for r in range(ns):
+            ja += list(range(r, r // 3 * 3 + 3))
+            ia.append(len(ja))
+        a = 0.1 * (rng.standard_normal((len(ja), bc, bc)) + 1j * rng.standard_normal((len(ja), bc, bc)))
+        f = B.Factor.from_complex(np.arange(ns + 1) * bc, (ia, ja, a.ravel()), (ia, ja, a.ravel()))
+        n = ns * 2 * bc
+        print(f"complex wide bc={bc} nrhs={nrhs}", flush=True)
+        dr, dz, dl = dev(B, rng.standard_normal((n, nrhs))), B.DeviceArray((n, nrhs)), B.DeviceArray((n, nrhs))
+        lctx = B.Context()
+        lctx.set_sweep_mode(0)
+        fctx.precond(f, dr, dz, nrhs)
+        lctx.precond(f, dr, dl, nrhs)
+        fctx.sync()
+        lctx.sync()
+        assert rel(dz.host(), dl.host()) < 1e-13
