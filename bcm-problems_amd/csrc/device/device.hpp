@@ -125,6 +125,7 @@ struct DevTri {
   DevBuf off;         // ndep blocks, row after row
   DevBuf diag;        // nsup inverted diagonal blocks
   DevBuf sp, doff, dgo;  // variable blocks: partition, value offsets of dependency and diagonal blocks
+  DevBuf cptr, ccol, roff;  // their columns: first per row, vector element of each, value offset of each row
   int64_t nval = 0;
   int64_t value_bytes() const {
     if (cplx) return ((int64_t)ndep + nsup) * b * b / 2 * 8;

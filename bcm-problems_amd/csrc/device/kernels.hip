@@ -731,6 +731,10 @@ struct SweepDir {
   const void* off;
   const void* diag;
   int forward;
+  // any block partition (k_sweep_free_var): ia and ja then count vector columns
+  const int* sp;
+  const int64_t* roff;  // first dependency value of each row
+  const int64_t* dgo;   // its diagonal block
 };
 
 // A sweep launch: `phases` sweeps (1 or 2) over npos = nsup * ng positions
@@ -1111,6 +1115,171 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free_cx(SweepJob<dou
       st_coherent(&y[(size_t)q * jb.n + (size_t)row * B + lane], sr);
       st_coherent(&y[(size_t)q * jb.n + (size_t)row * B + BC + lane], si);
     }
+  }
+}
+
+// The sync-free sweep for any block partition: protocol and positions of
+// k_sweep_free, one wave per block row and column of the vectors. The
+// dependency blocks of row k, each stored with its b_k rows, are one
+// b_k x W column-major matrix (W the sum of the dependencies' sizes); ja
+// lists the vector element of each of its columns, ia its first column per
+// row. Lanes are g * b_k + r: group g of G = 64 / b_k takes the columns g, g +
+// G, ...; kVarHeld columns per lane are in flight during the wait (all of a
+// row's where its W <= kVarHeld * G), the others are loaded after it.
+// One launch per level was bound by the launches (3 us each): at 1320 rows
+// of 7 to 14 in 31 levels, a sweep took 95 us in 31 launches.
+constexpr int kVarHeld = 16;
+constexpr int kVarChunk = 192;  // columns staged at a time
+
+// Columns cols[0..nw) of y, and with bk > 0 the row's right-hand side (bk
+// values from element r0 of x, or of xw and then waited for), into s[64 + t]
+// and s[r].
+template <class TX>
+__device__ __forceinline__ void stage_var(int nw, const int* __restrict__ cols, const TX* y, int r0, int bk,
+                                          const void* x, int x64, const TX* xw, TX* s, int* ctl) {
+  constexpr int SJ = 1 + kVarChunk / 64;
+  const int lane = threadIdx.x & 63;
+  const TX* src[SJ];
+  TX val[SJ];
+  bool ok = true;
+#pragma unroll
+  for (int j = 0; j < SJ; ++j) {
+    src[j] = nullptr;
+    val[j] = TX(0);
+    if (j == 0) {
+      if (lane < bk) {
+        if (xw) src[j] = xw + r0 + lane;
+        else val[j] = x64 ? (TX) static_cast<const double*>(x)[r0 + lane] : static_cast<const TX*>(x)[r0 + lane];
+      }
+    } else if (lane + 64 * (j - 1) < nw) {
+      src[j] = y + cols[lane + 64 * (j - 1)];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < SJ; ++j)
+    if (src[j]) {
+      val[j] = ld_coherent(src[j]);
+      ok = ok && !is_sentinel(val[j]);
+    }
+  int spins = 0;
+  while (!__all(ok)) {
+    ok = true;
+#pragma unroll
+    for (int j = 0; j < SJ; ++j)
+      if (src[j] && is_sentinel(val[j])) {
+        val[j] = ld_coherent(src[j]);
+        ok = ok && !is_sentinel(val[j]);
+      }
+    ++spins;
+    if (__any(spins > kSpinLimit || ((spins & 1023) == 0 && ld_coherent(&ctl[2]) != 0))) {
+      if (lane == 0) st_coherent(&ctl[2], 1);
+      break;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < SJ; ++j)
+    if (j > 0 || bk > 0) s[lane + 64 * j] = val[j];
+  wave_lds_sync();
+}
+
+// Sum over the G lane groups of v for the rows r < bk (valid in lanes < bk).
+template <class Acc>
+__device__ __forceinline__ Acc fold_groups(Acc v, Acc* red, int lane, int bk, int G) {
+  red[lane] = v;
+  wave_lds_sync();
+  Acc sum = Acc(0);
+  for (int h0 = 0; h0 < G; h0 += 8) {
+    Acc p[8];
+#pragma unroll
+    for (int h = 0; h < 8; ++h) p[h] = red[h0 + h < G ? ((h0 + h) * bk + lane) & 63 : lane];
+#pragma unroll
+    for (int h = 0; h < 8; ++h) sum += h0 + h < G ? p[h] : Acc(0);
+  }
+  wave_lds_sync();
+  return sum;
+}
+
+template <class TA, class TX>
+__global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free_var(SweepJob<TX> jb) {
+  if (jb.skip && *jb.skip) return;
+  using Acc = typename AccOf<TX>::type;
+  __shared__ TX lds[kSweepWaves][64 + kVarChunk];
+  __shared__ Acc fold[kSweepWaves][64];
+  const int pos = sweep_position(jb);
+  if (pos < 0) return;  // wave-uniform; no workgroup-level synchronisation below
+  const int lane = threadIdx.x & 63;
+  TX* s = lds[threadIdx.x >> 6];
+  Acc* red = fold[threadIdx.x >> 6];
+  const bool second = pos >= jb.npos;
+  const int tp = second ? pos - jb.npos : pos, t = tp / jb.ng;
+  const size_t q0 = (size_t)(tp - t * jb.ng) * jb.n;
+  const int* order = second ? jb.d1.order : jb.d0.order;
+  const int fwd = second ? jb.d1.forward : jb.d0.forward;
+  const int* __restrict__ ia = second ? jb.d1.ia : jb.d0.ia;
+  const int* __restrict__ ja = second ? jb.d1.ja : jb.d0.ja;
+  const int* __restrict__ sp = second ? jb.d1.sp : jb.d0.sp;
+  TX* y = (second ? jb.y1 : jb.y0) + q0;
+  const TX* xw = second ? jb.y0 + q0 : nullptr;
+  const char* x = static_cast<const char*>(jb.x) + q0 * (jb.x64 ? sizeof(double) : sizeof(TX));
+  const int row = order ? order[t] : (fwd ? t : jb.nsup - 1 - t);
+  const int r0 = sp[row], bk = sp[row + 1] - r0;
+  const int G = 64 / bk;
+  const bool act = lane < G * bk;
+  const int g = act ? lane / bk : 0, r = act ? lane - g * bk : 0;
+  const TA* val = static_cast<const TA*>(second ? jb.d1.off : jb.d0.off) + (second ? jb.d1.roff : jb.d0.roff)[row] + r;
+  const TA* d = static_cast<const TA*>(second ? jb.d1.diag : jb.d0.diag) + (second ? jb.d1.dgo : jb.d0.dgo)[row] + r;
+  TA pd[kVarHeld], av[kVarHeld];
+#pragma unroll
+  for (int i = 0; i < kVarHeld; ++i) {
+    const int c = g + i * G;
+    pd[i] = TA(0);
+    if (act && c < bk) pd[i] = __builtin_nontemporal_load(d + (size_t)c * bk);
+  }
+  int c0 = ia[row], W = ia[row + 1] - c0;
+  Acc acc = Acc(0);
+  for (; W > kVarChunk; W -= kVarChunk, c0 += kVarChunk, val += (size_t)kVarChunk * bk) {
+    stage_var<TX>(kVarChunk, ja + c0, y, 0, 0, x, jb.x64, xw, s, jb.ctl);
+    if (act)
+      for (int c = g; c < kVarChunk; c += G) acc += (Acc)ldnt(val + (size_t)c * bk) * (Acc)s[64 + c];
+    wave_lds_sync();
+  }
+#pragma unroll
+  for (int i = 0; i < kVarHeld; ++i) {
+    const int c = g + i * G;
+    av[i] = TA(0);
+    if (act && c < W) av[i] = __builtin_nontemporal_load(val + (size_t)c * bk);
+  }
+  stage_var<TX>(W, ja + c0, y, r0, bk, x, jb.x64, xw, s, jb.ctl);
+#pragma unroll
+  for (int i0 = 0; i0 < kVarHeld; i0 += 4)
+    if (i0 * G < W) {
+#pragma unroll
+      for (int i = i0; i < i0 + 4; ++i) {
+        const int c = g + i * G;
+        acc += (Acc)ldv(&av[i]) * (c < W ? (Acc)s[64 + c] : Acc(0));
+      }
+    }
+  if (act)
+    for (int c = g + kVarHeld * G; c < W; c += G) acc += (Acc)ldnt(val + (size_t)c * bk) * (Acc)s[64 + c];
+  Acc sum = fold_groups(acc, red, lane, bk, G);
+  if (lane < bk) s[lane] = (TX)((Acc)s[lane] - sum);
+  wave_lds_sync();
+  acc = Acc(0);
+#pragma unroll
+  for (int i0 = 0; i0 < kVarHeld; i0 += 4)
+    if (i0 * G < bk) {
+#pragma unroll
+      for (int i = i0; i < i0 + 4; ++i) {
+        const int c = g + i * G;
+        acc += (Acc)ldv(&pd[i]) * (c < bk ? (Acc)s[c] : Acc(0));
+      }
+    }
+  if (act)
+    for (int c = g + kVarHeld * G; c < bk; c += G) acc += (Acc)ldnt(d + (size_t)c * bk) * (Acc)s[c];
+  sum = fold_groups(acc, red, lane, bk, G);
+  if (lane < bk) {
+    st_coherent(&y[r0 + lane], (TX)sum);
+    if (second && jb.out) jb.out[q0 + r0 + lane] = (double)(TX)sum;
   }
 }
 
@@ -1580,6 +1749,23 @@ static void build_tri_var(const BlockCsr& f, bool forward, int prec, DevTri& t) 
   t.sp.upload(f.sprnd.data(), f.sprnd.size() * 4);
   t.doff.upload(doff.data(), std::max<size_t>(doff.size(), 1) * 8);
   t.dgo.upload(dgo.data(), dgo.size() * 8);
+  // the vector element of every column of a row's dependency blocks (which are
+  // stored one after another), for the sync-free sweep
+  std::vector<int> cptr(ns + 1, 0), ccol;
+  std::vector<int64_t> roff(ns, 0);
+  int64_t ncol = 0;
+  for (int j : ja) ncol += f.bla(j);
+  if (ncol > INT32_MAX) return;
+  ccol.reserve(ncol);
+  for (int k = 0; k < ns; ++k) {
+    if (ia[k] < ia[k + 1]) roff[k] = doff[ia[k]];
+    for (int j = ia[k]; j < ia[k + 1]; ++j)
+      for (int c = f.sprnd[ja[j]]; c < f.sprnd[ja[j] + 1]; ++c) ccol.push_back(c);
+    cptr[k + 1] = (int)ccol.size();
+  }
+  t.cptr.upload(cptr.data(), cptr.size() * 4);
+  t.ccol.upload(ccol.data(), std::max<size_t>(ccol.size(), 1) * 4);
+  t.roff.upload(roff.data(), std::max<size_t>(roff.size(), 1) * 8);
 }
 
 template <class TA, class TX>
@@ -2191,6 +2377,12 @@ static bool sweep_split_columns(const DevTri& T, int nrhs) {
   return level_rows * nrhs <= 4LL * device_cu_count();
 }
 
+// Whether a factor of any block partition takes the sync-free sweep: where its
+// column list and the positions of nrhs columns fit 32-bit indices.
+static bool sweep_var_listed(const DevTri& T, int nrhs) {
+  return T.cptr.p && (int64_t)T.nsup * nrhs * 2 <= INT32_MAX - kSweepWaves;
+}
+
 // A set of sweeps of one launch: the first over T1, the second (if T2) over T2.
 struct SweepLaunch {
   const DevTri* T1;
@@ -2213,6 +2405,15 @@ static SweepDir sweep_dir(const DevTri& T, const SweepSync& sync) {
   d.off = T.off.p;
   d.diag = T.diag.p;
   d.forward = T.forward ? 1 : 0;
+  d.sp = nullptr;
+  d.roff = d.dgo = nullptr;
+  if (T.b == 0) {
+    d.ia = T.cptr.as<int>();
+    d.ja = T.ccol.as<int>();
+    d.sp = T.sp.as<int>();
+    d.roff = T.roff.as<int64_t>();
+    d.dgo = T.dgo.as<int64_t>();
+  }
   return d;
 }
 
@@ -2278,6 +2479,11 @@ static void sweep_free_cx(const SweepLaunch& l, int nrhs) {
   }
 }
 
+template <class TA, class TX>
+static void sweep_free_var(const SweepLaunch& l, int nrhs) {
+  sweep_launch<TX>(k_sweep_free_var<TA, TX>, l, 0, 1, nrhs);
+}
+
 template <int B, int NR, class TA, class TX>
 static void sweep_b(const DevTri& T, const void* x, void* y, hipStream_t s, const int* skip, RowGate gate) {
   const int* rows = T.level_rows.as<int>();
@@ -2332,7 +2538,8 @@ static void sweep_cx_level(const DevTri& T, const double* x, double* y, hipStrea
   jb.phases = 1;
   jb.x64 = 1;
   jb.fixed = 1;
-  jb.d0 = SweepDir{nullptr, T.ia.as<int>(), T.ja.as<int>(), T.off.p, T.diag.p, T.forward ? 1 : 0};
+  jb.d0 = SweepDir{nullptr, T.ia.as<int>(), T.ja.as<int>(), T.off.p, T.diag.p, T.forward ? 1 : 0,
+                   nullptr, nullptr, nullptr};
   jb.x = x;
   jb.y0 = y;
   jb.ctl = T.lctl.as<int>();
@@ -2368,6 +2575,13 @@ static void sweep_cx(const SweepLaunch& l, int nrhs) {
 static void sweep_dispatch(const SweepLaunch& l, int vec_prec, int nrhs, RowGate gate) {
   const DevTri& T = *l.T1;
   if (l.sync) l.sync->ensure(T.nsup, l.s);
+  if (T.b == 0) {
+    if (T.prec == kF64 && vec_prec == kF64) sweep_free_var<double, double>(l, nrhs);
+    else if (T.prec == kF32 && vec_prec == kF32) sweep_free_var<float, float>(l, nrhs);
+    else if (T.prec == kBF16 && vec_prec == kF32) sweep_free_var<uint16_t, float>(l, nrhs);
+    else throw Error(kErrArg, "unsupported factor/vector precision pair (fp64/fp64, fp32/fp32, bf16/fp32)");
+    return;
+  }
   if (T.cplx) {
     if (gate.active) throw Error(kErrArg, "row-gated sweeps are not defined for complex factors");
     if (vec_prec != kF64) throw Error(kErrArg, "complex factors sweep FP64 vectors");
@@ -2398,8 +2612,8 @@ static void sweep_dispatch(const SweepLaunch& l, int vec_prec, int nrhs, RowGate
 void launch_sweep(const DevTri& T, const void* x, void* y, int vec_prec, int nrhs, hipStream_t s,
                   const int* skip, SweepSync* sync, RowGate gate) {
   if (x == y) throw Error(kErrArg, "triangular sweep: input and output must not alias");
-  if (T.b == 0) {  // variable blocks: level by level whatever the schedule
-    if (gate.active) throw Error(kErrArg, "row-gated sweeps need a uniform tuned block size");
+  if (T.b == 0 && gate.active) throw Error(kErrArg, "row-gated sweeps need a uniform tuned block size");
+  if (T.b == 0 && !(sync && sweep_var_listed(T, nrhs))) {
     launch_sweep_var(T, x, y, vec_prec, nrhs, s, skip);
     return;
   }
@@ -2412,7 +2626,8 @@ void launch_sweep_pair(const DevTri& T1, const DevTri& T2, const double* r, doub
   const char *rb = reinterpret_cast<const char*>(r), *zb = reinterpret_cast<const char*>(z);
   const bool apart = rb + vb <= zb || zb + vb <= rb;
   // In one launch z is filled before r is read and written while it still is.
-  if (sync && T1.b && T1.b == T2.b && T1.nsup == T2.nsup && T1.cplx == T2.cplx && T1.prec == T2.prec &&
+  const bool listed = T1.b || (sweep_var_listed(T1, nrhs) && sweep_var_listed(T2, nrhs));
+  if (sync && listed && T1.b == T2.b && T1.nsup == T2.nsup && T1.cplx == T2.cplx && T1.prec == T2.prec &&
       apart) {
     void* y1 = vec_prec == kF64 ? static_cast<void*>(z) : w1;
     double* out = vec_prec == kF64 ? nullptr : z;

@@ -147,3 +147,31 @@ def test_syncfree_complex_wide_levels(B, fctx):
         fctx.sync()
         lctx.sync()
         assert rel(dz.host(), dl.host()) < 1e-13
+
+
+# Any block partition: one-row blocks, the largest (64), and rows whose
+# dependencies span more columns than are staged at a time (8 x 64 > 192).
+@pytest.mark.parametrize("blocks,size,ngroup,nrhs", [
+    ([1], 3, 40, 1), ([64, 1, 33], 9, 6, 2), ([5, 7, 14, 11], 4, 50, 1), ([10], 9, 20, 3), ([64], 5, 4, 6)])
+def test_syncfree_any_partition_matches_level_schedule(B, fctx, blocks, size, ngroup, nrhs):
+    m, f = coupled_groups(B, size, ngroup, blocks, seed=3)
+    print(f"any partition {blocks} groups {ngroup} x {size} nrhs={nrhs}", flush=True)
+    r = np.random.default_rng(7).standard_normal((m.n, nrhs))
+    lctx = B.Context()
+    lctx.set_sweep_mode(0)
+    for precision, tol in ((0, 1e-13), (1, 2e-5), (2, 2e-5)):
+        for transpose in (False, True):
+            dr, dz, dl = dev(B, r), B.DeviceArray((m.n, nrhs)), B.DeviceArray((m.n, nrhs))
+            fctx.precond(f, dr, dz, nrhs, precision=precision, transpose=transpose)
+            lctx.precond(f, dr, dl, nrhs, precision=precision, transpose=transpose)
+            fctx.sync()
+            lctx.sync()
+            assert rel(dz.host(), dl.host()) < tol
+        dy, dm = B.DeviceArray((m.n, nrhs)), B.DeviceArray((m.n, nrhs))
+        if precision == 0:
+            for fn in ("solve_l", "solve_u"):
+                getattr(fctx, fn)(f, 1, dr, dy, nrhs)
+                getattr(lctx, fn)(f, 1, dr, dm, nrhs)
+                fctx.sync()
+                lctx.sync()
+                assert rel(dy.host(), dm.host()) < 1e-13
