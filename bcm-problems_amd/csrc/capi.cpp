@@ -1036,10 +1036,11 @@ int bcm_mlp_forward(bcm_context c, bcm_mlp m, int batch, const float* x, float* 
 int bcm_mlp_backward(bcm_context c, bcm_mlp m, int batch, const float* x, const float* t, double* loss) {
   return guarded([&] {
     need(c && m && x && t && batch > 0, "mlp_backward: bad argument");
-    double* dl = c->c.vec(60, 16);
+    // the last kernel writes the loss into pinned host memory: no copy behind it
+    double* dl = &c->c.host_state->sc[0];
     m->m->backward(c->c.stream, batch, x, t, dl);
     BCM_HIP(hipStreamSynchronize(c->c.stream));
-    if (loss) BCM_HIP(hipMemcpy(loss, dl, 8, hipMemcpyDeviceToHost));
+    if (loss) *loss = *dl;
   });
 }
 

@@ -167,6 +167,303 @@ __global__ void k_to_bf16(int64_t n, const float* __restrict__ w, unsigned short
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) wb[i] = f2bf(w[i]);
 }
 
+// ---- the network in fused kernels ----
+//
+// At the sizes a guess model has (a few hundred neurons, up to some thousand
+// cells) a training step is 1 GFLOP over 1 MB: as one launch per product, bias
+// sum and reduction (21 of them) it took 263 us at 1024 x 4-256-256-384, all of
+// it launches and gathers of 2-byte operands. It is now three launches:
+//  * k_mlp_chain: 16 rows of the batch per workgroup through the whole network,
+//    the loss, and back through the activations; rows stay in LDS.
+//  * k_mlp_wgrad: all weight and bias gradients and the loss sum.
+//  * k_mlp_adam.
+// Operands are kept as MFMA fragments, so that every load is 16 bytes a lane
+// and consecutive over the wave. A fragment holds, for 16 columns j and 32
+// steps k of the contraction, lane (j % 16) + 16 * (k % 32 / 8) its 8 values k
+// % 8; columns and steps past the end are zero. Weights are packed once per
+// update (for the products and, transposed, for the way back); activations and
+// their gradients are written as fragments over the rows of the batch.
+// Chosen where the rows of a workgroup fit 63 KB of LDS; larger networks
+// take one product after another (k_gemm_bf16).
+constexpr int kFrag = 512;            // values of a fragment
+constexpr int kChainThreads = 1024;   // one 16-column tile per wave and pass
+constexpr int kChainWaves = kChainThreads / 64;
+
+__host__ __device__ constexpr int up16(int n) { return (n + 15) & ~15; }
+__host__ __device__ constexpr int up32(int n) { return (n + 31) & ~31; }
+
+// Offset of element (k, j) in fragments of `ks` steps of 32 per column tile.
+__device__ __forceinline__ size_t frag_at(int k, int j, int ks) {
+  return ((size_t)(j >> 4) * ks + (k >> 5)) * kFrag + (size_t)((j & 15) + 16 * ((k & 31) >> 3)) * 8 + (k & 7);
+}
+
+// Sizes and the packed weights: f[l] for the product with W_l, r[l] (layers 1
+// and 2) for the product with its transpose.
+struct MlpDims {
+  int nin, nh, nout;
+  int64_t w_off[3], b_off[3];
+  int64_t f[3], r[3];
+};
+
+__device__ __forceinline__ void pack_weight(const MlpDims& d, int64_t i, unsigned short v, unsigned short* pk) {
+  for (int l = 0; l < 3; ++l) {
+    if (i < d.w_off[l] || i >= d.b_off[l]) continue;
+    const int nj = l == 2 ? d.nout : d.nh, nk = l == 0 ? d.nin : d.nh;
+    const int e = (int)(i - d.w_off[l]), k = e / nj, j = e - k * nj;
+    pk[d.f[l] + frag_at(k, j, up32(nk) >> 5)] = v;
+    if (l > 0) pk[d.r[l] + frag_at(j, k, up32(nj) >> 5)] = v;
+  }
+}
+
+__global__ void k_mlp_pack(int64_t n, MlpDims d, const float* __restrict__ w, unsigned short* __restrict__ pk) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) pack_weight(d, i, f2bf(w[i]), pk);
+}
+
+// What a pass over the batch leaves for the gradients: fragments over the rows
+// (the k of the gradient products) and per-16-row sums.
+struct MlpTape {
+  unsigned short *x, *h1, *h2, *dz1, *dz2, *dy;
+  float* colpart;    // per row tile: column sums of dz1, dz2, dy
+  double* losspart;  // per row tile: sum of squared errors
+};
+
+// acc of the tiles tn = wave, wave + kChainWaves, ... of A (16 rows in LDS, ks
+// steps of 32) times packed weights, handed to `epi(tn, acc)`.
+template <class F>
+__device__ __forceinline__ void chain_product(const unsigned short* a, int lda, const unsigned short* __restrict__ w,
+                                              int ks, int tiles, F epi) {
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const unsigned short* ar = a + r * lda + 8 * g;
+  for (int tn = threadIdx.x >> 6; tn < tiles; tn += kChainWaves) {
+    const v8u* wp = reinterpret_cast<const v8u*>(w + (size_t)tn * ks * kFrag) + lane;
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int k = 0; k < ks; ++k) {
+      const v8u bv = wp[k * 64];
+      const v8u av = *reinterpret_cast<const v8u*>(ar + 32 * k);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, av), __builtin_bit_cast(v8bf, bv), acc,
+                                                    0, 0, 0);
+    }
+    epi(tn, acc);
+  }
+}
+
+// This lane's four rows (4g .. 4g + 3 of the tile at m0) of column tile tn as
+// a fragment over ms steps of 32 rows.
+__device__ __forceinline__ void store_frag(unsigned short* f, int tn, int ms, int m0, const float (&v)[4]) {
+  const int lane = threadIdx.x & 63, m = (m0 & 31) + 4 * (lane >> 4);
+  ushort4 b;
+  b.x = f2bf(v[0]);
+  b.y = f2bf(v[1]);
+  b.z = f2bf(v[2]);
+  b.w = f2bf(v[3]);
+  const size_t o = ((size_t)tn * ms + (m0 >> 5)) * kFrag + (size_t)((lane & 15) + 16 * (m >> 3)) * 8 + (m & 7);
+  *reinterpret_cast<ushort4*>(f + o) = b;
+}
+
+// Sums over the tile's 16 rows (valid in lanes < 16).
+__device__ __forceinline__ float tile_colsum(const float (&v)[4]) {
+  float s = (v[0] + v[1]) + (v[2] + v[3]);
+  s += __shfl_xor(s, 16);
+  s += __shfl_xor(s, 32);
+  return s;
+}
+
+// LDS bytes of a chain workgroup: h1 and h2 in FP32, the BF16 operands x, h1
+// (then dz2), h2 and dy, rows 8 values apart in the banks.
+size_t chain_lds(int nin, int nh, int nout) {
+  return (size_t)16 * (2 * 4 * up16(nh) + 2 * (up32(nin) + 8 + 2 * (up32(nh) + 8) + up32(nout) + 8));
+}
+
+// Rows [16 * blockIdx.x, + 16) of the batch: out = MLP(x) if t is null, else
+// the loss against t, the activations' gradients and the tape.
+__global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int M, int ms, MlpDims d, const float* __restrict__ p,
+                                                             const unsigned short* __restrict__ pk,
+                                                             const float* __restrict__ x, const float* __restrict__ t,
+                                                             float* __restrict__ out, float scale, MlpTape tape) {
+  extern __shared__ __align__(16) char smem[];
+  const int hc = up16(d.nh), lx = up32(d.nin) + 8, lh = up32(d.nh) + 8, ly = up32(d.nout) + 8;
+  float* h1f = reinterpret_cast<float*>(smem);
+  float* h2f = h1f + 16 * hc;
+  unsigned short* xb = reinterpret_cast<unsigned short*>(h2f + 16 * hc);
+  unsigned short* h1b = xb + 16 * lx;
+  unsigned short* h2b = h1b + 16 * lh;
+  unsigned short* dyb = h2b + 16 * lh;
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int m0 = blockIdx.x * 16;
+  // operands: x in BF16, zeros in the padding that no product writes
+  for (int e = threadIdx.x; e < 16 * lx; e += kChainThreads) {
+    const int i = e / lx, k = e - i * lx;
+    xb[e] = m0 + i < M && k < d.nin ? f2bf(x[(size_t)(m0 + i) * d.nin + k]) : (unsigned short)0;
+  }
+  for (int e = threadIdx.x; e < 16 * (2 * lh + ly); e += kChainThreads) h1b[e] = 0;
+  __syncthreads();
+  const int ki = up32(d.nin) >> 5, kh = up32(d.nh) >> 5, ko = up32(d.nout) >> 5, th = hc >> 4, to = up16(d.nout) >> 4;
+  if (t) {  // x over the rows, for dW1
+    for (int e = threadIdx.x; e < 16 * up16(d.nin); e += kChainThreads) {
+      const int k = e >> 4, i = e & 15;
+      tape.x[frag_at(m0 + i, k, ms)] = xb[i * lx + k];
+    }
+  }
+  auto hidden = [&](const unsigned short* a, int lda, int ks, int l, float* hf, unsigned short* hb,
+                    unsigned short* frag) {
+    const float* b = p + d.b_off[l];
+    chain_product(a, lda, pk + d.f[l], ks, th, [&](int tn, v4f acc) {
+      const int j = tn * 16 + r;
+      const float bj = j < d.nh ? b[j] : 0.f;
+      float v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        v[q] = j < d.nh ? tanhf(acc[q] + bj) : 0.f;
+        hf[(4 * g + q) * hc + j] = v[q];
+        hb[(4 * g + q) * lh + j] = f2bf(v[q]);
+      }
+      if (t) store_frag(frag, tn, ms, m0, v);
+    });
+    __syncthreads();
+  };
+  hidden(xb, lx, ki, 0, h1f, h1b, tape.h1);
+  hidden(h1b, lh, kh, 1, h2f, h2b, tape.h2);
+  double loss = 0.0;
+  float* cp = t ? tape.colpart + (size_t)blockIdx.x * (2 * d.nh + d.nout) : nullptr;
+  {
+    const float* b = p + d.b_off[2];
+    chain_product(h2b, lh, pk + d.f[2], kh, to, [&](int tn, v4f acc) {
+      const int j = tn * 16 + r;
+      const float bj = j < d.nout ? b[j] : 0.f;
+      float v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int i = m0 + 4 * g + q;
+        const bool in = i < M && j < d.nout;
+        const float y = acc[q] + bj;
+        v[q] = 0.f;
+        if (!t) {
+          if (in) out[(size_t)i * d.nout + j] = y;
+        } else if (in) {
+          const float e = y - t[(size_t)i * d.nout + j];
+          loss += (double)e * (double)e;
+          v[q] = scale * e;
+        }
+        dyb[(4 * g + q) * ly + j] = f2bf(v[q]);
+      }
+      if (t) {
+        store_frag(tape.dy, tn, ms, m0, v);
+        const float s = tile_colsum(v);
+        if (lane < 16 && j < d.nout) cp[2 * d.nh + j] = s;
+      }
+    });
+  }
+  if (!t) return;  // uniform
+  __shared__ double ls[kChainWaves];
+  for (int o = 32; o > 0; o >>= 1) loss += __shfl_down(loss, o);
+  if (lane == 0) ls[threadIdx.x >> 6] = loss;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+    for (int w = 0; w < kChainWaves; ++w) s += ls[w];
+    tape.losspart[blockIdx.x] = s;
+  }
+  // dz2 = (dy W3^T) * (1 - h2^2) into h1's operand, dz1 = (dz2 W2^T) * (1 - h1^2)
+  chain_product(dyb, ly, pk + d.r[2], ko, th, [&](int tn, v4f acc) {
+    const int j = tn * 16 + r;
+    float v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float h = h2f[(4 * g + q) * hc + j];
+      v[q] = j < d.nh ? acc[q] * (1.0f - h * h) : 0.f;
+      h1b[(4 * g + q) * lh + j] = f2bf(v[q]);
+    }
+    store_frag(tape.dz2, tn, ms, m0, v);
+    const float s = tile_colsum(v);
+    if (lane < 16 && j < d.nh) cp[d.nh + j] = s;
+  });
+  __syncthreads();
+  chain_product(h1b, lh, pk + d.r[1], kh, th, [&](int tn, v4f acc) {
+    const int j = tn * 16 + r;
+    float v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float h = h1f[(4 * g + q) * hc + j];
+      v[q] = j < d.nh ? acc[q] * (1.0f - h * h) : 0.f;
+    }
+    store_frag(tape.dz1, tn, ms, m0, v);
+    const float s = tile_colsum(v);
+    if (lane < 16 && j < d.nh) cp[j] = s;
+  });
+}
+
+// Gradients from the tape. Workgroups [0, ntile): one 16 x 16 tile of dW3 =
+// H2^T dY, dW2 = H1^T dZ2 or dW1 = X^T dZ1, its rows of the batch split over
+// the four waves and added in order (1 KB operands a load, all from L2). Then
+// ones of 64 columns of the bias gradients, and one for the loss.
+__global__ __launch_bounds__(256) void k_mlp_wgrad(int ms, int mt, MlpDims d, MlpTape tape, float* __restrict__ grad,
+                                                   double loss_scale, double* loss) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int th = up16(d.nh) >> 4, to = up16(d.nout) >> 4, ti = up16(d.nin) >> 4;
+  const int n3 = th * to, n2 = th * th, n1 = ti * th;
+  int b = blockIdx.x;
+  if (b < n3 + n2 + n1) {
+    __shared__ float part[4][256];
+    const unsigned short *A, *Bm;
+    int l, tj, ni, nj;
+    if (b < n3) { l = 2; A = tape.h2; Bm = tape.dy; tj = to; ni = d.nh; nj = d.nout; }
+    else if (b < n3 + n2) { b -= n3; l = 1; A = tape.h1; Bm = tape.dz2; tj = th; ni = d.nh; nj = d.nh; }
+    else { b -= n3 + n2; l = 0; A = tape.x; Bm = tape.dz1; tj = th; ni = d.nin; nj = d.nh; }
+    const int bi = b / tj, bj = b - bi * tj;
+    const v8u* ap = reinterpret_cast<const v8u*>(A + (size_t)bi * ms * kFrag) + lane;
+    const v8u* bp = reinterpret_cast<const v8u*>(Bm + (size_t)bj * ms * kFrag) + lane;
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int k = wave; k < ms; k += 4)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, ap[(size_t)k * 64]),
+                                                    __builtin_bit_cast(v8bf, bp[(size_t)k * 64]), acc, 0, 0, 0);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) part[wave][(4 * (lane >> 4) + q) * 16 + (lane & 15)] = acc[q];
+    __syncthreads();
+    const int e = threadIdx.x, i = bi * 16 + (e >> 4), j = bj * 16 + (e & 15);
+    if (i < ni && j < nj)
+      grad[d.w_off[l] + (size_t)i * nj + j] = ((part[0][e] + part[1][e]) + part[2][e]) + part[3][e];
+    return;
+  }
+  b -= n3 + n2 + n1;
+  const int ncol = 2 * d.nh + d.nout, nb = (ncol + 63) / 64;
+  if (b < nb) {
+    __shared__ float sm[4][64];
+    const int c = b * 64 + lane;
+    float s = 0.f;
+    if (c < ncol)
+      for (int k = wave; k < mt; k += 4) s += tape.colpart[(size_t)k * ncol + c];
+    sm[wave][lane] = s;
+    __syncthreads();
+    if (wave == 0 && c < ncol) {
+      const int64_t o = c < d.nh ? d.b_off[0] + c : c < 2 * d.nh ? d.b_off[1] + c - d.nh : d.b_off[2] + c - 2 * d.nh;
+      grad[o] = ((sm[0][lane] + sm[1][lane]) + sm[2][lane]) + sm[3][lane];
+    }
+    return;
+  }
+  const double s = sum_partials(tape.losspart, mt, 1, 0);
+  if (threadIdx.x == 0 && loss) *loss = s * loss_scale;
+}
+
+// Adam step over all parameters; refreshes the packed weights.
+__global__ void k_mlp_adam(int64_t n, MlpDims d, float* __restrict__ w, const float* __restrict__ gr,
+                           float* __restrict__ m, float* __restrict__ v, unsigned short* __restrict__ pk, float lr,
+                           float b1, float b2, float eps, float c1, float c2) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const float g = gr[i];
+    const float mi = b1 * m[i] + (1.f - b1) * g;
+    const float vi = b2 * v[i] + (1.f - b2) * g * g;
+    m[i] = mi;
+    v[i] = vi;
+    const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    w[i] = wi;
+    pack_weight(d, i, f2bf(wi), pk);
+  }
+}
+
 // ---- FP64 tall-skinny products for the POD ----
 
 // Partial C_s = X(rows of split s)^T Y(rows of split s): X n x p, Y n x q
@@ -286,6 +583,29 @@ void gemm(hipStream_t s, int M, int N, int K, const TA* A, int ars, int acs, con
   BCM_HIP(hipGetLastError());
 }
 
+MlpDims mlp_dims(const Mlp& m) {
+  MlpDims d{};
+  d.nin = m.nin;
+  d.nh = m.nh;
+  d.nout = m.nout;
+  int64_t o = 0;
+  for (int l = 0; l < 3; ++l) {
+    d.w_off[l] = m.w_off[l];
+    d.b_off[l] = m.b_off[l];
+    const int nk = l == 0 ? m.nin : m.nh, nj = l == 2 ? m.nout : m.nh;
+    d.f[l] = o;
+    o += (int64_t)up16(nj) * up32(nk);
+    d.r[l] = o;
+    if (l > 0) o += (int64_t)up16(nk) * up32(nj);
+  }
+  return d;
+}
+
+int64_t packed_values(const Mlp& m) {
+  const MlpDims d = mlp_dims(m);
+  return d.r[2] + (int64_t)up16(m.nh) * up32(m.nout);
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -317,6 +637,12 @@ Mlp::Mlp(int nin_, int nh_, int nout_, uint64_t seed) : nin(nin_), nh(nh_), nout
   grads.alloc(nparam * 4);
   m1.alloc(nparam * 4);
   m2.alloc(nparam * 4);
+  fused = chain_lds(nin, nh, nout) <= (size_t)63 << 10;
+  if (fused) {
+    wpk.alloc(packed_values(*this) * 2);
+    set_params(h.data());
+    return;
+  }
   wbf.alloc(nweight * 2);
   std::vector<unsigned char> isw(nparam, 0);
   std::vector<int64_t> idx(nparam, 0);
@@ -335,7 +661,12 @@ void Mlp::set_params(const float* host) {
   BCM_HIP(hipMemset(m1.p, 0, nparam * 4));
   BCM_HIP(hipMemset(m2.p, 0, nparam * 4));
   BCM_HIP(hipMemset(grads.p, 0, nparam * 4));
-  for (int l = 0; l < 3; ++l) {
+  if (fused) {
+    BCM_HIP(hipMemset(wpk.p, 0, wpk.bytes));
+    hipLaunchKernelGGL(k_mlp_pack, dim3(grid1(nparam)), dim3(256), 0, nullptr, nparam, mlp_dims(*this),
+                       params.as<const float>(), wpk.as<unsigned short>());
+  }
+  for (int l = 0; l < 3 && !fused; ++l) {
     const int64_t cnt = b_off[l] - w_off[l];
     hipLaunchKernelGGL(k_to_bf16, dim3(grid1(cnt)), dim3(256), 0, nullptr, cnt, params.as<float>() + w_off[l],
                        wbf.as<unsigned short>() + wb_off[l]);
@@ -346,6 +677,13 @@ void Mlp::set_params(const float* host) {
 
 void Mlp::ensure_batch(int M) {
   if (M <= cap_batch) return;
+  if (fused) {  // the tape: fragments over the rows, padded to whole steps of 32
+    const size_t m32 = up32(M), mt = m32 / 16;
+    const size_t frags = m32 * (up16(nin) + 4 * (size_t)up16(nh) + up16(nout)) * 2;
+    tape.alloc(mt * 8 + frags + mt * (2 * (size_t)nh + nout) * 4);
+    cap_batch = M;
+    return;
+  }
   h1.alloc((size_t)M * nh * 4);
   h2.alloc((size_t)M * nh * 4);
   y.alloc((size_t)M * nout * 4);
@@ -357,7 +695,42 @@ void Mlp::ensure_batch(int M) {
   cap_batch = M;
 }
 
+// One pass of the chain over the batch; t == nullptr: out = MLP(x) only.
+void Mlp::chain(hipStream_t s, int M, const float* x, const float* t, float* out, double* loss_dev) {
+  const MlpDims d = mlp_dims(*this);
+  const int ms = up32(M) >> 5, mt = t ? 2 * ms : (M + 15) / 16;
+  MlpTape tp{};
+  if (t) {
+    ensure_batch(M);
+    const size_t m32 = up32(M);
+    tp.losspart = tape.as<double>();
+    unsigned short* f = reinterpret_cast<unsigned short*>(tp.losspart + mt);
+    tp.x = f;
+    tp.h1 = tp.x + m32 * up16(nin);
+    tp.h2 = tp.h1 + m32 * up16(nh);
+    tp.dz1 = tp.h2 + m32 * up16(nh);
+    tp.dz2 = tp.dz1 + m32 * up16(nh);
+    tp.dy = tp.dz2 + m32 * up16(nh);
+    tp.colpart = reinterpret_cast<float*>(tp.dy + m32 * up16(nout));
+  }
+  const double total = (double)M * nout;
+  hipLaunchKernelGGL(k_mlp_chain, dim3(mt), dim3(kChainThreads), chain_lds(nin, nh, nout), s, M, ms, d,
+                     params.as<const float>(), wpk.as<const unsigned short>(), x, t, out,
+                     2.0f / (float)((int64_t)M * nout), tp);
+  if (t) {
+    const int th = up16(nh) / 16, to = up16(nout) / 16, ti = up16(nin) / 16;
+    const int grid = th * to + th * th + ti * th + (2 * nh + nout + 63) / 64 + 1;
+    hipLaunchKernelGGL(k_mlp_wgrad, dim3(grid), dim3(256), 0, s, ms, mt, d, tp, grads.as<float>(), 1.0 / total,
+                       loss_dev);
+  }
+  BCM_HIP(hipGetLastError());
+}
+
 void Mlp::forward(hipStream_t s, int M, const float* x, float* out) {
+  if (fused && out) {
+    chain(s, M, x, nullptr, out, nullptr);
+    return;
+  }
   ensure_batch(M);
   const float* P = params.as<float>();
   const unsigned short* W = wbf.as<unsigned short>();
@@ -369,6 +742,10 @@ void Mlp::forward(hipStream_t s, int M, const float* x, float* out) {
 }
 
 void Mlp::backward(hipStream_t s, int M, const float* x, const float* t, double* loss_dev) {
+  if (fused) {
+    chain(s, M, x, t, nullptr, loss_dev);
+    return;
+  }
   forward(s, M, x, nullptr);
   float* G = grads.as<float>();
   const unsigned short* W = wbf.as<unsigned short>();
@@ -401,6 +778,13 @@ void Mlp::adam(hipStream_t s, float lr) {
   ++step;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const float c1 = 1.0f - std::pow(b1, (float)step), c2 = 1.0f - std::pow(b2, (float)step);
+  if (fused) {
+    hipLaunchKernelGGL(k_mlp_adam, dim3(grid1(nparam)), dim3(256), 0, s, nparam, mlp_dims(*this), params.as<float>(),
+                       grads.as<const float>(), m1.as<float>(), m2.as<float>(), wpk.as<unsigned short>(), lr, b1, b2,
+                       eps, c1, c2);
+    BCM_HIP(hipGetLastError());
+    return;
+  }
   hipLaunchKernelGGL(k_adam, dim3(grid1(nparam)), dim3(256), 0, s, nparam, params.as<float>(), grads.as<float>(),
                      m1.as<float>(), m2.as<float>(), wbf.as<unsigned short>(), is_w.as<unsigned char>(),
                      wb_index.as<int64_t>(), lr, b1, b2, eps, c1, c2);

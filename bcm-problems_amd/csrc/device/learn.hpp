@@ -21,14 +21,17 @@ struct Mlp {
   DevBuf h1, h2, y, dz1, dz2, dy, partials, colpart, kpart;
   int cap_batch = 0;
   int step = 0;  // Adam steps taken
+  bool fused = false;  // a workgroup's rows fit its LDS: packed weights and the fused kernels
+  DevBuf wpk, tape;    // fused: weights and the last pass as MFMA fragments
   Mlp(int nin, int nh, int nout, uint64_t seed);
   void set_params(const float* host);  // also resets the Adam moments
   void ensure_batch(int M);
-  // out (M x nout) = MLP(x); out == nullptr keeps the result in y.
+  // out (M x nout) = MLP(x); out == nullptr (networks that are not fused) keeps the result in y.
   void forward(hipStream_t s, int M, const float* x, float* out);
   // Gradients of mean((MLP(x) - t)^2) into grads; loss_dev (may be null) receives the loss.
   void backward(hipStream_t s, int M, const float* x, const float* t, double* loss_dev);
   void adam(hipStream_t s, float lr);
+  void chain(hipStream_t s, int M, const float* x, const float* t, float* out, double* loss_dev);
 };
 
 // C (p x q) = X^T Y for tall X (n x p), Y (n x q), column-major with leading

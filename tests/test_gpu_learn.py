@@ -131,3 +131,36 @@ def test_learned_guess_beats_zero_guess(B, ctx):
     print(f"guess rel err {err:.3e}; iterations zero {its0.mean():.1f} learned {its1.mean():.1f}", flush=True)
     assert err < 0.3
     assert its1.mean() < its0.mean()
+
+
+# Fused kernels: sizes around the 16-column and 32-step tiles, batches around
+# the 16- and 32-row ones; the last two networks take the separate products.
+@pytest.mark.parametrize("dims,batch", [((1, 1, 1), 1), ((4, 16, 16), 16), ((5, 17, 33), 31), ((33, 200, 47), 33),
+                                        ((4, 256, 384), 1024), ((2, 31, 500), 100), ((8, 300, 40), 77),
+                                        ((200, 64, 700), 65)])
+def test_mlp_sizes_match_oracle(B, ctx, dims, batch):
+    print(f"mlp {dims} batch {batch}", flush=True)
+    m = B.Mlp(*dims, seed=9)
+    rng = np.random.default_rng(sum(dims) + batch)
+    offs, npar = M.layout(*dims)
+    p = (rng.normal(size=npar) / np.sqrt(max(dims[1], dims[0]))).astype(np.float32)
+    m.set_params(p)
+    x = rng.normal(size=(batch, dims[0])).astype(np.float32)
+    t = rng.normal(size=(batch, dims[2])).astype(np.float32)
+    yo, _ = M.forward(p.astype(np.float64), x.astype(np.float64), *dims, bf16=True)
+    # operands that round to the other BF16 neighbour after FP32 sums: 2^-9 each, over the few that are that close
+    assert relerr(m.forward(ctx, x), yo) < 1e-3
+    for _ in range(2):  # the second pass over the same buffers
+        loss = m.backward(ctx, x, t)
+        lo, go = M.loss_grad(p.astype(np.float64), x.astype(np.float64), t.astype(np.float64), *dims, bf16=True)
+        g = m.grads().astype(np.float64)
+        assert abs(loss - lo) <= 1e-4 * lo
+        for name, (o, shp) in zip(["W1", "b1", "W2", "b2", "W3", "b3"], offs):
+            k = int(np.prod(shp))
+            assert relerr(g[o:o + k], go[o:o + k]) < 2e-3, name
+    p0, zero = m.params().astype(np.float64), np.zeros(npar)
+    m.adam_step(ctx, 1e-2)
+    pn, _, _ = M.adam(p0, g, zero, zero, 1, 1e-2)
+    assert relerr(m.params(), pn) < 1e-6
+    y1, _ = M.forward(m.params().astype(np.float64), x.astype(np.float64), *dims, bf16=True)
+    assert relerr(m.forward(ctx, x), y1) < 1e-3  # the packed weights follow the update
