@@ -228,22 +228,49 @@ struct MlpTape {
   double* losspart;  // per row tile: sum of squared errors
 };
 
+// Up to kChainHeld fragments of column tile tn, from step k0 on. A layer is a
+// few steps long, so a workgroup's time is the latency of its weights (the
+// other XCDs' last update, from beyond the L2): a wave loads a whole group at
+// once, and the first group of the next layer while it works on this one.
+constexpr int kChainHeld = 8;
+struct ChainHeld {
+  v8u b[kChainHeld];
+};
+__device__ __forceinline__ ChainHeld chain_load(const unsigned short* __restrict__ w, int ks, int tiles, int tn,
+                                                int k0) {
+  ChainHeld h;
+  const v8u* wp = reinterpret_cast<const v8u*>(w + (size_t)tn * ks * kFrag) + (threadIdx.x & 63);
+#pragma unroll
+  for (int q = 0; q < kChainHeld; ++q) {
+    h.b[q] = v8u{};
+    if (tn < tiles && k0 + q < ks) h.b[q] = wp[(k0 + q) * 64];
+  }
+  return h;
+}
+__device__ __forceinline__ ChainHeld chain_first(const unsigned short* __restrict__ w, int ks, int tiles) {
+  return chain_load(w, ks, tiles, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), 0);
+}
+
 // acc of the tiles tn = wave, wave + kChainWaves, ... of A (16 rows in LDS, ks
-// steps of 32) times packed weights, handed to `epi(tn, acc)`.
+// steps of 32) times packed weights, handed to `epi(tn, acc)`; `held` is the
+// wave's chain_first of these weights.
 template <class F>
 __device__ __forceinline__ void chain_product(const unsigned short* a, int lda, const unsigned short* __restrict__ w,
-                                              int ks, int tiles, F epi) {
+                                              int ks, int tiles, ChainHeld held, F epi) {
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const unsigned short* ar = a + r * lda + 8 * g;
-  for (int tn = threadIdx.x >> 6; tn < tiles; tn += kChainWaves) {
-    const v8u* wp = reinterpret_cast<const v8u*>(w + (size_t)tn * ks * kFrag) + lane;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int tn = wave; tn < tiles; tn += kChainWaves) {
     v4f acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-    for (int k = 0; k < ks; ++k) {
-      const v8u bv = wp[k * 64];
-      const v8u av = *reinterpret_cast<const v8u*>(ar + 32 * k);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, av), __builtin_bit_cast(v8bf, bv), acc,
-                                                    0, 0, 0);
+    for (int k0 = 0; k0 < ks; k0 += kChainHeld) {
+      if (tn != wave || k0) held = chain_load(w, ks, tiles, tn, k0);
+#pragma unroll
+      for (int q = 0; q < kChainHeld; ++q)
+        if (k0 + q < ks) {
+          const v8u av = *reinterpret_cast<const v8u*>(ar + 32 * (k0 + q));
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, av),
+                                                        __builtin_bit_cast(v8bf, held.b[q]), acc, 0, 0, 0);
+        }
     }
     epi(tn, acc);
   }
@@ -292,6 +319,8 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int M, int ms, MlpD
   unsigned short* dyb = h2b + 16 * lh;
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int m0 = blockIdx.x * 16;
+  const int ki = up32(d.nin) >> 5, kh = up32(d.nh) >> 5, ko = up32(d.nout) >> 5, th = hc >> 4, to = up16(d.nout) >> 4;
+  const ChainHeld w1 = chain_first(pk + d.f[0], ki, th), w2 = chain_first(pk + d.f[1], kh, th);
   // operands: x in BF16, zeros in the padding that no product writes
   for (int e = threadIdx.x; e < 16 * lx; e += kChainThreads) {
     const int i = e / lx, k = e - i * lx;
@@ -299,17 +328,16 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int M, int ms, MlpD
   }
   for (int e = threadIdx.x; e < 16 * (2 * lh + ly); e += kChainThreads) h1b[e] = 0;
   __syncthreads();
-  const int ki = up32(d.nin) >> 5, kh = up32(d.nh) >> 5, ko = up32(d.nout) >> 5, th = hc >> 4, to = up16(d.nout) >> 4;
   if (t) {  // x over the rows, for dW1
     for (int e = threadIdx.x; e < 16 * up16(d.nin); e += kChainThreads) {
       const int k = e >> 4, i = e & 15;
       tape.x[frag_at(m0 + i, k, ms)] = xb[i * lx + k];
     }
   }
-  auto hidden = [&](const unsigned short* a, int lda, int ks, int l, float* hf, unsigned short* hb,
-                    unsigned short* frag) {
+  auto hidden = [&](const unsigned short* a, int lda, int ks, int l, const ChainHeld& held, float* hf,
+                    unsigned short* hb, unsigned short* frag) {
     const float* b = p + d.b_off[l];
-    chain_product(a, lda, pk + d.f[l], ks, th, [&](int tn, v4f acc) {
+    chain_product(a, lda, pk + d.f[l], ks, th, held, [&](int tn, v4f acc) {
       const int j = tn * 16 + r;
       const float bj = j < d.nh ? b[j] : 0.f;
       float v[4];
@@ -323,13 +351,15 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int M, int ms, MlpD
     });
     __syncthreads();
   };
-  hidden(xb, lx, ki, 0, h1f, h1b, tape.h1);
-  hidden(h1b, lh, kh, 1, h2f, h2b, tape.h2);
+  hidden(xb, lx, ki, 0, w1, h1f, h1b, tape.h1);
+  const ChainHeld w3 = chain_first(pk + d.f[2], kh, to);
+  hidden(h1b, lh, kh, 1, w2, h2f, h2b, tape.h2);
+  const ChainHeld r3 = chain_first(pk + d.r[2], ko, t ? th : 0);
   double loss = 0.0;
   float* cp = t ? tape.colpart + (size_t)blockIdx.x * (2 * d.nh + d.nout) : nullptr;
   {
     const float* b = p + d.b_off[2];
-    chain_product(h2b, lh, pk + d.f[2], kh, to, [&](int tn, v4f acc) {
+    chain_product(h2b, lh, pk + d.f[2], kh, to, w3, [&](int tn, v4f acc) {
       const int j = tn * 16 + r;
       const float bj = j < d.nout ? b[j] : 0.f;
       float v[4];
@@ -356,6 +386,7 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int M, int ms, MlpD
     });
   }
   if (!t) return;  // uniform
+  const ChainHeld r2 = chain_first(pk + d.r[1], kh, th);
   __shared__ double ls[kChainWaves];
   for (int o = 32; o > 0; o >>= 1) loss += __shfl_down(loss, o);
   if (lane == 0) ls[threadIdx.x >> 6] = loss;
@@ -366,7 +397,7 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int M, int ms, MlpD
     tape.losspart[blockIdx.x] = s;
   }
   // dz2 = (dy W3^T) * (1 - h2^2) into h1's operand, dz1 = (dz2 W2^T) * (1 - h1^2)
-  chain_product(dyb, ly, pk + d.r[2], ko, th, [&](int tn, v4f acc) {
+  chain_product(dyb, ly, pk + d.r[2], ko, th, r3, [&](int tn, v4f acc) {
     const int j = tn * 16 + r;
     float v[4];
 #pragma unroll
@@ -380,7 +411,7 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int M, int ms, MlpD
     if (lane < 16 && j < d.nh) cp[d.nh + j] = s;
   });
   __syncthreads();
-  chain_product(h1b, lh, pk + d.r[1], kh, th, [&](int tn, v4f acc) {
+  chain_product(h1b, lh, pk + d.r[1], kh, th, r2, [&](int tn, v4f acc) {
     const int j = tn * 16 + r;
     float v[4];
 #pragma unroll
