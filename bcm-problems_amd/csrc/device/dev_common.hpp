@@ -36,6 +36,11 @@ template <class T> __device__ __forceinline__ void st_coherent(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Step seq of a solve has ended; `done` tells whether the solve has (one thread).
+__device__ __forceinline__ void publish_done(uint64_t* poll, uint64_t seq, int done) {
+  __hip_atomic_store(poll, seq << 1 | (done ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Orders this wave's LDS writes before its following LDS reads by other
 // lanes (and reads before later writes). LDS operations of one wave complete
 // in program order, so a wavefront-scope fence, which only stops the compiler

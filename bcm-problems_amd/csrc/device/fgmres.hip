@@ -194,11 +194,9 @@ __global__ __launch_bounds__(256) void k_gs_update(int64_t n, const KState* ks, 
 // Arnoldi step j: partials hold ||w||^2 of the orthogonalised vector. Builds
 // column j of H (h1 + h2, norm), applies the earlier rotations, forms the new
 // one, updates g and decides whether the cycle ends.
-__global__ __launch_bounds__(256) void k_gm_step(KState* ks, double* gm, GmLayout L, const double* partials,
-                                                 int nb, int j, double eps, int ittype, int steps_left) {
-  if (ks->st[kStCycleEnd]) return;
-  const double ww = sum_partials(partials, nb, 1, 0);
-  if (threadIdx.x != 0) return;
+// The end of the cycle is published to the host at step `seq`.
+__device__ void gm_step(KState* ks, double* gm, GmLayout L, double ww, int j, double eps, int ittype,
+                        int steps_left) {
   int* st = ks->st;
   const int m = L.m;
   double* col = gm + L.H() + (size_t)j * (m + 1);
@@ -242,6 +240,19 @@ __global__ __launch_bounds__(256) void k_gm_step(KState* ks, double* gm, GmLayou
     st[kStCycleEnd] = 1;
     st[kStDone] = 1;
   }
+}
+
+__global__ __launch_bounds__(256) void k_gm_step(KState* ks, double* gm, GmLayout L, const double* partials,
+                                                 int nb, int j, double eps, int ittype, int steps_left,
+                                                 uint64_t* poll, uint64_t seq) {
+  if (ks->st[kStCycleEnd]) {
+    if (threadIdx.x == 0) publish_done(poll, seq, 1);
+    return;
+  }
+  const double ww = sum_partials(partials, nb, 1, 0);
+  if (threadIdx.x != 0) return;
+  gm_step(ks, gm, L, ww, j, eps, ittype, steps_left);
+  publish_done(poll, seq, ks->st[kStCycleEnd]);
 }
 
 // Least squares: y = R^-1 g over the cycle's columns (upper triangular R in H).
@@ -340,11 +351,13 @@ void solve_fgmres(Matrix& A, Factor& F, Context& ctx, const SolveOptions& opt, c
       }
       gram_schmidt(n, ks, V, j + 1, w, gm, L, partials, nb, s);
       hipLaunchKernelGGL(k_gm_step, dim3(1), dim3(256), 0, s, ks, gm, L, partials, nb, j, opt.eps, opt.ittype,
-                         opt.niter - steps);
+                         opt.niter - steps, ctx.host_poll, ++ctx.poll_seq);
       hipLaunchKernelGGL(k_gm_scale, dim3(ge), dim3(256), 0, s, n, ks, gm, L.inv(), w, w);
-      if ((j + 1) % poll == 0 || j + 1 == m) {
-        ctx.pull_state();
-        if (ctx.host_state->st[kStCycleEnd]) break;
+      // one step is queued while the one before it runs; none past the end if polled at every step
+      if (poll == 1 || j + 1 == m) {
+        if (ctx.done_at(ctx.poll_seq)) break;
+      } else if (j > 0 && ctx.done_at(ctx.poll_seq - 1)) {
+        break;
       }
     }
     hipLaunchKernelGGL(k_gm_solve, dim3(1), dim3(1), 0, s, ks, gm, L);

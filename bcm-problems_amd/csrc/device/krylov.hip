@@ -60,20 +60,10 @@ __global__ void k_state_reset(KState* ks, int keep_scalars) {
   if (t < 8) ks->st[t] = 0;
 }
 
-// One-block scalar step. It first adds the pending per-block partials of the
-// preceding reduction (K values, stored from slot0 on), then thread 0 runs
-// the recurrence update `op`.
-__global__ __launch_bounds__(256) void k_scalar(int op, KState* ks, double eps2, int ittype, int niter,
-                                                const double* partials, int nb, int K, int slot0, int stamp) {
+// The recurrence update `op` (one thread).
+__device__ void scalar_update(int op, KState* ks, double eps2, int ittype, int niter, int stamp) {
   double* sc = ks->sc;
   int* st = ks->st;
-  if (st[0]) return;
-  double v[kMaxDots];
-#pragma unroll
-  for (int k = 0; k < kMaxDots; ++k)
-    if (k < K) v[k] = sum_partials(partials, nb, K, k);
-  if (threadIdx.x != 0) return;
-  for (int k = 0; k < K && k < kMaxDots; ++k) sc[slot0 + k] = v[k];
   switch (op) {
     case kOpPcgCheck: {
       const int k = ++st[1];
@@ -147,6 +137,27 @@ __global__ __launch_bounds__(256) void k_scalar(int op, KState* ks, double eps2,
     }
     default: break;
   }
+}
+
+// One-block scalar step. It first adds the pending per-block partials of the
+// preceding reduction (K values, stored from slot0 on), then thread 0 runs
+// the recurrence update `op` and, with a poll word, tells the host whether
+// the solve is done at step `seq`.
+__global__ __launch_bounds__(256) void k_scalar(int op, KState* ks, double eps2, int ittype, int niter,
+                                                const double* partials, int nb, int K, int slot0, int stamp,
+                                                uint64_t* poll, uint64_t seq) {
+  if (ks->st[0]) {
+    if (poll && threadIdx.x == 0) publish_done(poll, seq, 1);
+    return;
+  }
+  double v[kMaxDots];
+#pragma unroll
+  for (int k = 0; k < kMaxDots; ++k)
+    if (k < K) v[k] = sum_partials(partials, nb, K, k);
+  if (threadIdx.x != 0) return;
+  for (int k = 0; k < K && k < kMaxDots; ++k) ks->sc[slot0 + k] = v[k];
+  scalar_update(op, ks, eps2, ittype, niter, stamp);
+  if (poll) publish_done(poll, seq, ks->st[0]);
 }
 
 // ---- PCG vector kernels ----
@@ -309,12 +320,16 @@ int ew_grid(int64_t n) {
 
 // Launches the scalar step `op`, consuming the pending partials of ctx.rw
 // into sc[slot0..].
-void scalar_step(Context& ctx, int op, double eps2, int ittype, int niter, int slot0, int stamp = 0) {
+// With `poll`, publishes the done flag to the host; returns the poll number.
+uint64_t scalar_step(Context& ctx, int op, double eps2, int ittype, int niter, int slot0, int stamp = 0,
+                     bool poll = false) {
   RedWork& rw = ctx.rw;
   const int K = rw.pending_k, nb = rw.pending_blocks;
   rw.pending_k = 0;
   hipLaunchKernelGGL(k_scalar, dim3(1), dim3(256), 0, ctx.stream, op, ctx.dstate(), eps2, ittype, niter,
-                     rw.partials.as<double>(), nb, K, slot0, stamp);
+                     rw.partials.as<double>(), nb, K, slot0, stamp, poll ? ctx.host_poll : nullptr,
+                     poll ? ++ctx.poll_seq : ctx.poll_seq);
+  return ctx.poll_seq;
 }
 
 // Marks the partials a solver vector kernel left in ctx.rw as pending.
@@ -389,6 +404,8 @@ Context::Context() {
   BCM_HIP(hipStreamSynchronize(stream));
   BCM_HIP(hipHostMalloc((void**)&host_state, sizeof(KState), hipHostMallocDefault));
   std::memset(host_state, 0, sizeof(KState));
+  BCM_HIP(hipHostMalloc((void**)&host_poll, sizeof(uint64_t), hipHostMallocDefault));
+  *host_poll = 0;
   rw.ensure();
 }
 
@@ -398,6 +415,7 @@ Context::~Context() {
   for (auto& p : pending) { (void)hipEventDestroy(p.e0); (void)hipEventDestroy(p.e1); }
   for (auto e : ev_pool) (void)hipEventDestroy(e);
   if (host_state) (void)hipHostFree(host_state);
+  if (host_poll) (void)hipHostFree(host_poll);
   if (own_stream && stream) (void)hipStreamDestroy(stream);
 }
 
@@ -415,6 +433,21 @@ void Context::check_sweep_error() {
 void Context::pull_state() {
   BCM_HIP(hipMemcpyAsync(host_state, kstate.p, sizeof(KState), hipMemcpyDeviceToHost, stream));
   BCM_HIP(hipStreamSynchronize(stream));
+}
+
+bool Context::done_at(uint64_t seq) {
+  for (uint32_t spins = 1;; ++spins) {
+    const uint64_t v = __atomic_load_n(host_poll, __ATOMIC_RELAXED);
+    if (v >> 1 >= seq) return v & 1;
+    if (spins % 65536 == 0) {  // an error, or a stream that ended without the step, ends the wait
+      const hipError_t e = hipStreamQuery(stream);
+      if (e == hipErrorNotReady) continue;
+      BCM_HIP(e);
+      if (__atomic_load_n(host_poll, __ATOMIC_RELAXED) >> 1 < seq)
+        throw Error(kErrInternal, "solver poll: the stream ended before the awaited step");
+    }
+    __builtin_ia32_pause();
+  }
 }
 
 hipEvent_t Context::prof_begin() {
@@ -559,7 +592,6 @@ void pcg(Matrix& A, Factor& F, Context& ctx, const SolveOptions& opt, const doub
       const double* ys[2] = {b, r};
       launch_multidot(n, 2, xs, ys, &ks->sc[kBnorm2], ctx.rw, s);  // sc[20] = b.b, sc[21] = r0.r0
     }
-    int it = 0;
     const bool exact = opt.check_every == 1;
     while (true) {
       for (int c = 0; c < opt.check_every; ++c) {
@@ -571,7 +603,8 @@ void pcg(Matrix& A, Factor& F, Context& ctx, const SolveOptions& opt, const doub
           hipLaunchKernelGGL(k_maxabs, dim3(gm), dim3(256), 0, s, (int64_t)n, done, r, mpart);
           hipLaunchKernelGGL(k_maxabs_fold, dim3(1), dim3(256), 0, s, gm, done, mpart, ks, (int)kErrloc);
         }
-        scalar_step(ctx, kOpPcgCheck, eps2, opt.ittype, opt.niter - total, kEnrsq);  // (r,r) -> 8, (r,z) -> 9
+        const uint64_t seq = scalar_step(ctx, kOpPcgCheck, eps2, opt.ittype, opt.niter - total, kEnrsq, 0,
+                                         !exact);  // (r,r) -> 8, (r,z) -> 9
         if (exact) {  // no launch is queued past the convergence test
           ctx.pull_state();
           if (ctx.host_state->st[0]) break;
@@ -583,7 +616,8 @@ void pcg(Matrix& A, Factor& F, Context& ctx, const SolveOptions& opt, const doub
         }
         scalar_step(ctx, kOpPcgAlpha, eps2, opt.ittype, opt.niter - total, kPq);
         hipLaunchKernelGGL(k_pcg_xr, dim3(ew_grid(n)), dim3(256), 0, s, (int64_t)n, ks, p, q, x, r);
-        ++it;
+        // the rest of this step keeps the device busy while the next is queued
+        if (!exact && ctx.done_at(seq)) break;
       }
       ctx.pull_state();
       if (ctx.host_state->st[0]) break;
@@ -649,7 +683,7 @@ void cg_par(Matrix& A, Factor& F, Context& ctx, const SolveOptions& opt, const d
       scalar_step(ctx, kOpCgParAlpha, 0.0, opt.ittype, opt.niter, kCpUau);
       hipLaunchKernelGGL(k_cp_r, dim3(ge), dim3(256), 0, s, n, ks, au, r, ctx.rw.partials.as<double>());
       set_pending(ctx, ge, 1);
-      scalar_step(ctx, kOpCgParCheck, 0.0, opt.ittype, opt.niter, kCpRr);
+      const uint64_t seq = scalar_step(ctx, kOpCgParCheck, 0.0, opt.ittype, opt.niter, kCpRr, 0, !exact);
       precond_apply(F, ctx, r, v, opt.prec, false, 1, done);
       {
         const double* xs[1] = {v};
@@ -661,6 +695,8 @@ void cg_par(Matrix& A, Factor& F, Context& ctx, const SolveOptions& opt, const d
       if (exact) {
         ctx.pull_state();
         if (ctx.host_state->st[0]) break;
+      } else if (ctx.done_at(seq)) {
+        break;
       }
     }
     ctx.pull_state();
@@ -709,8 +745,12 @@ void bicgstab(Matrix& A, Factor& F, Context& ctx, const SolveOptions& opt, const
       scalar_step(ctx, kOpBicgInit, eps2, opt.ittype, opt.niter, kBnorm2);  // 20: b.b 21: r.r 22: rhat.r
     }
     const bool exact = opt.check_every == 1;
+    // A half step is queued while the one before it runs: it needs to know the
+    // outcome of the half before that.
+    uint64_t s_seq = 0, r_seq = 0;
     while (true) {
       for (int c = 0; c < opt.check_every; ++c) {
+        if (s_seq && ctx.done_at(s_seq)) break;
         ++stamp;
         hipLaunchKernelGGL(k_bicg_p, dim3(ge), dim3(256), 0, s, (int64_t)n, ks, r, v, p);
         precond_apply(F, ctx, p, phat, opt.prec, false, 1, done);
@@ -721,11 +761,14 @@ void bicgstab(Matrix& A, Factor& F, Context& ctx, const SolveOptions& opt, const
         scalar_step(ctx, kOpBicgAlpha, eps2, opt.ittype, opt.niter, kRv);
         hipLaunchKernelGGL(k_bicg_s, dim3(ge), dim3(256), 0, s, (int64_t)n, ks, r, v, sv, ctx.rw.partials.as<double>());
         set_pending(ctx, ge, 1);
-        scalar_step(ctx, kOpBicgSCheck, eps2, opt.ittype, opt.niter, kSs, stamp);
+        const uint64_t sq = scalar_step(ctx, kOpBicgSCheck, eps2, opt.ittype, opt.niter, kSs, stamp, !exact);
         hipLaunchKernelGGL(k_bicg_xs, dim3(ge), dim3(256), 0, s, (int64_t)n, ks, stamp, phat, x);
         if (exact) {  // no launch is queued past a convergence test
           ctx.pull_state();
           if (ctx.host_state->st[0]) break;
+        } else {
+          s_seq = sq;
+          if (r_seq && ctx.done_at(r_seq)) break;
         }
         precond_apply(F, ctx, sv, shat, opt.prec, false, 1, done);
         {
@@ -741,7 +784,8 @@ void bicgstab(Matrix& A, Factor& F, Context& ctx, const SolveOptions& opt, const
         hipLaunchKernelGGL(k_bicg_xr, dim3(ge), dim3(256), 0, s, (int64_t)n, ks, phat, shat, sv, t, rhat, x, r,
                            ctx.rw.partials.as<double>());
         set_pending(ctx, ge, 2);
-        scalar_step(ctx, kOpBicgNext, eps2, opt.ittype, opt.niter - total, kRr);
+        const uint64_t rq = scalar_step(ctx, kOpBicgNext, eps2, opt.ittype, opt.niter - total, kRr, 0, !exact);
+        if (!exact) r_seq = rq;
         if (exact) {
           ctx.pull_state();
           if (ctx.host_state->st[0]) break;

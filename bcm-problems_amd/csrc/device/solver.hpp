@@ -70,6 +70,11 @@ struct Context {
   KState* dstate() const { return kstate.as<KState>(); }
   double* vec(int i, size_t nbytes);  // returns work vector i of at least nbytes
   void pull_state();                  // copy state to the pinned mirror and wait
+  // Steps of a running solve publish (number << 1 | done) here, in pinned host
+  // memory: the host follows them without a copy or a wait for the stream.
+  uint64_t* host_poll = nullptr;
+  uint64_t poll_seq = 0;
+  bool done_at(uint64_t seq);  // waits for step seq; whether the solve is done then
   // profiling
   bool prof = false;
   ProfAcc prof_acc[kProfKinds];

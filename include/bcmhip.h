@@ -76,7 +76,8 @@ typedef struct bcm_solve_opts {
   double eps;
   int ittype;        /* 0 ||r|| <= eps ||r0||, 1 ||r|| <= eps, 2 (BCM_PCG only) max_i |r_i| <= |eps|,
                         3 ||b - A x|| <= eps ||b|| */
-  int check_every;   /* device state polled every k iterations */
+  int check_every;   /* 1: no work queued past the end; else a step may be, and the state is
+                        copied back every k iterations */
   int restart;       /* FGMRES cycle length */
   int precision;     /* preconditioner storage/application: BCM_F64, BCM_F32, BCM_BF16 */
   int max_restarts;  /* true-residual restarts */
