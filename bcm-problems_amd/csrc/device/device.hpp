@@ -125,6 +125,9 @@ struct DevTri {
   DevBuf off;         // ndep blocks, row after row
   DevBuf diag;        // nsup inverted diagonal blocks
   DevBuf sp, doff, dgo;  // variable blocks: partition, value offsets of dependency and diagonal blocks
+  // strips (0: none): rows strip by strip, first position of each, dependencies as positions or rows
+  int strips = 0, strip_rows_max = 0;
+  DevBuf strip_rows, strip_ptr, strip_code;
   DevBuf cptr, ccol, roff;  // their columns: first per row, vector element of each, value offset of each row
   int64_t nval = 0;
   int64_t value_bytes() const {

@@ -731,7 +731,8 @@ struct SweepDir {
   const void* off;
   const void* diag;
   int forward;
-  // any block partition (k_sweep_free_var): ia and ja then count vector columns
+  // any block partition (k_sweep_free_var): ia and ja then count vector columns;
+  // strips (k_sweep_strip): sp holds the first position of each
   const int* sp;
   const int64_t* roff;  // first dependency value of each row
   const int64_t* dgo;   // its diagonal block
@@ -1115,6 +1116,233 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free_cx(SweepJob<dou
       st_coherent(&y[(size_t)q * jb.n + (size_t)row * B + lane], sr);
       st_coherent(&y[(size_t)q * jb.n + (size_t)row * B + BC + lane], si);
     }
+  }
+}
+
+// The sync-free sweep in strips. The rows, in a depth-first topological order
+// (the row whose dependency finished last comes next, so that the order runs
+// along a line of the grid), are cut into consecutive strips; a strip depends
+// on itself and on earlier ones only. One workgroup of W waves owns a
+// strip: its waves take the strip's rows by level, and values within the strip
+// pass through LDS, which takes a fraction of the 0.9 us of a hand-over between
+// workgroups; only values from earlier strips (and the first sweep's output)
+// are polled in memory. Workgroups draw strips in order, so that, as with rows,
+// nothing depends on what else is resident. The factor values, the right-hand
+// side and the dependency list of a wave's next row are loaded before it waits
+// for the present one. `ja` holds, per dependency, the row, or for a row of the
+// same strip -1 minus its position there.
+//
+// Waves of a strip, and dependency blocks of a row held in registers (twice,
+// for the next row): 20 x 20 x 20 x block 8 took 136 us with 8 waves, 127 with
+// 16; 20 x 19 x 18 x block 12 (FP64) 166 and 220, block 16 120 and 203.
+constexpr int strip_waves(int b) { return b <= 9 ? 16 : 8; }
+constexpr int strip_held(int b) { return b >= 16 ? 3 : 4; }
+
+template <class T> __device__ __forceinline__ T ld_wg(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+template <class T> __device__ __forceinline__ void st_wg(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+template <int B, int W, class TA, class TX>
+__global__ __launch_bounds__(64 * W) void k_sweep_strip(SweepJob<TX> jb) {
+  if (jb.skip && *jb.skip) return;
+  using Acc = typename AccOf<TX>::type;
+  using Bits = typename Sentinel<TX>::Bits;
+  constexpr int V = sweep_free_width<B>();
+  using VT = typename VecOf<TA, V>::T;
+  constexpr int L = B / V, G = 64 / L, KD = strip_held(B);
+  constexpr int CK = (KD * B + G - 1) / G, PD = (B + G - 1) / G;
+  constexpr int SJ = ((1 + KD) * B + 63) / 64;
+  extern __shared__ __align__(16) char smem[];
+  TX* ly = reinterpret_cast<TX*>(smem);  // the strip's values, position after position
+  __shared__ __align__(16) TX lds[W][(1 + KD) * B];
+  __shared__ int ticket;
+  if (threadIdx.x == 0)
+    ticket = __hip_atomic_fetch_add(&jb.ctl[kSweepTicket], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const int unit = __builtin_amdgcn_readfirstlane(ticket);
+  const bool second = unit >= jb.npos;
+  const int tu = second ? unit - jb.npos : unit, strip = tu / jb.ng;
+  const size_t q0 = (size_t)(tu - strip * jb.ng) * jb.n;
+  const int* __restrict__ ia = second ? jb.d1.ia : jb.d0.ia;
+  const int* __restrict__ ja = second ? jb.d1.ja : jb.d0.ja;
+  const int* __restrict__ ptr = second ? jb.d1.sp : jb.d0.sp;
+  const int p0 = ptr[strip], np = ptr[strip + 1] - p0;
+  const int* __restrict__ order = (second ? jb.d1.order : jb.d0.order) + p0;
+  const TA* off = static_cast<const TA*>(second ? jb.d1.off : jb.d0.off);
+  const TA* diag = static_cast<const TA*>(second ? jb.d1.diag : jb.d0.diag);
+  TX* y = (second ? jb.y1 : jb.y0) + q0;
+  TX* xw = second ? jb.y0 + q0 : nullptr;
+  const char* x = static_cast<const char*>(jb.x) + q0 * (jb.x64 ? sizeof(double) : sizeof(TX));
+  for (int i = threadIdx.x; i < np * B; i += 64 * W) reinterpret_cast<Bits*>(ly)[i] = Sentinel<TX>::bits;
+  __syncthreads();  // the only workgroup-level synchronisation
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  TX* s = lds[wave];
+  const int lr = lane % L, g = lane / L < G ? lane / L : 0;
+  const bool act = lane < G * L;
+  const VT zero = {};
+
+  struct Row {
+    int row, j0, lead, nd;   // lead dependencies first, then nd <= KD held ones
+    VT pd[PD], av[CK];
+    const TX* src[SJ];       // value polled in memory (null: none)
+    int loc[SJ];             // value polled in LDS (-1: none)
+    TX val[SJ];
+  };
+  auto load = [&](int p, Row& R) {
+    if (p >= np) {
+      R.row = -1;
+      return;
+    }
+    R.row = order[p];
+    R.j0 = ia[R.row];
+    const int ndep = ia[R.row + 1] - R.j0;
+    R.nd = ndep < KD ? ndep : KD;
+    R.lead = ndep - R.nd;
+    const TA* d = diag + (size_t)R.row * B * B + lr * V;
+    const TA* blk = off + (size_t)(R.j0 + R.lead) * B * B + lr * V;
+#pragma unroll
+    for (int i = 0; i < CK; ++i) {
+      const int tt = g + i * G;
+      R.av[i] = zero;
+      if (act && tt < R.nd * B) R.av[i] = __builtin_nontemporal_load(reinterpret_cast<const VT*>(blk + (size_t)tt * B));
+    }
+#pragma unroll
+    for (int i = 0; i < PD; ++i) {
+      R.pd[i] = zero;
+      if (act && g + i * G < B)
+        R.pd[i] = __builtin_nontemporal_load(reinterpret_cast<const VT*>(d + (g + i * G) * B));
+    }
+#pragma unroll
+    for (int j = 0; j < SJ; ++j) {
+      const int e = lane + 64 * j, kk = e / B, c = e - kk * B;
+      R.src[j] = nullptr;
+      R.loc[j] = -1;
+      R.val[j] = TX(0);
+      if (kk == 0) {
+        const size_t xo = (size_t)R.row * B + c;
+        if (xw) R.src[j] = xw + xo;
+        else R.val[j] = jb.x64 ? (TX) reinterpret_cast<const double*>(x)[xo] : reinterpret_cast<const TX*>(x)[xo];
+      } else if (kk <= R.nd) {
+        const int code = ja[R.j0 + R.lead + kk - 1];
+        if (code < 0) R.loc[j] = (-1 - code) * B + c;
+        else R.src[j] = y + (size_t)code * B + c;
+      }
+    }
+  };
+  // waits for the values of src / loc and stages them at s[e]
+  auto stage = [&](const TX* const (&src)[SJ], const int (&loc)[SJ], TX(&val)[SJ], int e0) {
+    bool ok = true;
+#pragma unroll
+    for (int j = 0; j < SJ; ++j) {
+      if (src[j]) val[j] = ld_coherent(src[j]);
+      if (loc[j] >= 0) val[j] = ld_wg(ly + loc[j]);
+      ok = ok && !((src[j] || loc[j] >= 0) && is_sentinel(val[j]));
+    }
+    int spins = 0;
+    while (!__all(ok)) {
+      ok = true;
+#pragma unroll
+      for (int j = 0; j < SJ; ++j) {
+        if (src[j] && is_sentinel(val[j])) val[j] = ld_coherent(src[j]);
+        if (loc[j] >= 0 && is_sentinel(val[j])) val[j] = ld_wg(ly + loc[j]);
+        ok = ok && !((src[j] || loc[j] >= 0) && is_sentinel(val[j]));
+      }
+      ++spins;
+      if (__any(spins > kSpinLimit || ((spins & 1023) == 0 && ld_coherent(&jb.ctl[2]) != 0))) {
+        if (lane == 0) st_coherent(&jb.ctl[2], 1);
+        break;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < SJ; ++j) {
+      const int e = lane + 64 * j;
+      if (e >= e0 && e < (1 + KD) * B) s[e] = val[j];
+    }
+    wave_lds_sync();
+  };
+  auto process = [&](int p, Row& R) {
+    Acc acc[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) acc[k] = Acc(0);
+    for (int k0 = 0; k0 < R.lead; k0 += KD) {  // rows of more than KD dependencies
+      const int nb = R.lead - k0 < KD ? R.lead - k0 : KD;
+      const TX* src[SJ];
+      int loc[SJ];
+      TX val[SJ];
+#pragma unroll
+      for (int j = 0; j < SJ; ++j) {
+        const int e = lane + 64 * j, kk = e / B, c = e - kk * B;
+        src[j] = nullptr;
+        loc[j] = -1;
+        val[j] = TX(0);
+        if (kk > 0 && kk <= nb) {
+          const int code = ja[R.j0 + k0 + kk - 1];
+          if (code < 0) loc[j] = (-1 - code) * B + c;
+          else src[j] = y + (size_t)code * B + c;
+        }
+      }
+      stage(src, loc, val, B);
+      const TA* blk = off + (size_t)(R.j0 + k0) * B * B + lr * V;
+      if (act)
+        for (int tt = g; tt < nb * B; tt += G) {
+          const VT a = __builtin_nontemporal_load(reinterpret_cast<const VT*>(blk + (size_t)tt * B));
+#pragma unroll
+          for (int k = 0; k < V; ++k) acc[k] += (Acc)raw_elem<V, TA>(a, k) * (Acc)s[B + tt];
+        }
+      wave_lds_sync();
+    }
+    stage(R.src, R.loc, R.val, 0);
+#pragma unroll
+    for (int i = 0; i < CK; ++i) {
+      const int tt = g + i * G;
+      const Acc yv = (i + 1) * G <= KD * B || tt < KD * B ? (Acc)s[B + (tt < KD * B ? tt : 0)] : Acc(0);
+#pragma unroll
+      for (int k = 0; k < V; ++k) acc[k] += (Acc)raw_elem<V, TA>(R.av[i], k) * yv;
+    }
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      Acc sm = acc[k];
+#pragma unroll
+      for (int h = 1; h < G; ++h) sm += __shfl(acc[k], lane + h * L);
+      if (lane < L) s[lr * V + k] = (TX)((Acc)s[lr * V + k] - sm);
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < V; ++k) acc[k] = Acc(0);
+#pragma unroll
+    for (int i = 0; i < PD; ++i) {
+      const int c = g + i * G;
+      const Acc vc = (i + 1) * G <= B || c < B ? (Acc)s[c < B ? c : 0] : Acc(0);
+#pragma unroll
+      for (int k = 0; k < V; ++k) acc[k] += (Acc)raw_elem<V, TA>(R.pd[i], k) * vc;
+    }
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      Acc sm = acc[k];
+#pragma unroll
+      for (int h = 1; h < G; ++h) sm += __shfl(acc[k], lane + h * L);
+      if (lane < L) {
+        st_wg(ly + p * B + lr * V + k, (TX)sm);
+        const size_t e = (size_t)R.row * B + lr * V + k;
+        st_coherent(&y[e], (TX)sm);
+        if (second && jb.out) jb.out[q0 + e] = (double)(TX)sm;
+      }
+    }
+    wave_lds_sync();
+  };
+  Row a, b;
+  int p = wave;
+  load(p, a);
+  while (a.row >= 0) {
+    load(p + W, b);
+    process(p, a);
+    if (b.row < 0) break;
+    load(p + 2 * W, a);
+    process(p + W, b);
+    p += 2 * W;
   }
 }
 
@@ -2040,8 +2268,75 @@ static bool complex_blocks(const std::vector<double>& src, int b, std::vector<do
   return true;
 }
 
+// Block sizes of k_sweep_strip: up to 16 (at 24 a row's factor values no longer
+// fit the registers twice, and its rows are bound by their loads: 17 x 16 x 15 x
+// block 24 took 186 us by levels, 162 to 218 us in strips, a periodic 16^3 cell
+// 108 against 179).
+constexpr int kStripBlock = 16;
+
 static bool complex_sweep_block(int b) {
   return b == 6 || b == 8 || b == 12 || b == 16 || b == 24 || b == 32;
+}
+
+// Cuts the rows of t (dependency lists ia, ja; levels lev) into strips for
+// k_sweep_strip.
+static void build_strips(const std::vector<int>& ia, const std::vector<int>& ja, const std::vector<int>& lev,
+                         bool forward, DevTri& t) {
+  const int ns = t.nsup;
+  t.strips = 0;
+  // Mostly rows whose dependencies the kernel holds, and levels that stay
+  // narrow (sweep_in_strips); other factors need no strips.
+  int64_t more = 0;
+  for (int r = 0; r < ns; ++r) more += ia[r + 1] - ia[r] > strip_held(t.b) ? 1 : 0;
+  if (ns < 32 || more * 8 > ns || ns > 512LL * t.levels) return;
+  // 16 rows a strip, up to one strip per compute unit; a strip's values within
+  // 48 KB of LDS. (64 x 64 heat, block 9, both sweeps: 448 us by levels; strips
+  // of 16, 32, 64, 256, 512 rows: 264, 274, 274, 402, 587 us.)
+  const int64_t bytes = (int64_t)ns * t.b * 8, lds = 48 << 10;
+  const int P = (int)std::max<int64_t>(std::min(256, ns / 16), (bytes + lds - t.b * 8 - 1) / (lds - t.b * 8));
+  // depth-first topological order
+  std::vector<int> sptr(ns + 1, 0), succ(ja.size()), cnt(ns), seq, stack;
+  for (int r = 0; r < ns; ++r) cnt[r] = ia[r + 1] - ia[r];
+  for (int j = 0; j < ia[ns]; ++j) sptr[ja[j] + 1]++;
+  for (int r = 0; r < ns; ++r) sptr[r + 1] += sptr[r];
+  {
+    std::vector<int> at(sptr.begin(), sptr.end() - 1);
+    for (int q = 0; q < ns; ++q) {
+      const int r = forward ? q : ns - 1 - q;
+      for (int j = ia[r]; j < ia[r + 1]; ++j) succ[at[ja[j]]++] = r;
+    }
+  }
+  for (int q = ns - 1; q >= 0; --q) {
+    const int r = forward ? q : ns - 1 - q;
+    if (cnt[r] == 0) stack.push_back(r);
+  }
+  seq.reserve(ns);
+  while (!stack.empty()) {
+    const int r = stack.back();
+    stack.pop_back();
+    seq.push_back(r);
+    const size_t s0 = stack.size();
+    for (int k = sptr[r]; k < sptr[r + 1]; ++k)
+      if (--cnt[succ[k]] == 0) stack.push_back(succ[k]);
+    std::reverse(stack.begin() + s0, stack.end());
+  }
+  std::vector<int> ptr(P + 1), strip(ns), pos(ns), code(std::max<size_t>(ja.size(), 1));
+  for (int k = 0; k <= P; ++k) ptr[k] = (int)((int64_t)ns * k / P);
+  t.strip_rows_max = 0;
+  for (int k = 0; k < P; ++k) {
+    std::stable_sort(seq.begin() + ptr[k], seq.begin() + ptr[k + 1], [&](int a, int b) { return lev[a] < lev[b]; });
+    for (int i = ptr[k]; i < ptr[k + 1]; ++i) {
+      strip[seq[i]] = k;
+      pos[seq[i]] = i - ptr[k];
+    }
+    t.strip_rows_max = std::max(t.strip_rows_max, ptr[k + 1] - ptr[k]);
+  }
+  for (int r = 0; r < ns; ++r)
+    for (int j = ia[r]; j < ia[r + 1]; ++j) code[j] = strip[ja[j]] == strip[r] ? -1 - pos[ja[j]] : ja[j];
+  t.strips = P;
+  t.strip_rows.upload(seq.data(), std::max<size_t>(seq.size(), 1) * 4);
+  t.strip_ptr.upload(ptr.data(), ptr.size() * 4);
+  t.strip_code.upload(code.data(), code.size() * 4);
 }
 
 // cplx: the parts are real equivalents of complex factors; their blocks are
@@ -2167,6 +2462,7 @@ static void build_tri_parts(const std::vector<const BlockCsr*>& parts, bool forw
   t.level_rows.upload(rows.data(), std::max<size_t>(rows.size(), 1) * 4);
   t.ia.upload(ia_all.data(), ia_all.size() * 4);
   t.ja.upload(ja_all.data(), ja_all.size() * 4);
+  if (np == 1 && !cplx && b <= kStripBlock) build_strips(ia_all, ja_all, lev_all, forward, t);
 }
 
 void dev_tri_forward(const BlockCsr& f, int prec, DevTri& t, bool cplx) {
@@ -2377,6 +2673,14 @@ static bool sweep_split_columns(const DevTri& T, int nrhs) {
   return level_rows * nrhs <= 4LL * device_cu_count();
 }
 
+// Whether nrhs columns of a sweep run in strips. A compute unit does a strip's
+// rows at 0.3 - 0.6 us each, so 256 of them do some 2 ns a row, where the rows
+// of a level on all waves do 0.7 ns (block 9); a level costs 0.65 us in strips
+// and 1.2 us else. Strips therefore win up to some 600 rows a level.
+static bool sweep_in_strips(const DevTri& T, int nrhs) {
+  return T.strips > 0 && (int64_t)T.nsup * nrhs <= 512LL * T.levels && (int64_t)T.strips * nrhs <= INT32_MAX / 2;
+}
+
 // Whether a factor of any block partition takes the sync-free sweep: where its
 // column list and the positions of nrhs columns fit 32-bit indices.
 static bool sweep_var_listed(const DevTri& T, int nrhs) {
@@ -2417,10 +2721,11 @@ static SweepDir sweep_dir(const DevTri& T, const SweepSync& sync) {
   return d;
 }
 
-// Fills the outputs and launches `kern` (8 block rows per workgroup) over
-// columns c0 .. c0 + nr * ng - 1.
+// Fills the outputs and launches `kern` (8 block rows per workgroup, or a
+// strip per workgroup of strip_waves) over columns c0 .. c0 + nr * ng - 1.
 template <class TX>
-static void sweep_launch(void (*kern)(SweepJob<TX>), const SweepLaunch& l, int c0, int nr, int ng) {
+static void sweep_launch(void (*kern)(SweepJob<TX>), const SweepLaunch& l, int c0, int nr, int ng,
+                         int strip_waves = 0) {
   const DevTri& T = *l.T1;
   const size_t o = (size_t)c0 * T.n;
   SweepJob<TX> jb{};
@@ -2442,6 +2747,21 @@ static void sweep_launch(void (*kern)(SweepJob<TX>), const SweepLaunch& l, int c
   const int64_t ny = (int64_t)T.n * nr * ng;
   hipLaunchKernelGGL((k_sweep_fill<TX>), dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((ny + 255) / 256, 2048))),
                      dim3(256), 0, l.s, ny, jb.y0, jb.y1, jb.ctl, l.skip);
+  if (strip_waves) {
+    jb.npos = T.strips * ng;
+    auto dir = [](const DevTri& t, SweepDir& d) {
+      d.order = t.strip_rows.as<int>();
+      d.ja = t.strip_code.as<int>();
+      d.sp = t.strip_ptr.as<int>();
+    };
+    dir(T, jb.d0);
+    if (l.T2) dir(*l.T2, jb.d1);
+    const int units = (T.strips + (l.T2 ? l.T2->strips : 0)) * ng;
+    const int rows = std::max(T.strip_rows_max, l.T2 ? l.T2->strip_rows_max : 0);
+    hipLaunchKernelGGL(kern, dim3(units), dim3(64 * strip_waves), (size_t)rows * T.b * sizeof(TX), l.s, jb);
+    BCM_HIP(hipGetLastError());
+    return;
+  }
   const int grid = (jb.npos * jb.phases + kSweepWaves - 1) / kSweepWaves;
   hipLaunchKernelGGL(kern, dim3(std::max(1, grid)), dim3(64 * kSweepWaves), 0, l.s, jb);
   BCM_HIP(hipGetLastError());
@@ -2449,6 +2769,12 @@ static void sweep_launch(void (*kern)(SweepJob<TX>), const SweepLaunch& l, int c
 
 template <int B, class TA, class TX>
 static void sweep_free(const SweepLaunch& l, int nrhs) {
+  if constexpr (B <= kStripBlock) {
+    if (l.sync->level_order && sweep_in_strips(*l.T1, nrhs) && (!l.T2 || sweep_in_strips(*l.T2, nrhs))) {
+      sweep_launch<TX>(k_sweep_strip<B, strip_waves(B), TA, TX>, l, 0, 1, nrhs, strip_waves(B));
+      return;
+    }
+  }
   if (sweep_split_columns(*l.T1, nrhs)) {
     sweep_launch<TX>(k_sweep_free<B, 1, TA, TX>, l, 0, 1, nrhs);
     return;

@@ -175,3 +175,38 @@ def test_syncfree_any_partition_matches_level_schedule(B, fctx, blocks, size, ng
                 fctx.sync()
                 lctx.sync()
                 assert rel(dy.host(), dm.host()) < 1e-13
+
+
+# Strips (narrow levels): every block size they are built for, rows with more
+# dependencies than are held, a strip count that does not divide the rows, and
+# the smallest system that has strips (32 rows).
+@pytest.mark.parametrize("b,size,ngroup,nrhs", [
+    (3, 4, 8, 1), (6, 4, 60, 2), (8, 5, 83, 1), (9, 4, 90, 6), (12, 4, 70, 1), (16, 3, 50, 3), (16, 4, 12, 1)])
+def test_syncfree_strips_match_level_schedule(B, fctx, b, size, ngroup, nrhs):
+    rng = np.random.default_rng(b)
+    ns = size * ngroup  # a chain of coupled groups: row r depends on the rest of its group and the group before
+    ia, ja, vals = [0], [], []
+    for r in range(ns):
+        k = r // size * size
+        cols = list(range(max(0, k - (size if r == k else 0)), k + size))
+        if r == k + size - 1 and k + size < ns:
+            cols.append(k + size)
+        for c in cols:
+            blk = 0.1 * rng.standard_normal((b, b))
+            ja.append(c)
+            vals.append((blk + 8.0 * np.eye(b) if c == r else blk).ravel())
+        ia.append(len(ja))
+    m = B.Matrix.from_arrays(np.arange(ns + 1) * b, ia, ja, np.concatenate(vals), False)
+    f = B.Factor.ilu2(m, B.default_params(tau1=1e-6, tau2=1e-8))
+    print(f"strips b={b} ns={ns} nrhs={nrhs}", flush=True)
+    r = rng.standard_normal((m.n, nrhs))
+    lctx = B.Context()
+    lctx.set_sweep_mode(0)
+    for precision, tol in ((0, 1e-13), (1, 2e-5), (2, 2e-5)):
+        for transpose in (False, True):
+            dr, dz, dl = dev(B, r), B.DeviceArray((m.n, nrhs)), B.DeviceArray((m.n, nrhs))
+            fctx.precond(f, dr, dz, nrhs, precision=precision, transpose=transpose)
+            lctx.precond(f, dr, dl, nrhs, precision=precision, transpose=transpose)
+            fctx.sync()
+            lctx.sync()
+            assert rel(dz.host(), dl.host()) < tol
