@@ -1132,9 +1132,16 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free_cx(SweepJob<dou
 // for the present one. `ja` holds, per dependency, the row, or for a row of the
 // same strip -1 minus its position there.
 //
+// Four lanes share a row of the block (lane = 4 r + g, g taking the columns g, g
+// + 4, ...), so that a row's sum is two swaps within registers. With the layout
+// of k_sweep_free, whose sums cross the wave through LDS, both sweeps of 64 x 64
+// heat, block 9, took 264 us (now 244), of 20 x 19 x 18 x block 12 167 (120), of
+// 16^3 x block 16 120 (105).
+//
 // Waves of a strip, and dependency blocks of a row held in registers (twice,
-// for the next row): 20 x 20 x 20 x block 8 took 136 us with 8 waves, 127 with
-// 16; 20 x 19 x 18 x block 12 (FP64) 166 and 220, block 16 120 and 203.
+// for the next row): in that layout 20 x 20 x 20 x block 8 took 136 us with 8
+// waves, 127 with 16; 20 x 19 x 18 x block 12 (FP64) 166 and 220, block 16 120
+// and 203.
 constexpr int strip_waves(int b) { return b <= 9 ? 16 : 8; }
 constexpr int strip_held(int b) { return b >= 16 ? 3 : 4; }
 
@@ -1145,14 +1152,33 @@ template <class T> __device__ __forceinline__ void st_wg(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// Sum over the four lanes of a quad, to each of them (two register-lane swaps).
+template <int CTRL>
+__device__ __forceinline__ unsigned quad_swap(unsigned v) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, false);
+}
+template <int CTRL>
+__device__ __forceinline__ float quad_swap(float v) {
+  return __uint_as_float(quad_swap<CTRL>(__float_as_uint(v)));
+}
+template <int CTRL>
+__device__ __forceinline__ double quad_swap(double v) {
+  const unsigned lo = quad_swap<CTRL>((unsigned)__double2loint(v)), hi = quad_swap<CTRL>((unsigned)__double2hiint(v));
+  return __hiloint2double((int)hi, (int)lo);
+}
+template <class T>
+__device__ __forceinline__ T quad_sum(T v) {
+  v += quad_swap<0xB1>(v);  // lanes 1, 0, 3, 2
+  v += quad_swap<0x4E>(v);  // lanes 2, 3, 0, 1
+  return v;
+}
+
 template <int B, int W, class TA, class TX>
 __global__ __launch_bounds__(64 * W) void k_sweep_strip(SweepJob<TX> jb) {
   if (jb.skip && *jb.skip) return;
   using Acc = typename AccOf<TX>::type;
   using Bits = typename Sentinel<TX>::Bits;
-  constexpr int V = sweep_free_width<B>();
-  using VT = typename VecOf<TA, V>::T;
-  constexpr int L = B / V, G = 64 / L, KD = strip_held(B);
+  constexpr int G = 4, KD = strip_held(B);
   constexpr int CK = (KD * B + G - 1) / G, PD = (B + G - 1) / G;
   constexpr int SJ = ((1 + KD) * B + 63) / 64;
   extern __shared__ __align__(16) char smem[];
@@ -1180,13 +1206,12 @@ __global__ __launch_bounds__(64 * W) void k_sweep_strip(SweepJob<TX> jb) {
   __syncthreads();  // the only workgroup-level synchronisation
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   TX* s = lds[wave];
-  const int lr = lane % L, g = lane / L < G ? lane / L : 0;
-  const bool act = lane < G * L;
-  const VT zero = {};
+  const int r = lane >> 2 < B ? lane >> 2 : 0, g = lane & 3;
+  const bool act = lane >> 2 < B;
 
   struct Row {
     int row, j0, lead, nd;   // lead dependencies first, then nd <= KD held ones
-    VT pd[PD], av[CK];
+    TA pd[PD], av[CK];
     const TX* src[SJ];       // value polled in memory (null: none)
     int loc[SJ];             // value polled in LDS (-1: none)
     TX val[SJ];
@@ -1201,19 +1226,19 @@ __global__ __launch_bounds__(64 * W) void k_sweep_strip(SweepJob<TX> jb) {
     const int ndep = ia[R.row + 1] - R.j0;
     R.nd = ndep < KD ? ndep : KD;
     R.lead = ndep - R.nd;
-    const TA* d = diag + (size_t)R.row * B * B + lr * V;
-    const TA* blk = off + (size_t)(R.j0 + R.lead) * B * B + lr * V;
+    const TA* d = diag + (size_t)R.row * B * B + r;
+    const TA* blk = off + (size_t)(R.j0 + R.lead) * B * B + r;
 #pragma unroll
     for (int i = 0; i < CK; ++i) {
       const int tt = g + i * G;
-      R.av[i] = zero;
-      if (act && tt < R.nd * B) R.av[i] = __builtin_nontemporal_load(reinterpret_cast<const VT*>(blk + (size_t)tt * B));
+      R.av[i] = TA(0);
+      if (act && tt < R.nd * B) R.av[i] = __builtin_nontemporal_load(blk + (size_t)tt * B);
     }
 #pragma unroll
     for (int i = 0; i < PD; ++i) {
-      R.pd[i] = zero;
+      R.pd[i] = TA(0);
       if (act && g + i * G < B)
-        R.pd[i] = __builtin_nontemporal_load(reinterpret_cast<const VT*>(d + (g + i * G) * B));
+        R.pd[i] = __builtin_nontemporal_load(d + (g + i * G) * B);
     }
 #pragma unroll
     for (int j = 0; j < SJ; ++j) {
@@ -1264,9 +1289,7 @@ __global__ __launch_bounds__(64 * W) void k_sweep_strip(SweepJob<TX> jb) {
     wave_lds_sync();
   };
   auto process = [&](int p, Row& R) {
-    Acc acc[V];
-#pragma unroll
-    for (int k = 0; k < V; ++k) acc[k] = Acc(0);
+    Acc acc = Acc(0);
     for (int k0 = 0; k0 < R.lead; k0 += KD) {  // rows of more than KD dependencies
       const int nb = R.lead - k0 < KD ? R.lead - k0 : KD;
       const TX* src[SJ];
@@ -1285,51 +1308,35 @@ __global__ __launch_bounds__(64 * W) void k_sweep_strip(SweepJob<TX> jb) {
         }
       }
       stage(src, loc, val, B);
-      const TA* blk = off + (size_t)(R.j0 + k0) * B * B + lr * V;
+      const TA* blk = off + (size_t)(R.j0 + k0) * B * B + r;
       if (act)
-        for (int tt = g; tt < nb * B; tt += G) {
-          const VT a = __builtin_nontemporal_load(reinterpret_cast<const VT*>(blk + (size_t)tt * B));
-#pragma unroll
-          for (int k = 0; k < V; ++k) acc[k] += (Acc)raw_elem<V, TA>(a, k) * (Acc)s[B + tt];
-        }
+        for (int tt = g; tt < nb * B; tt += G) acc += (Acc)ldnt(blk + (size_t)tt * B) * (Acc)s[B + tt];
       wave_lds_sync();
     }
     stage(R.src, R.loc, R.val, 0);
+    Acc acc1 = Acc(0);  // two chains of dependent additions
 #pragma unroll
     for (int i = 0; i < CK; ++i) {
       const int tt = g + i * G;
       const Acc yv = (i + 1) * G <= KD * B || tt < KD * B ? (Acc)s[B + (tt < KD * B ? tt : 0)] : Acc(0);
-#pragma unroll
-      for (int k = 0; k < V; ++k) acc[k] += (Acc)raw_elem<V, TA>(R.av[i], k) * yv;
+      (i & 1 ? acc1 : acc) += (Acc)ldv(&R.av[i]) * yv;
     }
-#pragma unroll
-    for (int k = 0; k < V; ++k) {
-      Acc sm = acc[k];
-#pragma unroll
-      for (int h = 1; h < G; ++h) sm += __shfl(acc[k], lane + h * L);
-      if (lane < L) s[lr * V + k] = (TX)((Acc)s[lr * V + k] - sm);
-    }
+    acc = quad_sum(acc + acc1);
+    if (act && g == 0) s[r] = (TX)((Acc)s[r] - acc);
     wave_lds_sync();
-#pragma unroll
-    for (int k = 0; k < V; ++k) acc[k] = Acc(0);
+    acc = Acc(0);
 #pragma unroll
     for (int i = 0; i < PD; ++i) {
       const int c = g + i * G;
       const Acc vc = (i + 1) * G <= B || c < B ? (Acc)s[c < B ? c : 0] : Acc(0);
-#pragma unroll
-      for (int k = 0; k < V; ++k) acc[k] += (Acc)raw_elem<V, TA>(R.pd[i], k) * vc;
+      acc += (Acc)ldv(&R.pd[i]) * vc;
     }
-#pragma unroll
-    for (int k = 0; k < V; ++k) {
-      Acc sm = acc[k];
-#pragma unroll
-      for (int h = 1; h < G; ++h) sm += __shfl(acc[k], lane + h * L);
-      if (lane < L) {
-        st_wg(ly + p * B + lr * V + k, (TX)sm);
-        const size_t e = (size_t)R.row * B + lr * V + k;
-        st_coherent(&y[e], (TX)sm);
-        if (second && jb.out) jb.out[q0 + e] = (double)(TX)sm;
-      }
+    acc = quad_sum(acc);
+    if (act && g == 0) {
+      st_wg(ly + p * B + r, (TX)acc);
+      const size_t e = (size_t)R.row * B + r;
+      st_coherent(&y[e], (TX)acc);
+      if (second && jb.out) jb.out[q0 + e] = (double)(TX)acc;
     }
     wave_lds_sync();
   };
@@ -2268,10 +2275,10 @@ static bool complex_blocks(const std::vector<double>& src, int b, std::vector<do
   return true;
 }
 
-// Block sizes of k_sweep_strip: up to 16 (at 24 a row's factor values no longer
-// fit the registers twice, and its rows are bound by their loads: 17 x 16 x 15 x
-// block 24 took 186 us by levels, 162 to 218 us in strips, a periodic 16^3 cell
-// 108 against 179).
+// Block sizes of k_sweep_strip: up to 16 rows, four lanes each. (At 24, with the
+// layout of k_sweep_free, a row's factor values did not fit the registers twice:
+// 17 x 16 x 15 took 186 us by levels, 162 to 218 us in strips, a periodic 16^3
+// cell 108 against 179.)
 constexpr int kStripBlock = 16;
 
 static bool complex_sweep_block(int b) {
@@ -2291,7 +2298,7 @@ static void build_strips(const std::vector<int>& ia, const std::vector<int>& ja,
   if (ns < 32 || more * 8 > ns || ns > 512LL * t.levels) return;
   // 16 rows a strip, up to one strip per compute unit; a strip's values within
   // 48 KB of LDS. (64 x 64 heat, block 9, both sweeps: 448 us by levels; strips
-  // of 16, 32, 64, 256, 512 rows: 264, 274, 274, 402, 587 us.)
+  // of 16, 32, 64 rows: 244, 249, 254 us.)
   const int64_t bytes = (int64_t)ns * t.b * 8, lds = 48 << 10;
   const int P = (int)std::max<int64_t>(std::min(256, ns / 16), (bytes + lds - t.b * 8 - 1) / (lds - t.b * 8));
   // depth-first topological order
