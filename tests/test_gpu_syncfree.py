@@ -1,6 +1,7 @@
-"""Sync-free triangular sweeps (one launch per sweep; static row ownership;
-the output pre-filled with a sentinel that marks unfinished rows; each row's
-dependency values staged through LDS behind a bounded, wave-voted wait)
+"""Sync-free triangular sweeps (one launch per sweep or
+pair of sweeps; rows drawn in topological order; the output pre-filled with a
+sentinel that marks unfinished rows; each row's dependency values staged
+through LDS behind a bounded, wave-voted wait; strips of rows for narrow levels)
 against the CPU oracle, and against the level-scheduled sweeps."""
 
 import numpy as np
