@@ -759,6 +759,14 @@ void Mlp::chain(hipStream_t s, int M, const float* x, const float* t, float* out
 
 void Mlp::forward(hipStream_t s, int M, const float* x, float* out) {
   if (fused && out) {
+    // A workgroup writes its rows of out while others still read x: where the
+    // two share memory, x is read from a copy.
+    const size_t nx = (size_t)M * nin, ny = (size_t)M * nout;
+    if (out < x + nx && x < out + ny) {
+      if (xcopy.bytes < nx * 4) xcopy.alloc(nx * 4);
+      BCM_HIP(hipMemcpyAsync(xcopy.p, x, nx * 4, hipMemcpyDeviceToDevice, s));
+      x = xcopy.as<const float>();
+    }
     chain(s, M, x, nullptr, out, nullptr);
     return;
   }

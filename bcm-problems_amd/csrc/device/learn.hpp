@@ -23,6 +23,7 @@ struct Mlp {
   int step = 0;  // Adam steps taken
   bool fused = false;  // a workgroup's rows fit its LDS: packed weights and the fused kernels
   DevBuf wpk, tape;    // fused: weights and the last pass as MFMA fragments
+  DevBuf xcopy;        // fused: the input of a forward pass whose output overlaps it
   Mlp(int nin, int nh, int nout, uint64_t seed);
   void set_params(const float* host);  // also resets the Adam moments
   void ensure_batch(int M);

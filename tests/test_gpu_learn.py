@@ -164,3 +164,22 @@ def test_mlp_sizes_match_oracle(B, ctx, dims, batch):
     assert relerr(m.params(), pn) < 1e-6
     y1, _ = M.forward(m.params().astype(np.float64), x.astype(np.float64), *dims, bf16=True)
     assert relerr(m.forward(ctx, x), y1) < 1e-3  # the packed weights follow the update
+
+
+# One buffer for input and output: the output starts where the input does, or
+# inside it; rows of the output wider, narrower and as wide as the input's.
+@pytest.mark.parametrize("dims,shift", [((4, 16, 8), 0), ((8, 16, 4), 0), ((6, 16, 6), 0), ((6, 16, 6), 3),
+                                        ((4, 16, 8), 1000), ((200, 64, 700), 0)])
+def test_mlp_forward_overlapping_buffers(B, ctx, dims, shift):
+    nin, _, nout = dims
+    batch = 20000 if nin < 10 else 500
+    print(f"mlp {dims} one buffer, output {shift} floats behind the input", flush=True)
+    m = B.Mlp(*dims, seed=4)
+    x = np.random.default_rng(3).normal(size=(batch, nin)).astype(np.float32)
+    want = m.forward(ctx, x)
+    buf = np.zeros(shift + batch * max(nin, nout), np.float32)
+    buf[:x.size] = x.ravel()
+    d = B.DeviceArray.from_host(buf)
+    B._check(B.lib().bcm_mlp_forward(ctx.h, m.h, batch, B.ptr(d), B.ptr(d) + 4 * shift))
+    ctx.sync()
+    assert np.array_equal(d.host()[shift:shift + batch * nout].reshape(batch, nout), want)
