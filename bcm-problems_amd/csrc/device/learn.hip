@@ -343,7 +343,7 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int M, int ms, MlpD
       float v[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        v[q] = j < d.nh ? tanhf(acc[q] + bj) : 0.f;
+        v[q] = j < d.nh && m0 + 4 * g + q < M ? tanhf(acc[q] + bj) : 0.f;
         hf[(4 * g + q) * hc + j] = v[q];
         hb[(4 * g + q) * lh + j] = f2bf(v[q]);
       }
@@ -403,7 +403,7 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int M, int ms, MlpD
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const float h = h2f[(4 * g + q) * hc + j];
-      v[q] = j < d.nh ? acc[q] * (1.0f - h * h) : 0.f;
+      v[q] = j < d.nh && m0 + 4 * g + q < M ? acc[q] * (1.0f - h * h) : 0.f;
       h1b[(4 * g + q) * lh + j] = f2bf(v[q]);
     }
     store_frag(tape.dz2, tn, ms, m0, v);
@@ -417,7 +417,7 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int M, int ms, MlpD
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const float h = h1f[(4 * g + q) * hc + j];
-      v[q] = j < d.nh ? acc[q] * (1.0f - h * h) : 0.f;
+      v[q] = j < d.nh && m0 + 4 * g + q < M ? acc[q] * (1.0f - h * h) : 0.f;
     }
     store_frag(tape.dz1, tn, ms, m0, v);
     const float s = tile_colsum(v);

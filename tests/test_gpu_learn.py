@@ -183,3 +183,27 @@ def test_mlp_forward_overlapping_buffers(B, ctx, dims, shift):
     B._check(B.lib().bcm_mlp_forward(ctx.h, m.h, batch, B.ptr(d), B.ptr(d) + 4 * shift))
     ctx.sync()
     assert np.array_equal(d.host()[shift:shift + batch * nout].reshape(batch, nout), want)
+
+
+# An infinite weight saturates one unit. Rows past the batch, which fill up the
+# last tile of rows, add nothing to any gradient then either.
+@pytest.mark.parametrize("layer", [0, 2])
+@pytest.mark.parametrize("batch", [17, 33, 64])
+def test_mlp_infinite_weight(B, ctx, layer, batch):
+    dims = (5, 20, 33)
+    rng = np.random.default_rng(layer + batch)
+    offs, npar = M.layout(*dims)
+    p = rng.normal(0, 0.3, npar).astype(np.float32)
+    p[offs[layer][0]] = np.inf
+    x = rng.normal(size=(batch, dims[0])).astype(np.float32)
+    t = rng.normal(size=(batch, dims[2])).astype(np.float32)
+    print(f"mlp infinite weight layer {layer // 2 + 1} batch {batch}", flush=True)
+    m = B.Mlp(*dims, seed=2)
+    m.set_params(p)
+    loss = m.backward(ctx, x, t)
+    with np.errstate(invalid="ignore"):
+        lo, go = M.loss_grad(p.astype(np.float64), x.astype(np.float64), t.astype(np.float64), *dims, bf16=True)
+    g = m.grads().astype(np.float64)
+    assert abs(loss - lo) <= 1e-4 * lo
+    assert np.array_equal(np.isfinite(g), np.isfinite(go))
+    assert relerr(g[np.isfinite(go)], go[np.isfinite(go)]) < 2e-3  # as the gradients of finite weights
