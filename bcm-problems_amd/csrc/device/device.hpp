@@ -117,6 +117,7 @@ struct DevTri {
   bool forward = true;
   int prec = kF64;
   int levels = 0;
+  int deps_max = 0;  // most dependencies of a row
   int cplx = 0;  // 1: real equivalent of a complex factor, off/diag holding its complex (b/2)^2 blocks
   DevBuf lctl;   // complex factors: control words of the per-level launches of the complex sweep kernel
   std::vector<int> level_ptr;  // host: rows of level l are level_rows[level_ptr[l] .. level_ptr[l+1])

@@ -19,6 +19,7 @@
 // on another wave.
 #include "device.hpp"
 #include "dev_common.hpp"
+#include "sweep_plan.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -681,7 +682,8 @@ __global__ __launch_bounds__(256) void k_sweep_level(int nrows, const int* __res
 // device-scope relaxed atomic loads/stores (coherent across the 8 L2s, the
 // protocol rocPRIM's look-back scan uses on gfx942/gfx950); there is no
 // separate flag and no fence on the critical path. A wait that exceeds its
-// bound raises ctl[2], which stops every other wait; the host reports it.
+// bound (a time, sweep_wait_seconds) raises ctl[2], which stops every other
+// wait; the host reports it.
 //
 // What bounds it: a single system's sweep is a chain of dependency levels,
 // each one hand-over (0.4-0.6 us between two waves through the coherent
@@ -754,6 +756,7 @@ struct SweepJob {
   double* out;
   int* ctl;
   const int* skip;
+  uint64_t wait;  // bound of a dependency wait, in ticks of the wall clock
 };
 
 // Draws the workgroup's ticket; returns this wave's position (-1: past the end).
@@ -768,6 +771,21 @@ __device__ __forceinline__ int sweep_position(const SweepJob<TX>& jb) {
   return pos < jb.npos * jb.phases ? pos : -1;
 }
 
+// Whether a wave's dependency wait gives up after `polls` rounds: every 1024
+// of them it looks at the error flag, which ends every wait of the launch, and
+// at the time since `since` (0: not yet taken), which raises the flag. The
+// bound is a time because a round may take 0.05 us (a value of the wave's own
+// workgroup) or 1 us (memory), while a wait is as long as the part of the
+// sweep that it waits for. Uniform over the wave.
+__device__ __forceinline__ bool wait_over(int polls, uint64_t& since, uint64_t bound, int* ctl) {
+  if ((polls & 1023) != 0) return false;
+  const uint64_t now = wall_clock64();
+  if (since == 0) since = now;
+  if (!__any(now - since > bound || ld_coherent(&ctl[2]) != 0)) return false;
+  if ((threadIdx.x & 63) == 0) st_coherent(&ctl[2], 1);
+  return true;
+}
+
 // Stages nd (<= KM) dependency blocks of a row (block rows cols[0..nd) of y,
 // NR columns of leading dimension n) into s[((1 + k) * B + c) * NR + q], and
 // with row >= 0 the row's right-hand side into block 0 of s: x (already a
@@ -779,7 +797,7 @@ __device__ __forceinline__ int sweep_position(const SweepJob<TX>& jb) {
 // wait.
 template <int B, int NR, int KM, class TX>
 __device__ __forceinline__ void stage_deps(int nd, int npad, const int* __restrict__ cols, TX* y, int n, int row,
-                                           const void* x, int x64, TX* xw, TX* s, int* ctl) {
+                                           const void* x, int x64, TX* xw, TX* s, int* ctl, uint64_t bound) {
   constexpr int M = B * NR, SJ = ((1 + KM) * M + 63) / 64;
   const int lane = threadIdx.x & 63;
   const TX* src[SJ];  // polled values (null: not polled)
@@ -804,7 +822,8 @@ __device__ __forceinline__ void stage_deps(int nd, int npad, const int* __restri
       val[j] = ld_coherent(src[j]);
       ok = ok && !is_sentinel(val[j]);
     }
-  int spins = 0;
+  int polls = 0;
+  uint64_t since = 0;
   while (!__all(ok)) {
     ok = true;
 #pragma unroll
@@ -813,11 +832,7 @@ __device__ __forceinline__ void stage_deps(int nd, int npad, const int* __restri
         val[j] = ld_coherent(src[j]);
         ok = ok && !is_sentinel(val[j]);
       }
-    ++spins;
-    if (__any(spins > kSpinLimit || ((spins & 1023) == 0 && ld_coherent(&ctl[2]) != 0))) {
-      if (lane == 0) st_coherent(&ctl[2], 1);
-      break;
-    }
+    if (wait_over(++polls, since, bound, ctl)) break;
   }
   const int e1 = (1 + npad) * M;
 #pragma unroll
@@ -928,7 +943,7 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free(SweepJob<TX> jb
   int k0 = 0;
   for (; ndep - k0 > NC * KD; k0 += KD) {
     load_chunk(k0, KD, av[0]);
-    stage_deps<B, NR, KD>(KD, KD, ja + j0 + k0, y, jb.n, -1, x, jb.x64, xw, s, jb.ctl);
+    stage_deps<B, NR, KD>(KD, KD, ja + j0 + k0, y, jb.n, -1, x, jb.x64, xw, s, jb.ctl, jb.wait);
     multiply(0, av[0]);
     wave_lds_sync();
   }
@@ -937,7 +952,7 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free(SweepJob<TX> jb
   if constexpr (NC == 2)
     if (nd > KD) load_chunk(k0 + KD, nd - KD, av[1]);
   stage_deps<B, NR, NC * KD>(nd, nd > KD ? NC * KD : (nd > 0 ? KD : 0), ja + j0 + k0, y, jb.n, row, x, jb.x64, xw, s,
-                             jb.ctl);
+                             jb.ctl, jb.wait);
   if (nd > 0) multiply(0, av[0]);
   if constexpr (NC == 2)
     if (nd > KD) multiply(1, av[1]);
@@ -1064,7 +1079,7 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free_cx(SweepJob<dou
   int k0 = 0;
   for (; ndep - k0 > NC * KD; k0 += KD) {
     load_chunk(k0, KD, av[0]);
-    stage_deps<B, NR, KD>(KD, KD, ja + j0 + k0, y, jb.n, -1, x, 0, xw, s, jb.ctl);
+    stage_deps<B, NR, KD>(KD, KD, ja + j0 + k0, y, jb.n, -1, x, 0, xw, s, jb.ctl, jb.wait);
     multiply(0, av[0]);
     wave_lds_sync();
   }
@@ -1073,7 +1088,7 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free_cx(SweepJob<dou
   if constexpr (NC == 2)
     if (nd > KD) load_chunk(k0 + KD, nd - KD, av[1]);
   stage_deps<B, NR, NC * KD>(nd, nd > KD ? NC * KD : (nd > 0 ? KD : 0), ja + j0 + k0, y, jb.n, row, x, 0, xw, s,
-                             jb.ctl);
+                             jb.ctl, jb.wait);
   if (nd > 0) multiply(0, av[0]);
   if constexpr (NC == 2)
     if (nd > KD) multiply(1, av[1]);
@@ -1266,7 +1281,8 @@ __global__ __launch_bounds__(64 * W) void k_sweep_strip(SweepJob<TX> jb) {
       if (loc[j] >= 0) val[j] = ld_wg(ly + loc[j]);
       ok = ok && !((src[j] || loc[j] >= 0) && is_sentinel(val[j]));
     }
-    int spins = 0;
+    int polls = 0;
+  uint64_t since = 0;
     while (!__all(ok)) {
       ok = true;
 #pragma unroll
@@ -1275,11 +1291,7 @@ __global__ __launch_bounds__(64 * W) void k_sweep_strip(SweepJob<TX> jb) {
         if (loc[j] >= 0 && is_sentinel(val[j])) val[j] = ld_wg(ly + loc[j]);
         ok = ok && !((src[j] || loc[j] >= 0) && is_sentinel(val[j]));
       }
-      ++spins;
-      if (__any(spins > kSpinLimit || ((spins & 1023) == 0 && ld_coherent(&jb.ctl[2]) != 0))) {
-        if (lane == 0) st_coherent(&jb.ctl[2], 1);
-        break;
-      }
+      if (wait_over(++polls, since, jb.wait, jb.ctl)) break;
     }
 #pragma unroll
     for (int j = 0; j < SJ; ++j) {
@@ -1371,7 +1383,8 @@ constexpr int kVarChunk = 192;  // columns staged at a time
 // and s[r].
 template <class TX>
 __device__ __forceinline__ void stage_var(int nw, const int* __restrict__ cols, const TX* y, int r0, int bk,
-                                          const void* x, int x64, const TX* xw, TX* s, int* ctl) {
+                                          const void* x, int x64, const TX* xw, TX* s, int* ctl,
+                                          uint64_t bound) {
   constexpr int SJ = 1 + kVarChunk / 64;
   const int lane = threadIdx.x & 63;
   const TX* src[SJ];
@@ -1396,7 +1409,8 @@ __device__ __forceinline__ void stage_var(int nw, const int* __restrict__ cols, 
       val[j] = ld_coherent(src[j]);
       ok = ok && !is_sentinel(val[j]);
     }
-  int spins = 0;
+  int polls = 0;
+  uint64_t since = 0;
   while (!__all(ok)) {
     ok = true;
 #pragma unroll
@@ -1405,11 +1419,7 @@ __device__ __forceinline__ void stage_var(int nw, const int* __restrict__ cols, 
         val[j] = ld_coherent(src[j]);
         ok = ok && !is_sentinel(val[j]);
       }
-    ++spins;
-    if (__any(spins > kSpinLimit || ((spins & 1023) == 0 && ld_coherent(&ctl[2]) != 0))) {
-      if (lane == 0) st_coherent(&ctl[2], 1);
-      break;
-    }
+    if (wait_over(++polls, since, bound, ctl)) break;
   }
 #pragma unroll
   for (int j = 0; j < SJ; ++j)
@@ -1473,7 +1483,7 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free_var(SweepJob<TX
   int c0 = ia[row], W = ia[row + 1] - c0;
   Acc acc = Acc(0);
   for (; W > kVarChunk; W -= kVarChunk, c0 += kVarChunk, val += (size_t)kVarChunk * bk) {
-    stage_var<TX>(kVarChunk, ja + c0, y, 0, 0, x, jb.x64, xw, s, jb.ctl);
+    stage_var<TX>(kVarChunk, ja + c0, y, 0, 0, x, jb.x64, xw, s, jb.ctl, jb.wait);
     if (act)
       for (int c = g; c < kVarChunk; c += G) acc += (Acc)ldnt(val + (size_t)c * bk) * (Acc)s[64 + c];
     wave_lds_sync();
@@ -1484,7 +1494,7 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free_var(SweepJob<TX
     av[i] = TA(0);
     if (act && c < W) av[i] = __builtin_nontemporal_load(val + (size_t)c * bk);
   }
-  stage_var<TX>(W, ja + c0, y, r0, bk, x, jb.x64, xw, s, jb.ctl);
+  stage_var<TX>(W, ja + c0, y, r0, bk, x, jb.x64, xw, s, jb.ctl, jb.wait);
 #pragma unroll
   for (int i0 = 0; i0 < kVarHeld; i0 += 4)
     if (i0 * G < W) {
@@ -1964,6 +1974,7 @@ static void build_tri_var(const BlockCsr& f, bool forward, int prec, DevTri& t) 
     mx = std::max(mx, l);
   }
   t.levels = ns ? mx + 1 : 0;
+  for (int k = 0; k < ns; ++k) t.deps_max = std::max(t.deps_max, ia[k + 1] - ia[k]);
   t.level_ptr.assign(t.levels + 1, 0);
   for (int i = 0; i < ns; ++i) t.level_ptr[lev[i] + 1]++;
   for (int l = 0; l < t.levels; ++l) t.level_ptr[l + 1] += t.level_ptr[l];
@@ -2455,6 +2466,7 @@ static void build_tri_parts(const std::vector<const BlockCsr*>& parts, bool forw
   }
   const int mx = np ? *std::max_element(part_mx.begin(), part_mx.end()) : 0;
   t.levels = nsup ? mx + 1 : 0;
+  for (int64_t k = 0; k < nsup; ++k) t.deps_max = std::max(t.deps_max, ia_all[k + 1] - ia_all[k]);
   t.level_ptr.assign(t.levels + 1, 0);
   for (int64_t i = 0; i < nsup; ++i) t.level_ptr[lev_all[i] + 1]++;
   for (int l = 0; l < t.levels; ++l) t.level_ptr[l + 1] += t.level_ptr[l];
@@ -2708,6 +2720,23 @@ struct SweepLaunch {
   SweepSync* sync;
 };
 
+// sweep_wait_seconds of a launch, in ticks of wall_clock64.
+static uint64_t sweep_wait_ticks(const DevTri& T1, const DevTri* T2, int nrhs) {
+  static const double per_second = [] {
+    int dev = 0, khz = 0;
+    BCM_HIP(hipGetDevice(&dev));
+    BCM_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+    return 1e3 * khz;
+  }();
+  int64_t levels = T1.levels, deps = T1.deps_max, blocks = (int64_t)T1.ndep + T1.nsup;
+  if (T2) {
+    levels += T2->levels;
+    deps = std::max<int64_t>(deps, T2->deps_max);
+    blocks += (int64_t)T2->ndep + T2->nsup;
+  }
+  return (uint64_t)(per_second * sweep_wait_seconds(levels, deps, blocks, nrhs));
+}
+
 static SweepDir sweep_dir(const DevTri& T, const SweepSync& sync) {
   SweepDir d;
   d.order = sync.level_order ? T.level_rows.as<int>() : nullptr;
@@ -2751,6 +2780,7 @@ static void sweep_launch(void (*kern)(SweepJob<TX>), const SweepLaunch& l, int c
   jb.out = l.out ? l.out + o : nullptr;
   jb.ctl = l.sync->ext_ctl ? l.sync->ext_ctl : l.sync->ctl.as<int>();
   jb.skip = l.skip;
+  jb.wait = sweep_wait_ticks(T, l.T2, nr * ng);
   const int64_t ny = (int64_t)T.n * nr * ng;
   hipLaunchKernelGGL((k_sweep_fill<TX>), dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((ny + 255) / 256, 2048))),
                      dim3(256), 0, l.s, ny, jb.y0, jb.y1, jb.ctl, l.skip);
@@ -2877,6 +2907,7 @@ static void sweep_cx_level(const DevTri& T, const double* x, double* y, hipStrea
   jb.y0 = y;
   jb.ctl = T.lctl.as<int>();
   jb.skip = skip;
+  jb.wait = sweep_wait_ticks(T, nullptr, NR);
   for (int l = 0; l < T.levels; ++l) {
     jb.nsup = jb.npos = T.level_ptr[l + 1] - T.level_ptr[l];
     jb.d0.order = T.level_rows.as<int>() + T.level_ptr[l];

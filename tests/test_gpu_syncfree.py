@@ -211,3 +211,40 @@ def test_syncfree_strips_match_level_schedule(B, fctx, b, size, ngroup, nrhs):
             fctx.sync()
             lctx.sync()
             assert rel(dz.host(), dl.host()) < tol
+
+
+def chain(B, ns, b, seed):
+    """Block-tridiagonal system and its ILU2 factor, which is then exact: one
+    row a level, as many levels as rows."""
+    rng = np.random.default_rng(seed)
+    rows = np.arange(ns)
+    ja = np.stack([rows - 1, rows, rows + 1], axis=1)
+    keep = (ja >= 0) & (ja < ns)
+    a = 0.2 * rng.standard_normal((ns, 3, b, b))
+    a[:, 1] += 4.0 * np.eye(b)
+    ia = np.concatenate([[0], np.cumsum(keep.sum(axis=1))])
+    m = B.Matrix.from_arrays(np.arange(ns + 1) * b, ia, ja[keep], a[keep].ravel(), False)
+    return m, a  # a[r, j]: transposed block (r, r - 1 + j)
+
+
+@pytest.mark.parametrize("ns,b", [(1000000, 3), (60000, 16)])
+def test_syncfree_long_chain(B, fctx, ns, b):
+    """A million levels: rows wait for as long as the sweep lasts, with no
+    other reason to give up (0.4 s a sweep, most of it polls of values within
+    a strip). M = A here, so M^-1 (A x) = x."""
+    m, a = chain(B, ns, b, seed=b)
+    f = B.Factor.ilu2(m, B.default_params(tau1=1e-9, tau2=1e-11))
+    print(f"long chain ns={ns} b={b}", flush=True)
+    x = np.random.default_rng(9).standard_normal((ns, b))
+    ax = np.einsum("rcb,rc->rb", a[:, 1], x)
+    ax[1:] += np.einsum("rcb,rc->rb", a[1:, 0], x[:-1])
+    ax[:-1] += np.einsum("rcb,rc->rb", a[:-1, 2], x[1:])
+    dr, dz = dev(B, ax.ravel()), B.DeviceArray(m.n)
+    fctx.precond(f, dr, dz)
+    fctx.sync()
+    # dominant diagonal blocks: nothing grows along the chain, and ILU2 drops what is below 1e-9
+    assert rel(dz.host(), x.ravel()) < 1e-7
+    y = dz.host()
+    fctx.precond(f, dr, dz)
+    fctx.sync()
+    assert np.array_equal(dz.host(), y)
