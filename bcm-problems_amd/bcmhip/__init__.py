@@ -578,7 +578,7 @@ class Context:
 
     def raise_wait_flag(self):
         """Test hook: the next solve's sync-free waits exit at once and the
-        solve is repeated from its initial guess."""
+        solve is repeated from its initial guess, level by level."""
         _check(lib().bcm_context_raise_wait_flag(self.h))
 
     def profile(self, enable: bool = True):

@@ -832,20 +832,28 @@ void solve(Matrix& A, Factor& F, Context& ctx, const SolveOptions& opt, const do
     BCM_HIP(hipStreamSynchronize(ctx.stream));
   };
   // If a wait of a sync-free sweep hit its bound (another process held the
-  // GPU for long), the solve is repeated from the same x0.
-  const bool fast = ctx.sweep_mode == 1;
+  // GPU for long), the solve is repeated from the same x0 with one launch per
+  // dependency level, which never waits.
+  const bool syncfree = ctx.sweep_mode == 1;
   const int64_t n = A.d.n;
   double* x0 = nullptr;
-  if (fast) {
+  if (syncfree) {
     x0 = ctx.vec(87, (size_t)n * 8);
     launch_copy(n, x, x0, ctx.stream);
   }
   run();
-  if (fast && ctx.sync.error(ctx.stream)) {
+  if (syncfree && ctx.sync.error(ctx.stream)) {
     ctx.sync.clear(ctx.stream);
     launch_copy(n, x0, x, ctx.stream);
     st = SolveStats();
-    run();
+    ctx.sweep_mode = 0;
+    try {
+      run();
+    } catch (...) {
+      ctx.sweep_mode = 1;
+      throw;
+    }
+    ctx.sweep_mode = 1;
   }
   ctx.check_sweep_error();
   st.seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

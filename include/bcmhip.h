@@ -238,7 +238,7 @@ int bcm_context_set_sweep_mode(bcm_context c, int mode);
 int bcm_context_set_sweep_waves(bcm_context c, int waves_per_cu);
 /* Test hook: marks the sync-free sweeps' dependency wait as having reached its
  * bound, so that every wait of the next solve exits at once and the solve
- * takes its recovery path (repeated from x0 after the flag is cleared). No
+ * takes its recovery path (repeated from x0 with one launch per level). No
  * counterpart in the reference. */
 int bcm_context_raise_wait_flag(bcm_context c);
 
