@@ -2697,14 +2697,15 @@ static bool sweep_split_columns(const DevTri& T, int nrhs) {
 // of a level on all waves do 0.7 ns (block 9); a level costs 0.65 us in strips
 // and 1.2 us else. Strips therefore win up to some 600 rows a level.
 static bool sweep_in_strips(const DevTri& T, int nrhs) {
-  return T.strips > 0 && (int64_t)T.nsup * nrhs <= 512LL * T.levels && (int64_t)T.strips * nrhs <= INT32_MAX / 2;
+  return T.strips > 0 && (int64_t)T.nsup * nrhs <= 512LL * T.levels;
 }
 
-// Whether a factor of any block partition takes the sync-free sweep: where its
-// column list and the positions of nrhs columns fit 32-bit indices.
-static bool sweep_var_listed(const DevTri& T, int nrhs) {
-  return T.cptr.p && (int64_t)T.nsup * nrhs * 2 <= INT32_MAX - kSweepWaves;
-}
+constexpr int64_t kLaunchThreads = (1LL << 32) - 1;                      // most threads of a launch
+constexpr int64_t kMostPositions = kLaunchThreads / 64 - 2 * kSweepWaves;  // one wave each
+
+// Whether a factor's sweeps, both in one launch, take the sync-free kernels: where
+// a column's positions fit a launch, and any block partition has its column list.
+static bool sweep_listed(const DevTri& T) { return 2LL * T.nsup <= kMostPositions && (T.b || T.cptr.p); }
 
 // A set of sweeps of one launch: the first over T1, the second (if T2) over T2.
 struct SweepLaunch {
@@ -2758,17 +2759,25 @@ static SweepDir sweep_dir(const DevTri& T, const SweepSync& sync) {
 }
 
 // Fills the outputs and launches `kern` (8 block rows per workgroup, or a
-// strip per workgroup of strip_waves) over columns c0 .. c0 + nr * ng - 1.
+// strip per workgroup of strip_waves) over columns c0 .. c0 + nr * ng - 1. The
+// threads of a launch stay below 2^32 (beyond it ends early, without an error):
+// as many groups of columns a launch as that allows.
 template <class TX>
 static void sweep_launch(void (*kern)(SweepJob<TX>), const SweepLaunch& l, int c0, int nr, int ng,
                          int strip_waves = 0) {
   const DevTri& T = *l.T1;
+  const int64_t group = strip_waves ? (int64_t)T.strips + (l.T2 ? l.T2->strips : 0) : (int64_t)T.nsup * (l.T2 ? 2 : 1);
+  const int64_t most = strip_waves ? kLaunchThreads / (64 * strip_waves) : kMostPositions;
+  const int groups = (int)std::max<int64_t>(1, std::min<int64_t>(ng, most / std::max<int64_t>(1, group)));
+  if (groups < ng) {
+    for (int g = 0; g < ng; g += groups) sweep_launch<TX>(kern, l, c0 + g * nr, nr, std::min(groups, ng - g), strip_waves);
+    return;
+  }
   const size_t o = (size_t)c0 * T.n;
   SweepJob<TX> jb{};
   jb.nsup = T.nsup;
   jb.n = T.n;
   jb.ng = ng;
-  if ((int64_t)T.nsup * ng * 2 > INT32_MAX - kSweepWaves) throw Error(kErrArg, "device sweep exceeds 32-bit indexing");
   jb.npos = T.nsup * ng;
   jb.phases = l.T2 ? 2 : 1;
   jb.x64 = l.x_prec == kF64 ? 1 : 0;
@@ -2977,7 +2986,8 @@ void launch_sweep(const DevTri& T, const void* x, void* y, int vec_prec, int nrh
                   const int* skip, SweepSync* sync, RowGate gate) {
   if (x == y) throw Error(kErrArg, "triangular sweep: input and output must not alias");
   if (T.b == 0 && gate.active) throw Error(kErrArg, "row-gated sweeps need a uniform tuned block size");
-  if (T.b == 0 && !(sync && sweep_var_listed(T, nrhs))) {
+  if (!sweep_listed(T)) sync = nullptr;  // level by level
+  if (T.b == 0 && !sync) {
     launch_sweep_var(T, x, y, vec_prec, nrhs, s, skip);
     return;
   }
@@ -2990,8 +3000,7 @@ void launch_sweep_pair(const DevTri& T1, const DevTri& T2, const double* r, doub
   const char *rb = reinterpret_cast<const char*>(r), *zb = reinterpret_cast<const char*>(z);
   const bool apart = rb + vb <= zb || zb + vb <= rb;
   // In one launch z is filled before r is read and written while it still is.
-  const bool listed = T1.b || (sweep_var_listed(T1, nrhs) && sweep_var_listed(T2, nrhs));
-  if (sync && listed && T1.b == T2.b && T1.nsup == T2.nsup && T1.cplx == T2.cplx && T1.prec == T2.prec &&
+  if (sync && sweep_listed(T1) && sweep_listed(T2) && T1.b == T2.b && T1.nsup == T2.nsup && T1.cplx == T2.cplx && T1.prec == T2.prec &&
       apart) {
     void* y1 = vec_prec == kF64 ? static_cast<void*>(z) : w1;
     double* out = vec_prec == kF64 ? nullptr : z;

@@ -213,6 +213,23 @@ def test_syncfree_strips_match_level_schedule(B, fctx, b, size, ngroup, nrhs):
             assert rel(dz.host(), dl.host()) < tol
 
 
+def test_syncfree_more_positions_than_a_launch(B, fctx):
+    """70000 rows x 512 columns x 2 sweeps are 71.7 million waves, more than the
+    2^32 threads that one launch takes."""
+    ns, nrhs = 70000, 512
+    m, f = coupled_groups(B, 2, ns // 2, [1], seed=4)
+    print(f"{ns} rows x {nrhs} columns", flush=True)
+    r = np.asfortranarray(np.random.default_rng(8).standard_normal((ns, nrhs)))
+    lctx = B.Context()
+    lctx.set_sweep_mode(0)
+    dr, dz, dl = dev(B, r), B.DeviceArray((ns, nrhs)), B.DeviceArray((ns, nrhs))
+    fctx.precond(f, dr, dz, nrhs)
+    lctx.precond(f, dr, dl, nrhs)
+    fctx.sync()
+    lctx.sync()
+    assert rel(dz.host(), dl.host()) < 1e-13
+
+
 def chain(B, ns, b, seed):
     """Block-tridiagonal system and its ILU2 factor, which is then exact: one
     row a level, as many levels as rows."""
