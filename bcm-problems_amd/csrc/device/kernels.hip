@@ -771,6 +771,24 @@ __device__ __forceinline__ int sweep_position(const SweepJob<TX>& jb) {
   return pos < jb.npos * jb.phases ? pos : -1;
 }
 
+// Sum of v over the W lane groups of L lanes, in the lanes of group g = 0. The
+// swaps go through the LDS pipe, which the eight rows of a workgroup share: with
+// one for every group, 20 x 20 x 20 x complex block 3 (W = 21) took 702 us, with
+// halves added to halves 397. Few groups are added one by one, as their swaps do
+// not wait for each other: a chain of rows of 24 (W = 5) took 2653 us, 2923 in halves.
+template <int W, int L, class T>
+__device__ __forceinline__ T group_sum(T v, int lane, int g) {
+  if constexpr (W > 5) {
+    constexpr int H = (W + 1) / 2;
+    const T t = __shfl(v, lane + H * L);
+    return group_sum<H, L>(g + H < W ? v + t : v, lane, g);
+  }
+  T sum = v;
+#pragma unroll
+  for (int h = 1; h < W; ++h) sum += __shfl(v, lane + h * L);
+  return sum;
+}
+
 // Whether a wave's dependency wait gives up after `polls` rounds: every 1024
 // of them it looks at the error flag, which ends every wait of the launch, and
 // at the time since `since` (0: not yet taken), which raises the flag. The
@@ -960,9 +978,7 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free(SweepJob<TX> jb
   for (int q = 0; q < NR; ++q)
 #pragma unroll
     for (int k = 0; k < V; ++k) {
-      Acc sm = acc[q][k];
-#pragma unroll
-      for (int h = 1; h < G; ++h) sm += __shfl(acc[q][k], lane + h * L);
+      const Acc sm = group_sum<G, L>(acc[q][k], lane, g);
       if (lane < L) s[(lr * V + k) * NR + q] = (TX)((Acc)s[(lr * V + k) * NR + q] - sm);
     }
   wave_lds_sync();
@@ -984,9 +1000,7 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free(SweepJob<TX> jb
   for (int q = 0; q < NR; ++q)
 #pragma unroll
     for (int k = 0; k < V; ++k) {
-      Acc sm = acc[q][k];
-#pragma unroll
-      for (int h = 1; h < G; ++h) sm += __shfl(acc[q][k], lane + h * L);
+      const Acc sm = group_sum<G, L>(acc[q][k], lane, g);
       if (lane < L) {
         const size_t e = (size_t)q * jb.n + (size_t)row * B + lr * V + k;
         st_coherent(&y[e], (TX)sm);
@@ -1094,12 +1108,7 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free_cx(SweepJob<dou
     if (nd > KD) multiply(1, av[1]);
 #pragma unroll
   for (int q = 0; q < NR; ++q) {
-    double sr = ar[q], si = ai[q];
-#pragma unroll
-    for (int h = 1; h < G; ++h) {
-      sr += __shfl(ar[q], lane + h * BC);
-      si += __shfl(ai[q], lane + h * BC);
-    }
+    const double sr = group_sum<G, BC>(ar[q], lane, g), si = group_sum<G, BC>(ai[q], lane, g);
     if (lane < BC) {
       s[lane * NR + q] -= sr;
       s[(BC + lane) * NR + q] -= si;
@@ -1121,12 +1130,7 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free_cx(SweepJob<dou
   }
 #pragma unroll
   for (int q = 0; q < NR; ++q) {
-    double sr = ar[q], si = ai[q];
-#pragma unroll
-    for (int h = 1; h < G; ++h) {
-      sr += __shfl(ar[q], lane + h * BC);
-      si += __shfl(ai[q], lane + h * BC);
-    }
+    const double sr = group_sum<G, BC>(ar[q], lane, g), si = group_sum<G, BC>(ai[q], lane, g);
     if (lane < BC) {
       st_coherent(&y[(size_t)q * jb.n + (size_t)row * B + lane], sr);
       st_coherent(&y[(size_t)q * jb.n + (size_t)row * B + BC + lane], si);
