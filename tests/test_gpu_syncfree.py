@@ -128,26 +128,62 @@ def test_syncfree_pair_matches_level_schedule(B, fctx, b, size, ngroup, nrhs):
         assert rel(dr.host(), want) < tol
 
 
-def test_syncfree_complex_wide_levels(B, fctx):
+def complex_precond(ns, b, low, up, x):
+    """(U D)^-1-type application in numpy, row by row: low by columns, up by
+    rows, inverted diagonal blocks first, blocks column-major."""
+    (lia, lja, la), (uia, uja, ua) = low, up
+    v = x.reshape(ns, b, -1).copy()
+    lb, ub = la.reshape(-1, b, b), ua.reshape(-1, b, b)  # transposed blocks
+    for i in range(ns):
+        v[i] = lb[lia[i]] @ v[i]
+        for j in range(lia[i] + 1, lia[i + 1]):
+            v[lja[j]] -= lb[j] @ v[i]
+    y = v.copy()
+    for i in range(ns - 1, -1, -1):
+        for j in range(uia[i] + 1, uia[i + 1]):
+            v[i] -= ub[j].T @ v[uja[j]]
+        v[i] = ub[uia[i]].T @ v[i]
+    return y.reshape(x.shape), v.reshape(x.shape)
+
+
+# 400 groups of 3: wide levels; 30 groups of 8: rows with more dependencies than
+# two chunks hold. Against complex arithmetic in numpy, in every schedule.
+@pytest.mark.parametrize("bc,size,ngroup,nrhs", [(3, 3, 400, 2), (12, 3, 400, 3), (16, 3, 400, 6), (4, 3, 400, 6), (3, 8, 30, 1),
+                                                 (4, 8, 30, 2), (6, 8, 30, 7), (8, 8, 30, 1), (12, 9, 20, 1), (16, 8, 12, 2)])
+def test_syncfree_complex_levels(B, fctx, bc, size, ngroup, nrhs):
     rng = np.random.default_rng(8)
-    for bc, nrhs in ((3, 2), (12, 3), (16, 6), (4, 6)):
-        ns = 1200  # 400 groups of 3
-        ia, ja = [0], []
-        for r in range(ns):
-            ja += list(range(r, r // 3 * 3 + 3))
-            ia.append(len(ja))
-        a = 0.1 * (rng.standard_normal((len(ja), bc, bc)) + 1j * rng.standard_normal((len(ja), bc, bc)))
-        f = B.Factor.from_complex(np.arange(ns + 1) * bc, (ia, ja, a.ravel()), (ia, ja, a.ravel()))
-        n = ns * 2 * bc
-        print(f"complex wide bc={bc} nrhs={nrhs}", flush=True)
-        dr, dz, dl = dev(B, rng.standard_normal((n, nrhs))), B.DeviceArray((n, nrhs)), B.DeviceArray((n, nrhs))
-        lctx = B.Context()
-        lctx.set_sweep_mode(0)
-        fctx.precond(f, dr, dz, nrhs)
-        lctx.precond(f, dr, dl, nrhs)
-        fctx.sync()
-        lctx.sync()
-        assert rel(dz.host(), dl.host()) < 1e-13
+    ns = size * ngroup
+    ia, ja = [0], []
+    for r in range(ns):
+        ja += list(range(r, r // size * size + size))
+        ia.append(len(ja))
+    ia, ja = np.array(ia), np.array(ja)
+    sp = np.arange(ns + 1) * bc
+    low, up = [(ia, ja, (0.1 * (rng.standard_normal((len(ja), bc, bc)) + 1j * rng.standard_normal((len(ja), bc, bc)))).ravel())
+               for _ in range(2)]
+    f = B.Factor.from_complex(sp, low, up)
+    print(f"complex levels bc={bc} groups {ngroup} x {size} nrhs={nrhs}", flush=True)
+    z = rng.standard_normal((ns * bc, nrhs)) + 1j * rng.standard_normal((ns * bc, nrhs))
+    y, want = complex_precond(ns, bc, low, up, z)
+    dr = dev(B, B.complex_to_real(sp, z))
+    dz, dn = B.DeviceArray((2 * ns * bc, nrhs)), B.DeviceArray((2 * ns * bc, nrhs))
+    try:
+        for mode in (1, 2, 0):
+            fctx.set_sweep_mode(mode)
+            fctx.solve_l(f, 0, dr, dz, nrhs)
+            fctx.sync()
+            assert rel_c(B.real_to_complex(sp, dz.host()), y) < 1e-13, mode
+            fctx.precond(f, dr, dz, nrhs)
+            fctx.precond_noalloc(f, dr, dn, nrhs)
+            fctx.sync()
+            assert rel_c(B.real_to_complex(sp, dz.host()), want) < 1e-12, mode
+            assert np.array_equal(dz.host(), dn.host()), mode
+    finally:
+        fctx.set_sweep_mode(1)
+
+
+def rel_c(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
 
 
 # Any block partition: one-row blocks, the largest (64), and rows whose
