@@ -742,7 +742,7 @@ struct SweepDir {
 
 // A sweep launch: `phases` sweeps (1 or 2) over npos = nsup * ng positions
 // each; position p is block row p / ng (in the order of its direction) and
-// column group p % ng of NR columns. Phase 0 reads x (doubles if x64, else
+// column p % ng. Phase 0 reads x (doubles if x64, else
 // vector values) and writes y0; phase 1 reads y0 and writes y1, and out (as
 // doubles) if given.
 template <class TX>
@@ -806,8 +806,7 @@ __device__ __forceinline__ bool wait_over(int polls, uint64_t& since, uint64_t b
 }
 
 // Stages nd (<= KM) dependency blocks of a row (block rows cols[0..nd) of y,
-// NR columns of leading dimension n) into s[((1 + k) * B + c) * NR + q], and
-// with row >= 0 the row's right-hand side into block 0 of s: x (already a
+// NR columns of leading dimension n) into s[((1 + k) * B + c) * NR + q], and with row >= 0 the row's right-hand side into block 0 of s: x (already a
 // complete vector; doubles if x64) or, when xw is given, the row of xw, waited
 // for like a dependency. Blocks nd .. npad-1 are zero-filled. Each value is
 // loaded once, by one of the 64 lanes, and the lanes re-poll the values still
@@ -882,8 +881,8 @@ __device__ __forceinline__ auto raw_elem(const typename VecOf<TA, V>::T& v, int 
   }
 }
 
-template <int B, int NR, class TA, class TX>
-__global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free(SweepJob<TX> jb) {
+template <int B, int NR, int W, class TA, class TX>
+__global__ __launch_bounds__(64 * W) void k_sweep_free(SweepJob<TX> jb) {
   if (jb.skip && *jb.skip) return;
   using Acc = typename AccOf<TX>::type;
   constexpr int V = sweep_free_width<B>();  // consecutive rows per lane (one vector load per column)
@@ -894,16 +893,16 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free(SweepJob<TX> jb
   constexpr int CK = (KD * B + G - 1) / G;  // columns of a chunk per lane
   constexpr int PD = (B + G - 1) / G;       // diagonal-block columns per lane
   // chunks whose factor values are in flight during the wait: two where they
-  // take up to 240 bytes of registers a lane each, and 64 KB of LDS hold the values
-  constexpr int NC = CK * V * (int)sizeof(TA) <= 240 && B * NR <= 144 ? 2 : 1;
-  __shared__ __align__(16) TX lds[kSweepWaves][(1 + NC * KD) * B * NR];
-  const int pos = sweep_position<kSweepWaves>(jb);
+  // take up to 240 bytes of registers a lane
+  constexpr int NC = CK * V * (int)sizeof(TA) <= 240 && B * NR < 144 ? 2 : 1;
+  __shared__ __align__(16) TX lds[W][(1 + NC * KD) * B * NR];
+  const int pos = sweep_position<W>(jb);
   if (pos < 0) return;  // wave-uniform; no workgroup-level synchronisation below
-  const int lane = threadIdx.x & 63;
   TX* s = lds[threadIdx.x >> 6];
+  const int lane = threadIdx.x & 63;
   const bool second = pos >= jb.npos;
   const int tp = second ? pos - jb.npos : pos, t = tp / jb.ng;
-  const size_t q0 = (size_t)(tp - t * jb.ng) * NR * jb.n;  // first value of the column group
+  const size_t q0 = (size_t)(tp - t * jb.ng) * NR * jb.n;  // first value of the columns
   const int* order = second ? jb.d1.order : jb.d0.order;
   const int fwd = second ? jb.d1.forward : jb.d0.forward;
   const int* __restrict__ ia = second ? jb.d1.ia : jb.d0.ia;
@@ -956,6 +955,7 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free(SweepJob<TX> jb
 #pragma unroll
         for (int k = 0; k < V; ++k) acc[q][k] += (Acc)raw_elem<V, TA>(a[i], k) * yv;
       }
+      if constexpr (NR > 1) __builtin_amdgcn_sched_barrier(0);  // else all of the chunk's values are read first, and spill
     }
   };
   // rows with more than NC chunks of dependencies: the leading ones first
@@ -981,12 +981,9 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free(SweepJob<TX> jb
     for (int k = 0; k < V; ++k) {
       const Acc sm = group_sum<G, L>(acc[q][k], lane, g);
       if (lane < L) s[(lr * V + k) * NR + q] = (TX)((Acc)s[(lr * V + k) * NR + q] - sm);
+      acc[q][k] = Acc(0);
     }
   wave_lds_sync();
-#pragma unroll
-  for (int q = 0; q < NR; ++q)
-#pragma unroll
-    for (int k = 0; k < V; ++k) acc[q][k] = Acc(0);
 #pragma unroll
   for (int i = 0; i < PD; ++i) {
     const int c = g + i * G, cc = c < B ? c : B - 1;
@@ -996,6 +993,7 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free(SweepJob<TX> jb
 #pragma unroll
       for (int k = 0; k < V; ++k) acc[q][k] += (Acc)raw_elem<V, TA>(pd[i], k) * vc;
     }
+    if constexpr (NR > 1) __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
   for (int q = 0; q < NR; ++q)
@@ -1021,7 +1019,7 @@ __device__ __forceinline__ VecOf<double, 2>::T ldnt_c(const double* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const VecOf<double, 2>::T*>(p));
 }
 
-template <int BC, int NR, int W>
+template <int BC, int W>
 __global__ __launch_bounds__(64 * W) void k_sweep_free_cx(SweepJob<double> jb) {
   if (jb.skip && *jb.skip) return;
   using C2 = VecOf<double, 2>::T;
@@ -1030,15 +1028,15 @@ __global__ __launch_bounds__(64 * W) void k_sweep_free_cx(SweepJob<double> jb) {
   constexpr int KD = 3;                       // dependency blocks per chunk
   constexpr int CK = (KD * BC + G - 1) / G;   // complex columns of a chunk per lane
   constexpr int PD = (BC + G - 1) / G;        // diagonal-block columns per lane
-  constexpr int NC = CK * 16 <= 240 && B * NR <= 144 ? 2 : 1;  // chunks in flight, as in k_sweep_free
-  __shared__ __align__(16) double lds[W][(1 + NC * KD) * B * NR];
+  constexpr int NC = CK * 16 <= 240 ? 2 : 1;  // chunks in flight, as in k_sweep_free
+  __shared__ __align__(16) double lds[W][(1 + NC * KD) * B];
   const int pos = sweep_position<W>(jb);
   if (pos < 0) return;  // wave-uniform; no workgroup-level synchronisation below
-  const int lane = threadIdx.x & 63;
   double* s = lds[threadIdx.x >> 6];
+  const int lane = threadIdx.x & 63;
   const bool second = pos >= jb.npos;
   const int tp = second ? pos - jb.npos : pos, t = tp / jb.ng;
-  const size_t q0 = (size_t)(tp - t * jb.ng) * NR * jb.n;
+  const size_t q0 = (size_t)(tp - t * jb.ng) * jb.n;
   const int* order = second ? jb.d1.order : jb.d0.order;
   const int fwd = second ? jb.d1.forward : jb.d0.forward;
   const int* __restrict__ ia = second ? jb.d1.ia : jb.d0.ia;
@@ -1060,12 +1058,7 @@ __global__ __launch_bounds__(64 * W) void k_sweep_free_cx(SweepJob<double> jb) {
     pd[i] = zero;
     if (act && g + i * G < BC) pd[i] = ldnt_c(d + ((g + i * G) * BC + r) * 2);
   }
-  double ar[NR], ai[NR];
-#pragma unroll
-  for (int q = 0; q < NR; ++q) {
-    ar[q] = 0.0;
-    ai[q] = 0.0;
-  }
+  double ar = 0.0, ai = 0.0;
   C2 av[NC][CK];
   auto load_chunk = [&](int k0, int nb, C2(&a)[CK]) {
     const double* blk = off + (size_t)(j0 + k0) * BC * BC * 2 + r * 2;
@@ -1077,24 +1070,21 @@ __global__ __launch_bounds__(64 * W) void k_sweep_free_cx(SweepJob<double> jb) {
     }
   };
   auto multiply = [&](int c, const C2(&a)[CK]) {
-    const double* sc = s + (1 + c * KD) * B * NR;
+    const double* sc = s + (1 + c * KD) * B;
 #pragma unroll
     for (int i = 0; i < CK; ++i) {
       const int tt = g + i * G, tc = tt < KD * BC ? tt : KD * BC - 1;
       const int k = tc / BC, cc = tc - k * BC;
       const bool in = (i + 1) * G <= KD * BC || tt < KD * BC;
-#pragma unroll
-      for (int q = 0; q < NR; ++q) {
-        const double yr = in ? sc[(k * B + cc) * NR + q] : 0.0, yi = in ? sc[(k * B + BC + cc) * NR + q] : 0.0;
-        ar[q] += a[i].x * yr - a[i].y * yi;
-        ai[q] += a[i].y * yr + a[i].x * yi;
-      }
+      const double yr = in ? sc[k * B + cc] : 0.0, yi = in ? sc[k * B + BC + cc] : 0.0;
+      ar += a[i].x * yr - a[i].y * yi;
+      ai += a[i].y * yr + a[i].x * yi;
     }
   };
   int k0 = 0;
   for (; ndep - k0 > NC * KD; k0 += KD) {
     load_chunk(k0, KD, av[0]);
-    stage_deps<B, NR, KD>(KD, KD, ja + j0 + k0, y, jb.n, -1, x, 0, xw, s, jb.ctl, jb.wait);
+    stage_deps<B, 1, KD>(KD, KD, ja + j0 + k0, y, jb.n, -1, x, 0, xw, s, jb.ctl, jb.wait);
     multiply(0, av[0]);
     wave_lds_sync();
   }
@@ -1102,40 +1092,32 @@ __global__ __launch_bounds__(64 * W) void k_sweep_free_cx(SweepJob<double> jb) {
   if (nd > 0) load_chunk(k0, nd < KD ? nd : KD, av[0]);
   if constexpr (NC == 2)
     if (nd > KD) load_chunk(k0 + KD, nd - KD, av[1]);
-  stage_deps<B, NR, NC * KD>(nd, nd > KD ? NC * KD : (nd > 0 ? KD : 0), ja + j0 + k0, y, jb.n, row, x, 0, xw, s,
-                             jb.ctl, jb.wait);
+  stage_deps<B, 1, NC * KD>(nd, nd > KD ? NC * KD : (nd > 0 ? KD : 0), ja + j0 + k0, y, jb.n, row, x, 0, xw, s, jb.ctl,
+                            jb.wait);
   if (nd > 0) multiply(0, av[0]);
   if constexpr (NC == 2)
     if (nd > KD) multiply(1, av[1]);
-#pragma unroll
-  for (int q = 0; q < NR; ++q) {
-    const double sr = group_sum<G, BC>(ar[q], lane, g), si = group_sum<G, BC>(ai[q], lane, g);
+  {
+    const double sr = group_sum<G, BC>(ar, lane, g), si = group_sum<G, BC>(ai, lane, g);
     if (lane < BC) {
-      s[lane * NR + q] -= sr;
-      s[(BC + lane) * NR + q] -= si;
+      s[lane] -= sr;
+      s[BC + lane] -= si;
     }
-    ar[q] = 0.0;
-    ai[q] = 0.0;
   }
+  ar = ai = 0.0;
   wave_lds_sync();
 #pragma unroll
   for (int i = 0; i < PD; ++i) {
     const int c = g + i * G, cc = c < BC ? c : BC - 1;
     const bool in = (i + 1) * G <= BC || c < BC;
-#pragma unroll
-    for (int q = 0; q < NR; ++q) {
-      const double vr = in ? s[cc * NR + q] : 0.0, vi = in ? s[(BC + cc) * NR + q] : 0.0;
-      ar[q] += pd[i].x * vr - pd[i].y * vi;
-      ai[q] += pd[i].y * vr + pd[i].x * vi;
-    }
+    const double vr = in ? s[cc] : 0.0, vi = in ? s[BC + cc] : 0.0;
+    ar += pd[i].x * vr - pd[i].y * vi;
+    ai += pd[i].y * vr + pd[i].x * vi;
   }
-#pragma unroll
-  for (int q = 0; q < NR; ++q) {
-    const double sr = group_sum<G, BC>(ar[q], lane, g), si = group_sum<G, BC>(ai[q], lane, g);
-    if (lane < BC) {
-      st_coherent(&y[(size_t)q * jb.n + (size_t)row * B + lane], sr);
-      st_coherent(&y[(size_t)q * jb.n + (size_t)row * B + BC + lane], si);
-    }
+  const double sr = group_sum<G, BC>(ar, lane, g), si = group_sum<G, BC>(ai, lane, g);
+  if (lane < BC) {
+    st_coherent(&y[(size_t)row * B + lane], sr);
+    st_coherent(&y[(size_t)row * B + BC + lane], si);
   }
 }
 
@@ -1483,9 +1465,9 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_sweep_free_var(SweepJob<TX
   __shared__ Acc fold[kSweepWaves][64];
   const int pos = sweep_position<kSweepWaves>(jb);
   if (pos < 0) return;  // wave-uniform; no workgroup-level synchronisation below
-  const int lane = threadIdx.x & 63;
   TX* s = lds[threadIdx.x >> 6];
   Acc* red = fold[threadIdx.x >> 6];
+  const int lane = threadIdx.x & 63;
   const bool second = pos >= jb.npos;
   const int tp = second ? pos - jb.npos : pos, t = tp / jb.ng;
   const size_t q0 = (size_t)(tp - t * jb.ng) * jb.n;
@@ -2708,32 +2690,31 @@ void launch_spmv(const DevBsr& A, const double* x, double* y, const double* bsub
   }
 }
 
-// Columns per wave and column groups of a sync-free sweep over nrhs columns.
-// A wave that carries all columns reads every factor value once; one wave per
-// column reads them nrhs times (from L2 mostly) but its row takes a fraction
-// of the time, and that is on the dependency chain. So columns are split while
-// the waves of an average level stay within a quarter of the chip's wave slots
-// (16 a CU at these registers): such a sweep is bound by its chain, not by its
-// loads.
-static bool sweep_split_columns(const DevTri& T, int nrhs) {
-  const int64_t level_rows = T.levels > 0 ? (T.nsup + T.levels - 1) / T.levels : 1;
-  return level_rows * nrhs <= 4LL * device_cu_count();
-}
-
 // Whether nrhs columns of a sweep run in strips. A compute unit does a strip's
 // rows at 0.3 - 0.6 us each, so 256 of them do some 2 ns a row, where the rows
 // of a level on all waves do 0.7 ns (block 9); a level costs 0.65 us in strips
 // and 1.2 us else. Strips therefore win up to some 600 rows a level.
-static bool sweep_in_strips(const DevTri& T, int nrhs) {
+static bool in_strips(const DevTri& T, int nrhs) {
   return T.strips > 0 && (int64_t)T.nsup * nrhs <= 512LL * T.levels;
 }
+
+// Rows and columns of an average level: what a launch can work on at a time.
+static int64_t sweep_width(const DevTri& T, int64_t ncol) { return T.levels > 0 ? T.nsup * ncol / T.levels : 0; }
 
 constexpr int64_t kLaunchThreads = (1LL << 32) - 1;                      // most threads of a launch
 constexpr int64_t kMostPositions = kLaunchThreads / 64 - 2 * kSweepWaves;  // one wave each
 
-// Whether a factor's sweeps, both in one launch, take the sync-free kernels: where
-// a column's positions fit a launch, and any block partition has its column list.
-static bool sweep_listed(const DevTri& T) { return 2LL * T.nsup <= kMostPositions && (T.b || T.cptr.p); }
+// Whether nrhs columns of a factor's sweeps, both in one launch, take the
+// sync-free kernels: where a column's positions fit a launch, any block partition
+// has its column list, and with large blocks levels are not as wide as to be
+// bound by memory alone, where one launch per level, all columns of a row on one
+// wave, reads the least. (Cells of block 24, six columns, FP32, ms for 55 steps,
+// sync-free and by levels: 16 cells, 5760 rows and columns a level, 45.6 and 45.5; 40
+// cells 93 and 70.)
+static bool sweep_listed(const DevTri& T, int nrhs) {
+  if (T.b > kStripBlock && !T.cplx && sweep_width(T, nrhs) > 6144) return false;
+  return 2LL * T.nsup <= kMostPositions && (T.b || T.cptr.p);
+}
 
 // A set of sweeps of one launch: the first over T1, the second (if T2) over T2.
 struct SweepLaunch {
@@ -2786,43 +2767,26 @@ static SweepDir sweep_dir(const DevTri& T, const SweepSync& sync) {
   return d;
 }
 
-// Fills the outputs and launches `kern` (8 block rows per workgroup, or a
-// strip per workgroup of strip_waves) over columns c0 .. c0 + nr * ng - 1. The
-// threads of a launch stay below 2^32 (beyond it ends early, without an error):
-// as many groups of columns a launch as that allows.
+// Fills the outputs and launches `kern`, nrhs columns from `first` on, nr of
+// them a position (nrhs is a multiple): `waves` positions at a time and
+// workgroup, or with `strip` a strip and column. Indices and the
+// threads of a launch stay below 2^31 and 2^32: as many columns a launch as
+// that allows.
 template <class TX>
-static void sweep_launch(void (*kern)(SweepJob<TX>), const SweepLaunch& l, int c0, int nr, int ng,
-                         int strip_waves = 0) {
+static void sweep_launch(void (*kern)(SweepJob<TX>), const SweepLaunch& l, int first, int nrhs, int nr, int waves,
+                         bool strip = false) {
   const DevTri& T = *l.T1;
-  const int64_t group = strip_waves ? (int64_t)T.strips + (l.T2 ? l.T2->strips : 0) : (int64_t)T.nsup * (l.T2 ? 2 : 1);
-  const int64_t most = strip_waves ? kLaunchThreads / (64 * strip_waves) : kMostPositions;
-  const int groups = (int)std::max<int64_t>(1, std::min<int64_t>(ng, most / std::max<int64_t>(1, group)));
-  if (groups < ng) {
-    for (int g = 0; g < ng; g += groups) sweep_launch<TX>(kern, l, c0 + g * nr, nr, std::min(groups, ng - g), strip_waves);
-    return;
-  }
-  const size_t o = (size_t)c0 * T.n;
   SweepJob<TX> jb{};
   jb.nsup = T.nsup;
   jb.n = T.n;
-  jb.ng = ng;
-  jb.npos = T.nsup * ng;
   jb.phases = l.T2 ? 2 : 1;
   jb.x64 = l.x_prec == kF64 ? 1 : 0;
   jb.d0 = sweep_dir(T, *l.sync);
   if (l.T2) jb.d1 = sweep_dir(*l.T2, *l.sync);
-  jb.x = static_cast<const char*>(l.x) + o * (jb.x64 ? 8 : 4);
-  jb.y0 = static_cast<TX*>(l.y0) + o;
-  jb.y1 = l.T2 ? static_cast<TX*>(l.y1) + o : nullptr;
-  jb.out = l.out ? l.out + o : nullptr;
   jb.ctl = l.sync->ext_ctl ? l.sync->ext_ctl : l.sync->ctl.as<int>();
   jb.skip = l.skip;
-  jb.wait = sweep_wait_ticks(T, l.T2, nr * ng);
-  const int64_t ny = (int64_t)T.n * nr * ng;
-  hipLaunchKernelGGL((k_sweep_fill<TX>), dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((ny + 255) / 256, 2048))),
-                     dim3(256), 0, l.s, ny, jb.y0, jb.y1, jb.ctl, l.skip);
-  if (strip_waves) {
-    jb.npos = T.strips * ng;
+  jb.wait = sweep_wait_ticks(T, l.T2, nrhs);
+  if (strip) {
     auto dir = [](const DevTri& t, SweepDir& d) {
       d.order = t.strip_rows.as<int>();
       d.ja = t.strip_code.as<int>();
@@ -2830,58 +2794,76 @@ static void sweep_launch(void (*kern)(SweepJob<TX>), const SweepLaunch& l, int c
     };
     dir(T, jb.d0);
     if (l.T2) dir(*l.T2, jb.d1);
-    const int units = (T.strips + (l.T2 ? l.T2->strips : 0)) * ng;
-    const int rows = std::max(T.strip_rows_max, l.T2 ? l.T2->strip_rows_max : 0);
-    hipLaunchKernelGGL(kern, dim3(units), dim3(64 * strip_waves), (size_t)rows * T.b * sizeof(TX), l.s, jb);
-    BCM_HIP(hipGetLastError());
-    return;
   }
-  const int grid = (jb.npos * jb.phases + kSweepWaves - 1) / kSweepWaves;
-  hipLaunchKernelGGL(kern, dim3(std::max(1, grid)), dim3(64 * kSweepWaves), 0, l.s, jb);
-  BCM_HIP(hipGetLastError());
+  const int64_t threads = 64LL * waves;
+  // positions (or strips) of a group of columns, and the most a launch takes
+  const int64_t column = strip ? (int64_t)T.strips + (l.T2 ? l.T2->strips : 0) : (int64_t)T.nsup * jb.phases;
+  const int64_t most = strip ? kLaunchThreads / threads : kMostPositions;
+  const int groups = (int)std::max<int64_t>(1, std::min<int64_t>(nrhs / nr, most / std::max<int64_t>(1, column)));
+  for (int c0 = first; c0 < first + nrhs; c0 += groups * nr) {
+    const size_t o = (size_t)c0 * T.n;
+    jb.ng = std::min(groups, (first + nrhs - c0) / nr);
+    jb.x = static_cast<const char*>(l.x) + o * (jb.x64 ? 8 : 4);
+    jb.y0 = static_cast<TX*>(l.y0) + o;
+    jb.y1 = l.T2 ? static_cast<TX*>(l.y1) + o : nullptr;
+    jb.out = l.out ? l.out + o : nullptr;
+    const int64_t ny = (int64_t)T.n * jb.ng * nr;
+    hipLaunchKernelGGL((k_sweep_fill<TX>), dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((ny + 255) / 256, 2048))),
+                       dim3(256), 0, l.s, ny, jb.y0, jb.y1, jb.ctl, l.skip);
+    if (strip) {
+      jb.npos = T.strips * jb.ng;
+      const int rows = std::max(T.strip_rows_max, l.T2 ? l.T2->strip_rows_max : 0);
+      hipLaunchKernelGGL(kern, dim3((unsigned)(column * jb.ng)), dim3((unsigned)threads),
+                         (size_t)rows * T.b * sizeof(TX), l.s, jb);
+    } else {
+      jb.npos = T.nsup * jb.ng;
+      const int64_t grid = ((int64_t)jb.npos * jb.phases + waves - 1) / waves;
+      hipLaunchKernelGGL(kern, dim3((unsigned)std::max<int64_t>(1, grid)), dim3((unsigned)threads), 0, l.s, jb);
+    }
+    BCM_HIP(hipGetLastError());
+  }
 }
 
 template <int B, class TA, class TX>
 static void sweep_free(const SweepLaunch& l, int nrhs) {
   if constexpr (B <= kStripBlock) {
-    if (l.sync->level_order && sweep_in_strips(*l.T1, nrhs) && (!l.T2 || sweep_in_strips(*l.T2, nrhs))) {
-      sweep_launch<TX>(k_sweep_strip<B, strip_waves(B), TA, TX>, l, 0, 1, nrhs, strip_waves(B));
+    if (l.sync->level_order && in_strips(*l.T1, nrhs) && (!l.T2 || in_strips(*l.T2, nrhs))) {
+      sweep_launch<TX>(k_sweep_strip<B, strip_waves(B), TA, TX>, l, 0, nrhs, 1, strip_waves(B), true);
       return;
     }
   }
-  if (sweep_split_columns(*l.T1, nrhs)) {
-    sweep_launch<TX>(k_sweep_free<B, 1, TA, TX>, l, 0, 1, nrhs);
-    return;
+  // Workgroups draw their tickets one after another, 11 ns each: twice the rows
+  // a ticket for wide levels, where the registers of a row allow it. (Both
+  // sweeps in us, 8 and 16 rows a ticket: 46 x 46 x 46 x block 6, 382 rows a
+  // level, 642 and 638, two columns 815 and 691, six 1832 and 1215; 30 x 30 x 30 x
+  // block 12, 600 rows and columns a level, 387 and 403, 1800 607 and 534.)
+  const int64_t wide = sweep_width(*l.T1, nrhs);
+  if constexpr (B <= kStripBlock) {
+    if (wide > (B <= 9 ? 512 : 1024)) {
+      sweep_launch<TX>(k_sweep_free<B, 1, 2 * kSweepWaves, TA, TX>, l, 0, nrhs, 1, 2 * kSweepWaves);
+      return;
+    }
   }
+  // One wave per column: its row is short, and where the chain of levels is what
+  // takes the time that is all that counts. With larger blocks and levels that
+  // keep every wave busy, three columns a wave, which read a row's factor values
+  // once. (Cells of block 24, six columns, ms for 55 steps of their FP64 and FP32
+  // solves, one and three columns a wave: 4 cells, 1440 rows and columns a level, 25.3
+  // and 24.4, 20.3 and 21.9; 8 cells 42.0 and 34.4, 30.7 and 30.0; 16 cells 73.7 and
+  // 53.9, 50.1 and 45.6. Six columns a wave do not fit the registers.)
   int done = 0;
-  while (done < nrhs) {
-    const int left = nrhs - done;
-    if (left >= 6) { sweep_launch<TX>(k_sweep_free<B, 6, TA, TX>, l, done, 6, 1); done += 6; }
-    else if (left >= 3) { sweep_launch<TX>(k_sweep_free<B, 3, TA, TX>, l, done, 3, 1); done += 3; }
-    else if (left == 2) { sweep_launch<TX>(k_sweep_free<B, 2, TA, TX>, l, done, 2, 1); done += 2; }
-    else { sweep_launch<TX>(k_sweep_free<B, 1, TA, TX>, l, done, 1, 1); done += 1; }
+  if constexpr (B > kStripBlock) {
+    if (wide > 2048) {
+      done = nrhs / 3 * 3;
+      if (done) sweep_launch<TX>(k_sweep_free<B, 3, kSweepWaves, TA, TX>, l, 0, done, 3, kSweepWaves);
+    }
   }
-}
-
-template <int BC>
-static void sweep_free_cx(const SweepLaunch& l, int nrhs) {
-  if (sweep_split_columns(*l.T1, nrhs)) {
-    sweep_launch<double>(k_sweep_free_cx<BC, 1, kSweepWaves>, l, 0, 1, nrhs);
-    return;
-  }
-  int done = 0;
-  while (done < nrhs) {
-    const int left = nrhs - done;
-    if (left >= 6) { sweep_launch<double>(k_sweep_free_cx<BC, 6, kSweepWaves>, l, done, 6, 1); done += 6; }
-    else if (left >= 3) { sweep_launch<double>(k_sweep_free_cx<BC, 3, kSweepWaves>, l, done, 3, 1); done += 3; }
-    else if (left == 2) { sweep_launch<double>(k_sweep_free_cx<BC, 2, kSweepWaves>, l, done, 2, 1); done += 2; }
-    else { sweep_launch<double>(k_sweep_free_cx<BC, 1, kSweepWaves>, l, done, 1, 1); done += 1; }
-  }
+  if (done < nrhs) sweep_launch<TX>(k_sweep_free<B, 1, kSweepWaves, TA, TX>, l, done, nrhs - done, 1, kSweepWaves);
 }
 
 template <class TA, class TX>
 static void sweep_free_var(const SweepLaunch& l, int nrhs) {
-  sweep_launch<TX>(k_sweep_free_var<TA, TX>, l, 0, 1, nrhs);
+  sweep_launch<TX>(k_sweep_free_var<TA, TX>, l, 0, nrhs, 1, kSweepWaves);
 }
 
 template <int B, int NR, class TA, class TX>
@@ -2929,48 +2911,38 @@ static void sweep_prec(const SweepLaunch& l, int vec_prec, int nrhs, RowGate gat
   }
 }
 
-template <int BC, int NR>
-static void sweep_cx_level(const DevTri& T, const double* x, double* y, hipStream_t s, const int* skip) {
+template <int BC>
+static void sweep_cx(const SweepLaunch& l, int nrhs) {
+  if (l.sync) {
+    sweep_launch<double>(k_sweep_free_cx<BC, kSweepWaves>, l, 0, nrhs, 1, kSweepWaves);
+    return;
+  }
   // level by level: a launch's rows depend only on rows of earlier launches, so
   // its waits never spin; one wave a workgroup, which spreads a level over the
   // chip (10 x 10 x 10 x complex block 16, both sweeps: 333 us with eight, 252 with one)
+  const DevTri& T = *l.T1;
   SweepJob<double> jb{};
   jb.n = T.n;
-  jb.ng = 1;
   jb.phases = 1;
   jb.x64 = 1;
   jb.d0 = SweepDir{nullptr, T.ia.as<int>(), T.ja.as<int>(), T.off.p, T.diag.p, T.forward ? 1 : 0,
                    nullptr, nullptr, nullptr};
-  jb.x = x;
-  jb.y0 = y;
   jb.ctl = T.lctl.as<int>();
-  jb.skip = skip;
-  jb.wait = sweep_wait_ticks(T, nullptr, NR);
-  for (int l = 0; l < T.levels; ++l) {
-    jb.nsup = jb.npos = T.level_ptr[l + 1] - T.level_ptr[l];
-    jb.d0.order = T.level_rows.as<int>() + T.level_ptr[l];
-    hipLaunchKernelGGL((k_sweep_free_cx<BC, NR, 1>), dim3(jb.npos), dim3(64), 0, s, jb);
+  jb.skip = l.skip;
+  jb.wait = sweep_wait_ticks(T, nullptr, nrhs);
+  const int columns = (int)std::max<int64_t>(1, std::min<int64_t>(nrhs, kMostPositions / std::max(1, T.nsup)));
+  for (int c0 = 0; c0 < nrhs; c0 += columns) {
+    jb.ng = std::min(columns, nrhs - c0);
+    jb.x = static_cast<const double*>(l.x) + (size_t)c0 * T.n;
+    jb.y0 = static_cast<double*>(l.y0) + (size_t)c0 * T.n;
+    for (int lv = 0; lv < T.levels; ++lv) {
+      jb.nsup = T.level_ptr[lv + 1] - T.level_ptr[lv];
+      jb.npos = jb.nsup * jb.ng;
+      jb.d0.order = T.level_rows.as<int>() + T.level_ptr[lv];
+      hipLaunchKernelGGL((k_sweep_free_cx<BC, 1>), dim3(jb.npos), dim3(64), 0, l.s, jb);
+    }
   }
   BCM_HIP(hipGetLastError());
-}
-
-template <int BC>
-static void sweep_cx(const SweepLaunch& l, int nrhs) {
-  if (l.sync) {
-    sweep_free_cx<BC>(l, nrhs);
-    return;
-  }
-  const DevTri& T = *l.T1;
-  int done = 0;
-  while (done < nrhs) {
-    const int left = nrhs - done;
-    const double* x = static_cast<const double*>(l.x) + (size_t)done * T.n;
-    double* y = static_cast<double*>(l.y0) + (size_t)done * T.n;
-    if (left >= 6) { sweep_cx_level<BC, 6>(T, x, y, l.s, l.skip); done += 6; }
-    else if (left >= 3) { sweep_cx_level<BC, 3>(T, x, y, l.s, l.skip); done += 3; }
-    else if (left == 2) { sweep_cx_level<BC, 2>(T, x, y, l.s, l.skip); done += 2; }
-    else { sweep_cx_level<BC, 1>(T, x, y, l.s, l.skip); done += 1; }
-  }
 }
 
 static void sweep_dispatch(const SweepLaunch& l, int vec_prec, int nrhs, RowGate gate) {
@@ -3014,7 +2986,7 @@ void launch_sweep(const DevTri& T, const void* x, void* y, int vec_prec, int nrh
                   const int* skip, SweepSync* sync, RowGate gate) {
   if (x == y) throw Error(kErrArg, "triangular sweep: input and output must not alias");
   if (T.b == 0 && gate.active) throw Error(kErrArg, "row-gated sweeps need a uniform tuned block size");
-  if (!sweep_listed(T)) sync = nullptr;  // level by level
+  if (!sweep_listed(T, nrhs)) sync = nullptr;  // level by level
   if (T.b == 0 && !sync) {
     launch_sweep_var(T, x, y, vec_prec, nrhs, s, skip);
     return;
@@ -3028,7 +3000,7 @@ void launch_sweep_pair(const DevTri& T1, const DevTri& T2, const double* r, doub
   const char *rb = reinterpret_cast<const char*>(r), *zb = reinterpret_cast<const char*>(z);
   const bool apart = rb + vb <= zb || zb + vb <= rb;
   // In one launch z is filled before r is read and written while it still is.
-  if (sync && sweep_listed(T1) && sweep_listed(T2) && T1.b == T2.b && T1.nsup == T2.nsup && T1.cplx == T2.cplx && T1.prec == T2.prec &&
+  if (sync && sweep_listed(T1, nrhs) && sweep_listed(T2, nrhs) && T1.b == T2.b && T1.nsup == T2.nsup && T1.cplx == T2.cplx && T1.prec == T2.prec &&
       apart) {
     void* y1 = vec_prec == kF64 ? static_cast<void*>(z) : w1;
     double* out = vec_prec == kF64 ? nullptr : z;

@@ -98,10 +98,11 @@ def coupled_groups(B, size, ngroup, blocks, seed):
     return m, B.Factor.ilu2(m, B.default_params(tau1=1e-9, tau2=1e-11))
 
 
-# 600 groups of 3: level of 600 rows, one wave carries 2, 3 or 6 columns; 12
-# groups of 9: narrow levels, one wave per column, and rows of 8 dependencies
-# (more than the chunks held in registers)
-GROUPS = [(3, 600, 2), (3, 600, 3), (3, 400, 7), (9, 12, 1), (9, 12, 6), (9, 200, 6)]
+# 600 groups of 3: levels of 600 rows, 16 rows a workgroup (blocks up to 16) or
+# three columns a wave and a rest of one (above: 400 x 7); 16 columns of 400
+# rows: by levels above 16; 12 groups of 9: narrow levels, one wave per column,
+# and rows of 8 dependencies (more than the chunks held in registers)
+GROUPS = [(3, 600, 2), (3, 600, 3), (3, 400, 7), (3, 400, 16), (9, 12, 1), (9, 12, 6), (9, 200, 6)]
 
 
 @pytest.mark.parametrize("size,ngroup,nrhs", GROUPS)
