@@ -1139,13 +1139,6 @@ __global__ __launch_bounds__(64 * W) void k_sweep_free_cx(SweepJob<double> jb) {
 // of k_sweep_free, whose sums cross the wave through LDS, both sweeps of 64 x 64
 // heat, block 9, took 264 us (now 244), of 20 x 19 x 18 x block 12 167 (120), of
 // 16^3 x block 16 120 (105).
-//
-// Waves of a strip, and dependency blocks of a row held in registers (twice,
-// for the next row): in that layout 20 x 20 x 20 x block 8 took 136 us with 8
-// waves, 127 with 16; 20 x 19 x 18 x block 12 (FP64) 166 and 220, block 16 120
-// and 203.
-constexpr int strip_waves(int b) { return b <= 9 ? 16 : 8; }
-constexpr int strip_held(int b) { return b >= 16 ? 3 : 4; }
 
 template <class T> __device__ __forceinline__ T ld_wg(const T* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -2296,75 +2289,8 @@ static bool complex_blocks(const std::vector<double>& src, int b, std::vector<do
   return true;
 }
 
-// Block sizes of k_sweep_strip: up to 16 rows, four lanes each. (At 24, with the
-// layout of k_sweep_free, a row's factor values did not fit the registers twice:
-// 17 x 16 x 15 took 186 us by levels, 162 to 218 us in strips, a periodic 16^3
-// cell 108 against 179.)
-constexpr int kStripBlock = 16;
-
 static bool complex_sweep_block(int b) {
   return b == 6 || b == 8 || b == 12 || b == 16 || b == 24 || b == 32;
-}
-
-// Cuts the rows of t (dependency lists ia, ja; levels lev) into strips for
-// k_sweep_strip.
-static void build_strips(const std::vector<int>& ia, const std::vector<int>& ja, const std::vector<int>& lev,
-                         bool forward, DevTri& t) {
-  const int ns = t.nsup;
-  t.strips = 0;
-  // Mostly rows whose dependencies the kernel holds, and levels that stay
-  // narrow (sweep_in_strips); other factors need no strips.
-  int64_t more = 0;
-  for (int r = 0; r < ns; ++r) more += ia[r + 1] - ia[r] > strip_held(t.b) ? 1 : 0;
-  if (ns < 32 || more * 8 > ns || ns > 512LL * t.levels) return;
-  // 16 rows a strip, up to one strip per compute unit; a strip's values within
-  // 48 KB of LDS. (64 x 64 heat, block 9, both sweeps: 448 us by levels; strips
-  // of 16, 32, 64 rows: 244, 249, 254 us.)
-  const int64_t bytes = (int64_t)ns * t.b * 8, lds = 48 << 10;
-  const int P = (int)std::max<int64_t>(std::min(256, ns / 16), (bytes + lds - t.b * 8 - 1) / (lds - t.b * 8));
-  // depth-first topological order
-  std::vector<int> sptr(ns + 1, 0), succ(ja.size()), cnt(ns), seq, stack;
-  for (int r = 0; r < ns; ++r) cnt[r] = ia[r + 1] - ia[r];
-  for (int j = 0; j < ia[ns]; ++j) sptr[ja[j] + 1]++;
-  for (int r = 0; r < ns; ++r) sptr[r + 1] += sptr[r];
-  {
-    std::vector<int> at(sptr.begin(), sptr.end() - 1);
-    for (int q = 0; q < ns; ++q) {
-      const int r = forward ? q : ns - 1 - q;
-      for (int j = ia[r]; j < ia[r + 1]; ++j) succ[at[ja[j]]++] = r;
-    }
-  }
-  for (int q = ns - 1; q >= 0; --q) {
-    const int r = forward ? q : ns - 1 - q;
-    if (cnt[r] == 0) stack.push_back(r);
-  }
-  seq.reserve(ns);
-  while (!stack.empty()) {
-    const int r = stack.back();
-    stack.pop_back();
-    seq.push_back(r);
-    const size_t s0 = stack.size();
-    for (int k = sptr[r]; k < sptr[r + 1]; ++k)
-      if (--cnt[succ[k]] == 0) stack.push_back(succ[k]);
-    std::reverse(stack.begin() + s0, stack.end());
-  }
-  std::vector<int> ptr(P + 1), strip(ns), pos(ns), code(std::max<size_t>(ja.size(), 1));
-  for (int k = 0; k <= P; ++k) ptr[k] = (int)((int64_t)ns * k / P);
-  t.strip_rows_max = 0;
-  for (int k = 0; k < P; ++k) {
-    std::stable_sort(seq.begin() + ptr[k], seq.begin() + ptr[k + 1], [&](int a, int b) { return lev[a] < lev[b]; });
-    for (int i = ptr[k]; i < ptr[k + 1]; ++i) {
-      strip[seq[i]] = k;
-      pos[seq[i]] = i - ptr[k];
-    }
-    t.strip_rows_max = std::max(t.strip_rows_max, ptr[k + 1] - ptr[k]);
-  }
-  for (int r = 0; r < ns; ++r)
-    for (int j = ia[r]; j < ia[r + 1]; ++j) code[j] = strip[ja[j]] == strip[r] ? -1 - pos[ja[j]] : ja[j];
-  t.strips = P;
-  t.strip_rows.upload(seq.data(), std::max<size_t>(seq.size(), 1) * 4);
-  t.strip_ptr.upload(ptr.data(), ptr.size() * 4);
-  t.strip_code.upload(code.data(), code.size() * 4);
 }
 
 // cplx: the parts are real equivalents of complex factors; their blocks are
@@ -2491,7 +2417,16 @@ static void build_tri_parts(const std::vector<const BlockCsr*>& parts, bool forw
   t.level_rows.upload(rows.data(), std::max<size_t>(rows.size(), 1) * 4);
   t.ia.upload(ia_all.data(), ia_all.size() * 4);
   t.ja.upload(ja_all.data(), ja_all.size() * 4);
-  if (np == 1 && !cplx && b <= kStripBlock) build_strips(ia_all, ja_all, lev_all, forward, t);
+  if (np == 1 && !cplx) {
+    const Strips cut = cut_strips(b, prec_bytes(prec), t.levels, ia_all, ja_all, lev_all, forward);
+    t.strips = cut.count;
+    t.strip_rows_max = cut.rows_max;
+    if (cut.count) {
+      t.strip_rows.upload(cut.rows.data(), cut.rows.size() * 4);
+      t.strip_ptr.upload(cut.ptr.data(), cut.ptr.size() * 4);
+      t.strip_code.upload(cut.code.data(), cut.code.size() * 4);
+    }
+  }
 }
 
 void dev_tri_forward(const BlockCsr& f, int prec, DevTri& t, bool cplx) {
@@ -2690,12 +2625,8 @@ void launch_spmv(const DevBsr& A, const double* x, double* y, const double* bsub
   }
 }
 
-// Whether nrhs columns of a sweep run in strips. A compute unit does a strip's
-// rows at 0.3 - 0.6 us each, so 256 of them do some 2 ns a row, where the rows
-// of a level on all waves do 0.7 ns (block 9); a level costs 0.65 us in strips
-// and 1.2 us else. Strips therefore win up to some 600 rows a level.
 static bool in_strips(const DevTri& T, int nrhs) {
-  return T.strips > 0 && (int64_t)T.nsup * nrhs <= 512LL * T.levels;
+  return T.strips > 0 && sweep_in_strips(T.b, prec_bytes(T.prec), T.nsup, T.levels, nrhs);
 }
 
 // Rows and columns of an average level: what a launch can work on at a time.

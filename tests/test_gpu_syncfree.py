@@ -215,9 +215,7 @@ def test_syncfree_any_partition_matches_level_schedule(B, fctx, blocks, size, ng
                 assert rel(dy.host(), dm.host()) < 1e-13
 
 
-# Strips (narrow levels): every block size they are built for, rows with more
-# dependencies than are held, a strip count that does not divide the rows, and
-# the smallest system that has strips (32 rows).
+# Chains of coupled groups: as many levels as rows.
 @pytest.mark.parametrize("b,size,ngroup,nrhs", [
     (3, 4, 8, 1), (6, 4, 60, 2), (8, 5, 83, 1), (9, 4, 90, 6), (12, 4, 70, 1), (16, 3, 50, 3), (16, 4, 12, 1)])
 def test_syncfree_strips_match_level_schedule(B, fctx, b, size, ngroup, nrhs):
@@ -244,6 +242,57 @@ def test_syncfree_strips_match_level_schedule(B, fctx, b, size, ngroup, nrhs):
         for transpose in (False, True):
             dr, dz, dl = dev(B, r), B.DeviceArray((m.n, nrhs)), B.DeviceArray((m.n, nrhs))
             fctx.precond(f, dr, dz, nrhs, precision=precision, transpose=transpose)
+            lctx.precond(f, dr, dl, nrhs, precision=precision, transpose=transpose)
+            fctx.sync()
+            lctx.sync()
+            assert rel(dz.host(), dl.host()) < tol
+
+
+def grid_system(B, nx, ny, b, seed):
+    """An nx x ny grid, small couplings on a large diagonal: the factor keeps the
+    pattern. Every tenth row of a line has seven more earlier neighbours, of its
+    own strip and of others; no row is one of more than one such row. Levels stay
+    the antidiagonals of the grid."""
+    rng = np.random.default_rng(seed)
+    i, j = np.divmod(np.arange(nx * ny), nx)
+    pairs = []
+    for di, dj in ((0, 1), (1, 0), (0, 2), (0, 3), (1, 1), (2, 0), (3, 4), (1, 5), (5, 6)):
+        keep = (i >= di) & (j >= dj) & ((di + dj == 1) | (j % 10 == 9))
+        r = np.flatnonzero(keep)
+        pairs.append(np.stack([r, r - di * nx - dj], axis=1))
+    lo = np.concatenate(pairs)
+    ns = nx * ny
+    r = np.concatenate([lo[:, 0], lo[:, 1], np.arange(ns)])
+    c = np.concatenate([lo[:, 1], lo[:, 0], np.arange(ns)])
+    o = np.lexsort((c, r))
+    r, c = r[o], c[o]
+    a = rng.standard_normal((len(r), b, b)) / b
+    a[r == c] += 1000.0 * np.eye(b)
+    ia = np.concatenate([[0], np.cumsum(np.bincount(r, minlength=ns))])
+    m = B.Matrix.from_arrays(np.arange(ns + 1) * b, ia, c, a.ravel(), False)
+    return m, B.Factor.ilu2(m, B.default_params(tau1=1e-5, tau2=1e-5))
+
+
+# Strips: every block size they are built for; rows with more dependencies than
+# are held (nine: the leading five or six in two chunks), several rows of a level
+# in a strip, strips of three and more rows a wave, columns.
+@pytest.mark.parametrize("b,nx,ny,nrhs", [(3, 10, 103, 1), (6, 11, 372, 2), (8, 12, 341, 1), (9, 20, 660, 1), (9, 41, 40, 6),
+                                          (12, 13, 485, 1), (16, 13, 485, 1), (16, 33, 30, 2)])
+def test_syncfree_strips_with_leading_dependencies(B, plan, fctx, b, nx, ny, nrhs):
+    m, f = grid_system(B, nx, ny, b, seed=b)
+    for bytes_ in (8, 4, 2):
+        strips, deps, shared = plan.factor_strips(f, nx * ny, b, bytes_, nrhs)
+        assert strips and deps == 9 and (shared or nx > 20)
+    print(f"strips b={b} grid {nx} x {ny} nrhs={nrhs}", flush=True)
+    r = np.random.default_rng(6).standard_normal((m.n, nrhs))
+    lctx = B.Context()
+    lctx.set_sweep_mode(0)
+    # couplings are some 1e-4 of the diagonal: a wrong or missing one shows far above the tolerances
+    for precision, tol in ((0, 1e-13), (1, 2e-5), (2, 2e-5)):
+        for transpose in (False, True):
+            dr, dz, dl = dev(B, r), B.DeviceArray((m.n, nrhs)), B.DeviceArray((m.n, nrhs))
+            for _ in range(2):
+                fctx.precond(f, dr, dz, nrhs, precision=precision, transpose=transpose)
             lctx.precond(f, dr, dl, nrhs, precision=precision, transpose=transpose)
             fctx.sync()
             lctx.sync()
