@@ -16,12 +16,14 @@ import numpy as np
 import pytest
 
 from test_complex import complex_system, dense_complex
+from test_host import need_ref
 
 pytestmark = pytest.mark.gpu
 
 
 @pytest.fixture(scope="module")
 def csys(B, O):
+    need_ref(O)
     sp, ia, ja, ac = complex_system(B, 8, 6, 5, 12, seed=21)  # complex blocks of 12: real blocks of 24
     L, U = O.ref_cilu2(sp, ia, ja, ac)
     return dict(sp=sp, ia=ia, ja=ja, ac=ac, L=L, U=U, mc=B.Matrix.from_complex(sp, ia, ja, ac),
@@ -66,6 +68,7 @@ def test_complex_block_kernels_every_block_size(B, O, ctx, bc):
     residual form the solvers launch) through bcm_residual, and both sweep
     schedules against the reference's complex SolveL / SolveU on the
     reference's own complex ILU2 factors."""
+    need_ref(O)
     sp, ia, ja, ac = complex_system(B, 4, 3, 3, bc, seed=40 + bc)
     mc = B.Matrix.from_complex(sp, ia, ja, ac)
     L, U = O.ref_cilu2(sp, ia, ja, ac)
@@ -194,6 +197,7 @@ def _drop_in(B, O, sys_, bz, x0, reference=False, **prm):
     x = np.full(sp[-1], np.nan + 0j)
     cbs = _ccallbacks(B, O, sp, ia, ja, ac, bz, x0, x, reference)
     if reference:
+        need_ref(O)
         O.ref_abstract_solver_c(*cbs, memory=10.0, **prm)
         return x, None
     p = B.default_params(**prm)
