@@ -303,9 +303,10 @@ size_t chain_lds(int nin, int nh, int nout) {
   return (size_t)16 * (2 * 4 * up16(nh) + 2 * (up32(nin) + 8 + 2 * (up32(nh) + 8) + up32(nout) + 8));
 }
 
-// Rows [16 * blockIdx.x, + 16) of the batch: out = MLP(x) if t is null, else
+// Tile tile0 + blockIdx.x of 16 rows of the batch: out = MLP(x) if t is null, else
 // the loss against t, the activations' gradients and the tape.
-__global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int M, int ms, MlpDims d, const float* __restrict__ p,
+__global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int tile0, int M, int ms, MlpDims d,
+                                                             const float* __restrict__ p,
                                                              const unsigned short* __restrict__ pk,
                                                              const float* __restrict__ x, const float* __restrict__ t,
                                                              float* __restrict__ out, float scale, MlpTape tape) {
@@ -318,7 +319,7 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int M, int ms, MlpD
   unsigned short* h2b = h1b + 16 * lh;
   unsigned short* dyb = h2b + 16 * lh;
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  const int m0 = blockIdx.x * 16;
+  const int tile = tile0 + blockIdx.x, m0 = tile * 16;
   const int ki = up32(d.nin) >> 5, kh = up32(d.nh) >> 5, ko = up32(d.nout) >> 5, th = hc >> 4, to = up16(d.nout) >> 4;
   const ChainHeld w1 = chain_first(pk + d.f[0], ki, th), w2 = chain_first(pk + d.f[1], kh, th);
   // operands: x in BF16, zeros in the padding that no product writes
@@ -356,7 +357,7 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int M, int ms, MlpD
   hidden(h1b, lh, kh, 1, w2, h2f, h2b, tape.h2);
   const ChainHeld r3 = chain_first(pk + d.r[2], ko, t ? th : 0);
   double loss = 0.0;
-  float* cp = t ? tape.colpart + (size_t)blockIdx.x * (2 * d.nh + d.nout) : nullptr;
+  float* cp = t ? tape.colpart + (size_t)tile * (2 * d.nh + d.nout) : nullptr;
   {
     const float* b = p + d.b_off[2];
     chain_product(h2b, lh, pk + d.f[2], kh, to, w3, [&](int tn, v4f acc) {
@@ -394,7 +395,7 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int M, int ms, MlpD
   if (threadIdx.x == 0) {
     double s = 0.0;
     for (int w = 0; w < kChainWaves; ++w) s += ls[w];
-    tape.losspart[blockIdx.x] = s;
+    tape.losspart[tile] = s;
   }
   // dz2 = (dy W3^T) * (1 - h2^2) into h1's operand, dz1 = (dz2 W2^T) * (1 - h1^2)
   chain_product(dyb, ly, pk + d.r[2], ko, th, r3, [&](int tn, v4f acc) {
@@ -745,9 +746,11 @@ void Mlp::chain(hipStream_t s, int M, const float* x, const float* t, float* out
     tp.colpart = reinterpret_cast<float*>(tp.dy + m32 * up16(nout));
   }
   const double total = (double)M * nout;
-  hipLaunchKernelGGL(k_mlp_chain, dim3(mt), dim3(kChainThreads), chain_lds(nin, nh, nout), s, M, ms, d,
-                     params.as<const float>(), wpk.as<const unsigned short>(), x, t, out,
-                     2.0f / (float)((int64_t)M * nout), tp);
+  constexpr int kMostTiles = 1 << 21;  // of 1024 threads: a launch takes less than 2^32
+  for (int tile = 0; tile < mt; tile += kMostTiles)
+    hipLaunchKernelGGL(k_mlp_chain, dim3(std::min(kMostTiles, mt - tile)), dim3(kChainThreads), chain_lds(nin, nh, nout),
+                       s, tile, M, ms, d, params.as<const float>(), wpk.as<const unsigned short>(), x, t, out,
+                       2.0f / (float)((int64_t)M * nout), tp);
   if (t) {
     const int th = up16(nh) / 16, to = up16(nout) / 16, ti = up16(nin) / 16;
     const int grid = th * to + th * th + ti * th + (2 * nh + nout + 63) / 64 + 1;

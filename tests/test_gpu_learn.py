@@ -207,3 +207,16 @@ def test_mlp_infinite_weight(B, ctx, layer, batch):
     assert abs(loss - lo) <= 1e-4 * lo
     assert np.array_equal(np.isfinite(g), np.isfinite(go))
     assert relerr(g[np.isfinite(go)], go[np.isfinite(go)]) < 2e-3  # as the gradients of finite weights
+
+
+def test_mlp_more_rows_than_a_launch(B, ctx):
+    """70 million rows: at 16 rows for 1024 threads more than one launch takes."""
+    rows, dims = 70000000, (1, 250, 1)
+    print(f"mlp {dims} rows {rows}", flush=True)
+    m = B.Mlp(*dims, seed=6)
+    part = np.random.default_rng(1).normal(size=(1000003, 1)).astype(np.float32)
+    x = np.tile(part, (rows // len(part) + 1, 1))[:rows]
+    want = m.forward(ctx, part)
+    y = m.forward(ctx, x)
+    for k in range(0, rows, len(part)):  # a row's result does not depend on where it stands
+        assert np.array_equal(y[k:k + len(part)], want[:min(len(part), rows - k)]), k
