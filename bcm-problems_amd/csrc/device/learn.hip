@@ -186,8 +186,7 @@ __global__ void k_to_bf16(int64_t n, const float* __restrict__ w, unsigned short
 // Chosen where the rows of a workgroup fit 63 KB of LDS; larger networks
 // take one product after another (k_gemm_bf16).
 constexpr int kFrag = 512;            // values of a fragment
-constexpr int kChainThreads = 1024;   // one 16-column tile per wave and pass
-constexpr int kChainWaves = kChainThreads / 64;
+constexpr int kChainWaves = 16;       // most waves of a workgroup: one 16-column tile per wave and pass
 
 __host__ __device__ constexpr int up16(int n) { return (n + 15) & ~15; }
 __host__ __device__ constexpr int up32(int n) { return (n + 31) & ~31; }
@@ -251,7 +250,7 @@ __device__ __forceinline__ ChainHeld chain_first(const unsigned short* __restric
   return chain_load(w, ks, tiles, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), 0);
 }
 
-// acc of the tiles tn = wave, wave + kChainWaves, ... of A (16 rows in LDS, ks
+// acc of the tiles tn = wave, wave + waves, ... of A (16 rows in LDS, ks
 // steps of 32) times packed weights, handed to `epi(tn, acc)`; `held` is the
 // wave's chain_first of these weights.
 template <class F>
@@ -259,8 +258,8 @@ __device__ __forceinline__ void chain_product(const unsigned short* a, int lda, 
                                               int ks, int tiles, ChainHeld held, F epi) {
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const unsigned short* ar = a + r * lda + 8 * g;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (int tn = wave; tn < tiles; tn += kChainWaves) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  for (int tn = wave; tn < tiles; tn += waves) {
     v4f acc = {0.f, 0.f, 0.f, 0.f};
     for (int k0 = 0; k0 < ks; k0 += kChainHeld) {
       if (tn != wave || k0) held = chain_load(w, ks, tiles, tn, k0);
@@ -303,13 +302,17 @@ size_t chain_lds(int nin, int nh, int nout) {
   return (size_t)16 * (2 * 4 * up16(nh) + 2 * (up32(nin) + 8 + 2 * (up32(nh) + 8) + up32(nout) + 8));
 }
 
-// Tile tile0 + blockIdx.x of 16 rows of the batch: out = MLP(x) if t is null, else
-// the loss against t, the activations' gradients and the tape.
-__global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int tile0, int M, int ms, MlpDims d,
-                                                             const float* __restrict__ p,
-                                                             const unsigned short* __restrict__ pk,
-                                                             const float* __restrict__ x, const float* __restrict__ t,
-                                                             float* __restrict__ out, float scale, MlpTape tape) {
+// Tile tile0 + blockIdx.x of 16 rows of the batch: out = MLP(x), or to train the
+// loss against t, the activations' gradients and the tape. A forward pass has as
+// many waves as the widest layer has tiles, so that a small network leaves room
+// for other workgroups: 65536 rows through 1-1-1 took 80 us with 16 waves (13 as
+// separate products), 13 now; through 4-32-96 89 (54), 53 now.
+template <bool kTrain>
+__global__ __launch_bounds__(64 * kChainWaves) void k_mlp_chain(int tile0, int M, int ms, MlpDims d,
+                                                                const float* __restrict__ p,
+                                                                const unsigned short* __restrict__ pk,
+                                                                const float* __restrict__ x, const float* __restrict__ t,
+                                                                float* __restrict__ out, float scale, MlpTape tape) {
   extern __shared__ __align__(16) char smem[];
   const int hc = up16(d.nh), lx = up32(d.nin) + 8, lh = up32(d.nh) + 8, ly = up32(d.nout) + 8;
   float* h1f = reinterpret_cast<float*>(smem);
@@ -319,18 +322,23 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int tile0, int M, i
   unsigned short* h2b = h1b + 16 * lh;
   unsigned short* dyb = h2b + 16 * lh;
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  const int tile = tile0 + blockIdx.x, m0 = tile * 16;
+  const int tile = tile0 + blockIdx.x, m0 = tile * 16, nt = blockDim.x;
   const int ki = up32(d.nin) >> 5, kh = up32(d.nh) >> 5, ko = up32(d.nout) >> 5, th = hc >> 4, to = up16(d.nout) >> 4;
   const ChainHeld w1 = chain_first(pk + d.f[0], ki, th), w2 = chain_first(pk + d.f[1], kh, th);
-  // operands: x in BF16, zeros in the padding that no product writes
-  for (int e = threadIdx.x; e < 16 * lx; e += kChainThreads) {
-    const int i = e / lx, k = e - i * lx;
-    xb[e] = m0 + i < M && k < d.nin ? f2bf(x[(size_t)(m0 + i) * d.nin + k]) : (unsigned short)0;
+  // operands: x in BF16, eight values at a time, zeros in the padding that no product writes
+  for (int e = threadIdx.x; e < 2 * lx; e += nt) {
+    const int i = e / (lx >> 3), k0 = (e - i * (lx >> 3)) * 8;
+    const float* xr = x + (size_t)(m0 + i) * d.nin + k0;
+    v8u b{};
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (m0 + i < M && k0 + k < d.nin) b[k] = f2bf(xr[k]);
+    reinterpret_cast<v8u*>(xb)[e] = b;
   }
-  for (int e = threadIdx.x; e < 16 * (2 * lh + ly); e += kChainThreads) h1b[e] = 0;
+  for (int e = threadIdx.x; e < 2 * (2 * lh + ly); e += nt) reinterpret_cast<v8u*>(h1b)[e] = v8u{};
   __syncthreads();
-  if (t) {  // x over the rows, for dW1
-    for (int e = threadIdx.x; e < 16 * up16(d.nin); e += kChainThreads) {
+  if (kTrain) {  // x over the rows, for dW1
+    for (int e = threadIdx.x; e < 16 * up16(d.nin); e += nt) {
       const int k = e >> 4, i = e & 15;
       tape.x[frag_at(m0 + i, k, ms)] = xb[i * lx + k];
     }
@@ -348,16 +356,16 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int tile0, int M, i
         hf[(4 * g + q) * hc + j] = v[q];
         hb[(4 * g + q) * lh + j] = f2bf(v[q]);
       }
-      if (t) store_frag(frag, tn, ms, m0, v);
+      if (kTrain) store_frag(frag, tn, ms, m0, v);
     });
     __syncthreads();
   };
   hidden(xb, lx, ki, 0, w1, h1f, h1b, tape.h1);
   const ChainHeld w3 = chain_first(pk + d.f[2], kh, to);
   hidden(h1b, lh, kh, 1, w2, h2f, h2b, tape.h2);
-  const ChainHeld r3 = chain_first(pk + d.r[2], ko, t ? th : 0);
+  const ChainHeld r3 = chain_first(pk + d.r[2], ko, kTrain ? th : 0);
   double loss = 0.0;
-  float* cp = t ? tape.colpart + (size_t)tile * (2 * d.nh + d.nout) : nullptr;
+  float* cp = kTrain ? tape.colpart + (size_t)tile * (2 * d.nh + d.nout) : nullptr;
   {
     const float* b = p + d.b_off[2];
     chain_product(h2b, lh, pk + d.f[2], kh, to, w3, [&](int tn, v4f acc) {
@@ -370,23 +378,23 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int tile0, int M, i
         const bool in = i < M && j < d.nout;
         const float y = acc[q] + bj;
         v[q] = 0.f;
-        if (!t) {
+        if (!kTrain) {
           if (in) out[(size_t)i * d.nout + j] = y;
         } else if (in) {
           const float e = y - t[(size_t)i * d.nout + j];
           loss += (double)e * (double)e;
           v[q] = scale * e;
         }
-        dyb[(4 * g + q) * ly + j] = f2bf(v[q]);
+        if (kTrain) dyb[(4 * g + q) * ly + j] = f2bf(v[q]);
       }
-      if (t) {
+      if (kTrain) {
         store_frag(tape.dy, tn, ms, m0, v);
         const float s = tile_colsum(v);
         if (lane < 16 && j < d.nout) cp[2 * d.nh + j] = s;
       }
     });
   }
-  if (!t) return;  // uniform
+  if (!kTrain) return;
   const ChainHeld r2 = chain_first(pk + d.r[1], kh, th);
   __shared__ double ls[kChainWaves];
   for (int o = 32; o > 0; o >>= 1) loss += __shfl_down(loss, o);
@@ -394,7 +402,7 @@ __global__ __launch_bounds__(kChainThreads) void k_mlp_chain(int tile0, int M, i
   __syncthreads();
   if (threadIdx.x == 0) {
     double s = 0.0;
-    for (int w = 0; w < kChainWaves; ++w) s += ls[w];
+    for (int w = 0; w < nt >> 6; ++w) s += ls[w];
     tape.losspart[tile] = s;
   }
   // dz2 = (dy W3^T) * (1 - h2^2) into h1's operand, dz1 = (dz2 W2^T) * (1 - h1^2)
@@ -746,13 +754,17 @@ void Mlp::chain(hipStream_t s, int M, const float* x, const float* t, float* out
     tp.colpart = reinterpret_cast<float*>(tp.dy + m32 * up16(nout));
   }
   const double total = (double)M * nout;
+  const int th = up16(nh) / 16, to = up16(nout) / 16, ti = up16(nin) / 16;
+  int waves = t ? kChainWaves : std::min(kChainWaves, std::max(th, to));
+  // 16 waves fit a compute unit at these registers: many workgroups leave none of it idle
+  if (mt > 1024)
+    while (waves & (waves - 1)) waves &= waves - 1;
   constexpr int kMostTiles = 1 << 21;  // of 1024 threads: a launch takes less than 2^32
   for (int tile = 0; tile < mt; tile += kMostTiles)
-    hipLaunchKernelGGL(k_mlp_chain, dim3(std::min(kMostTiles, mt - tile)), dim3(kChainThreads), chain_lds(nin, nh, nout),
-                       s, tile, M, ms, d, params.as<const float>(), wpk.as<const unsigned short>(), x, t, out,
-                       2.0f / (float)((int64_t)M * nout), tp);
+    hipLaunchKernelGGL(t ? k_mlp_chain<true> : k_mlp_chain<false>, dim3(std::min(kMostTiles, mt - tile)), dim3(64 * waves),
+                       chain_lds(nin, nh, nout), s, tile, M, ms, d, params.as<const float>(),
+                       wpk.as<const unsigned short>(), x, t, out, 2.0f / (float)((int64_t)M * nout), tp);
   if (t) {
-    const int th = up16(nh) / 16, to = up16(nout) / 16, ti = up16(nin) / 16;
     const int grid = th * to + th * th + ti * th + (2 * nh + nout + 63) / 64 + 1;
     hipLaunchKernelGGL(k_mlp_wgrad, dim3(grid), dim3(256), 0, s, ms, mt, d, tp, grads.as<float>(), 1.0 / total,
                        loss_dev);
