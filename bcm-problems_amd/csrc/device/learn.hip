@@ -306,7 +306,7 @@ size_t chain_lds(int nin, int nh, int nout) {
 // loss against t, the activations' gradients and the tape. A forward pass has as
 // many waves as the widest layer has tiles, so that a small network leaves room
 // for other workgroups: 65536 rows through 1-1-1 took 80 us with 16 waves (13 as
-// separate products), 13 now; through 4-32-96 89 (54), 53 now.
+// separate products), 9 now; through 4-32-96 89 (54), 29 now.
 template <bool kTrain>
 __global__ __launch_bounds__(64 * kChainWaves) void k_mlp_chain(int tile0, int M, int ms, MlpDims d,
                                                                 const float* __restrict__ p,
@@ -773,7 +773,8 @@ void Mlp::chain(hipStream_t s, int M, const float* x, const float* t, float* out
 }
 
 void Mlp::forward(hipStream_t s, int M, const float* x, float* out) {
-  if (fused && out) {
+  if (fused) {
+    if (!out) throw Error(kErrArg, "mlp: the forward pass of a fused network needs an output");
     // A workgroup writes its rows of out while others still read x: where the
     // two share memory, x is read from a copy.
     const size_t nx = (size_t)M * nin, ny = (size_t)M * nout;
