@@ -573,7 +573,7 @@ class Context:
         _check(lib().bcm_context_set_sweep_mode(self.h, mode))
 
     def set_sweep_waves(self, waves_per_cu: int):
-        """Resident waves per CU of the sync-free sweeps (default 8)."""
+        """Accepted (1..64) and without effect."""
         _check(lib().bcm_context_set_sweep_waves(self.h, waves_per_cu))
 
     def raise_wait_flag(self):

@@ -734,8 +734,6 @@ int bcm_context_set_sweep_mode(bcm_context c, int mode) {
 int bcm_context_set_sweep_waves(bcm_context c, int waves_per_cu) {
   return guarded([&] {
     need(c != nullptr && waves_per_cu >= 1 && waves_per_cu <= 64, "context_set_sweep_waves: bad argument");
-    BCM_HIP(hipStreamSynchronize(c->c.stream));
-    c->c.sync.waves_per_cu = waves_per_cu;
   });
 }
 
@@ -743,7 +741,7 @@ int bcm_context_raise_wait_flag(bcm_context c) {
   return guarded([&] {
     need(c != nullptr, "context_raise_wait_flag: null handle");
     bcm::Context& x = c->c;
-    x.sync.ensure(0, x.stream);
+    x.sync.ensure(x.stream);
     const int one = 1;
     bcm::SetupGuard g;
     BCM_HIP(hipMemcpyAsync(x.sync.ctl.as<int>() + 2, &one, sizeof(int), hipMemcpyHostToDevice, x.stream));

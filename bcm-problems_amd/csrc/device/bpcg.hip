@@ -597,7 +597,7 @@ void iteration(Batch& bt, Context& ctx, const BWork& w, const SolveOptions& opt,
 struct BatchGraph {
   hipGraph_t g = nullptr;
   hipGraphExec_t exec = nullptr;
-  int nrhs = 0, prec = -1, iters = 0, sweep_mode = -1, waves = 0, order = -1, flex = 0, niter = 0, ittype = -1;
+  int nrhs = 0, prec = -1, iters = 0, sweep_mode = -1, order = -1, flex = 0, niter = 0, ittype = -1;
   double eps = 0.0;
   std::vector<const void*> key;  // device buffers the captured launches use
   ~BatchGraph() {
@@ -731,18 +731,15 @@ void solve_nr(Batch& bt, Context& ctx, const SolveOptions& opt, const double* b,
   const double eps2 = opt.eps * opt.eps;
   const BatchTune& tu = bt.tune;
   const int saved_mode = ctx.sweep_mode;
-  const int saved_waves = ctx.sync.waves_per_cu;
   const bool saved_order = ctx.sync.level_order;
   ctx.sweep_mode = tu.sweep_mode;
-  ctx.sync.waves_per_cu = tu.waves_per_cu;
   ctx.sync.level_order = tu.level_order != 0;
   auto restore = [&] {
     ctx.sweep_mode = saved_mode;
-    ctx.sync.waves_per_cu = saved_waves;
     ctx.sync.level_order = saved_order;
   };
   try {
-    ctx.sync.ensure(im.fwd.nsup, s);
+    ctx.sync.ensure(s);
     ctx.rw.ensure();
     hipLaunchKernelGGL(k_copy_vec, dim3(grid_vec(nn)), dim3(256), 0, s, nn, b, w.b);
     hipLaunchKernelGGL(k_copy_vec, dim3(grid_vec(nn)), dim3(256), 0, s, nn, (const double*)x, w.x);
@@ -783,8 +780,7 @@ void solve_nr(Batch& bt, Context& ctx, const SolveOptions& opt, const double* b,
       }
       BatchGraph* g = bt.graph.get();
       const bool valid = g && g->nrhs == NR && g->prec == opt.prec && g->iters == every &&
-                         g->sweep_mode == tu.sweep_mode && g->waves == tu.waves_per_cu &&
-                         g->order == tu.level_order && g->flex == flex &&
+                         g->sweep_mode == tu.sweep_mode && g->order == tu.level_order && g->flex == flex &&
                          g->niter == opt.niter && g->ittype == opt.ittype && g->eps == opt.eps && g->key == key;
       if (!valid) {
         bt.graph.reset(new BatchGraph());
@@ -802,7 +798,7 @@ void solve_nr(Batch& bt, Context& ctx, const SolveOptions& opt, const double* b,
         BCM_HIP(hipStreamEndCapture(s, &g->g));
         BCM_HIP(hipGraphInstantiate(&g->exec, g->g, nullptr, nullptr, 0));
         g->nrhs = NR; g->prec = opt.prec; g->iters = every; g->sweep_mode = tu.sweep_mode;
-        g->waves = tu.waves_per_cu; g->order = tu.level_order; g->flex = flex; g->niter = opt.niter; g->ittype = opt.ittype; g->eps = opt.eps;
+        g->order = tu.level_order; g->flex = flex; g->niter = opt.niter; g->ittype = opt.ittype; g->eps = opt.eps;
         g->key = key;
       }
     }

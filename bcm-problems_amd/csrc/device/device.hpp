@@ -163,10 +163,8 @@ void dev_tri_backward_parts(const std::vector<const BlockCsr*>& f, int prec, Dev
 struct SweepSync {
   DevBuf ctl;
   int* ext_ctl = nullptr;  // caller-provided control words (at least 16 ints, zeroed) used instead of ctl
-  int nsup = 0;
-  int waves_per_cu = 8;     // accepted bound on the resident waves per CU
   bool level_order = true;  // process rows sorted by dependency level (false: natural sweep order)
-  void ensure(int nsup, hipStream_t s);
+  void ensure(hipStream_t s);
   int error(hipStream_t s);
   void clear(hipStream_t s);  // resets the wait-bound error flag
 };

@@ -2444,12 +2444,11 @@ void dev_tri_backward_parts(const std::vector<const BlockCsr*>& f, int prec, Dev
   build_tri_parts(f, false, prec, t);
 }
 
-void SweepSync::ensure(int n, hipStream_t s) {
+void SweepSync::ensure(hipStream_t s) {
   if (ext_ctl || ctl.p) return;
   ctl.alloc(64);
   BCM_HIP(hipMemsetAsync(ctl.p, 0, 64, s));
   BCM_HIP(hipStreamSynchronize(s));
-  nsup = n;
 }
 
 void SweepSync::clear(hipStream_t s) {
@@ -2878,7 +2877,7 @@ static void sweep_cx(const SweepLaunch& l, int nrhs) {
 
 static void sweep_dispatch(const SweepLaunch& l, int vec_prec, int nrhs, RowGate gate) {
   const DevTri& T = *l.T1;
-  if (l.sync) l.sync->ensure(T.nsup, l.s);
+  if (l.sync) l.sync->ensure(l.s);
   if (T.b == 0) {
     if (T.prec == kF64 && vec_prec == kF64) sweep_free_var<double, double>(l, nrhs);
     else if (T.prec == kF32 && vec_prec == kF32) sweep_free_var<float, float>(l, nrhs);

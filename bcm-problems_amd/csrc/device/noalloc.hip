@@ -78,7 +78,6 @@ void precond_noalloc(Factor& F, Context& ctx, const double* r, double* z, int pr
   SweepSync local;
   SweepSync* sync = nullptr;
   if (const SweepSync* cs = ctx.sweep_sync()) {
-    local.waves_per_cu = cs->waves_per_cu;
     local.level_order = cs->level_order;
     local.ext_ctl = reinterpret_cast<int*>(ctl);
     hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, s, local.ext_ctl, (int)(kCtlBytes / 4));

@@ -233,8 +233,9 @@ int bcm_context_sync(bcm_context c);
  * the rows they depend on; 2 = as 1 over the natural sweep order. The schedules agree to rounding: per row they add
  * the same products, grouped differently across lanes for some block sizes. */
 int bcm_context_set_sweep_mode(bcm_context c, int mode);
-/* Resident waves per CU asked of the sync-free sweeps (1..64, default 8).
- * A hint without effect on results; the present kernels take what fits. */
+/* Resident waves per CU asked of the sync-free sweeps (1..64). Accepted and
+ * without effect: a sweep's waves take their rows as they start, so it needs no
+ * bound, and one did not make it faster. */
 int bcm_context_set_sweep_waves(bcm_context c, int waves_per_cu);
 /* Test hook: marks the sync-free sweeps' dependency wait as having reached its
  * bound, so that every wait of the next solve exits at once and the solve
@@ -319,7 +320,7 @@ typedef struct bcm_batch_stats {
 } bcm_batch_stats;
 typedef struct bcm_batch_tune {
   int sweep_mode;    /* 0 level-scheduled sweeps, 1 sync-free sweeps */
-  int waves_per_cu;  /* sync-free sweeps: resident waves per CU (hint) */
+  int waves_per_cu;  /* returned as set, without effect */
   int level_order;   /* sync-free sweeps: 1 rows in dependency-level order, 0 natural order */
   int graph;         /* 1: replay check_every iterations as one captured hipGraph */
   int check_every;   /* iterations between host polls */

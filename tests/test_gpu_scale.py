@@ -98,17 +98,21 @@ def cell16(B, O):
 
 @pytest.mark.parametrize("waves", [1, 8])
 def test_pcg_16cube_cell_waves_own_several_rows(B, O, cell16, waves):
-    """A 16^3 elasticity cell (4096 block rows of 24): with 1 or 8 resident
-    waves per CU every wave of the sync-free sweeps owns several rows in
-    turn (16 or 2); same iterations and solution as the oracle's Cg."""
+    """A 16^3 elasticity cell (4096 block rows of 24, more than the waves that
+    are resident at a time): same iterations and solution as the oracle's Cg.
+    The waves asked for are accepted and have no effect: bit for bit the
+    solution of another context with another number."""
     c = cell16
-    ctx = B.Context()
+    ctx, other = B.Context(), B.Context()
     ctx.set_sweep_waves(waves)
+    other.set_sweep_waves(64)
     print(f"pcg 16^3 waves_per_cu={waves} n={c['A'].n}", flush=True)
     x, st = solve(B, ctx, c["mo"], c["f"], c["b"][:, 0], kind=B.PCG, eps=1e-10, ittype=3)
     xo, r = O.cg(c["A"], c["U"], c["b"][:, 0], eps=1e-10, ittype=3)
     assert st.converged == 1 and st.iterations == r.updates
     assert rel(x, xo) < 1e-8 and st.relres_true <= 1e-10
+    y, _ = solve(B, other, c["mo"], c["f"], c["b"][:, 0], kind=B.PCG, eps=1e-10, ittype=3)
+    assert np.array_equal(x, y)
 
 
 def test_wait_bound_recovery_returns_the_solution(B, O, cell16):
