@@ -436,8 +436,10 @@ __global__ __launch_bounds__(64 * kChainWaves) void k_mlp_chain(int tile0, int M
 
 // Gradients from the tape. Workgroups [0, ntile): one 16 x 16 tile of dW3 =
 // H2^T dY, dW2 = H1^T dZ2 or dW1 = X^T dZ1, its rows of the batch split over
-// the four waves and added in order (1 KB operands a load, all from L2). Then
-// ones of 64 columns of the bias gradients, and one for the loss.
+// the four waves and added in order (1 KB operands a load, all from L2), 1024
+// rows of a wave at a time, so that the FP32 sums of long batches stay short. Then
+// ones of 64 columns of the bias gradients (tiles of 16 rows, added in FP64), and
+// one for the loss.
 __global__ __launch_bounds__(256) void k_mlp_wgrad(int ms, int mt, MlpDims d, MlpTape tape, float* __restrict__ grad,
                                                    double loss_scale, double* loss) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -454,13 +456,18 @@ __global__ __launch_bounds__(256) void k_mlp_wgrad(int ms, int mt, MlpDims d, Ml
     const int bi = b / tj, bj = b - bi * tj;
     const v8u* ap = reinterpret_cast<const v8u*>(A + (size_t)bi * ms * kFrag) + lane;
     const v8u* bp = reinterpret_cast<const v8u*>(Bm + (size_t)bj * ms * kFrag) + lane;
-    v4f acc = {0.f, 0.f, 0.f, 0.f};
+    v4f sum = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = wave; k0 < ms; k0 += 4 * 32) {
+      v4f acc = {0.f, 0.f, 0.f, 0.f};
+      const int k1 = min(ms, k0 + 4 * 32);
 #pragma unroll 8
-    for (int k = wave; k < ms; k += 4)
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, ap[(size_t)k * 64]),
-                                                    __builtin_bit_cast(v8bf, bp[(size_t)k * 64]), acc, 0, 0, 0);
+      for (int k = k0; k < k1; k += 4)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, ap[(size_t)k * 64]),
+                                                      __builtin_bit_cast(v8bf, bp[(size_t)k * 64]), acc, 0, 0, 0);
+      sum += acc;
+    }
 #pragma unroll
-    for (int q = 0; q < 4; ++q) part[wave][(4 * (lane >> 4) + q) * 16 + (lane & 15)] = acc[q];
+    for (int q = 0; q < 4; ++q) part[wave][(4 * (lane >> 4) + q) * 16 + (lane & 15)] = sum[q];
     __syncthreads();
     const int e = threadIdx.x, i = bi * 16 + (e >> 4), j = bj * 16 + (e & 15);
     if (i < ni && j < nj)
@@ -470,16 +477,17 @@ __global__ __launch_bounds__(256) void k_mlp_wgrad(int ms, int mt, MlpDims d, Ml
   b -= n3 + n2 + n1;
   const int ncol = 2 * d.nh + d.nout, nb = (ncol + 63) / 64;
   if (b < nb) {
-    __shared__ float sm[4][64];
+    __shared__ double sm[4][64];
     const int c = b * 64 + lane;
-    float s = 0.f;
+    double s = 0.0;
     if (c < ncol)
-      for (int k = wave; k < mt; k += 4) s += tape.colpart[(size_t)k * ncol + c];
+#pragma unroll 8
+      for (int k = wave; k < mt; k += 4) s += (double)tape.colpart[(size_t)k * ncol + c];
     sm[wave][lane] = s;
     __syncthreads();
     if (wave == 0 && c < ncol) {
       const int64_t o = c < d.nh ? d.b_off[0] + c : c < 2 * d.nh ? d.b_off[1] + c - d.nh : d.b_off[2] + c - 2 * d.nh;
-      grad[o] = ((sm[0][lane] + sm[1][lane]) + sm[2][lane]) + sm[3][lane];
+      grad[o] = (float)(((sm[0][lane] + sm[1][lane]) + sm[2][lane]) + sm[3][lane]);
     }
     return;
   }

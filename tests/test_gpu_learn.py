@@ -220,3 +220,27 @@ def test_mlp_more_rows_than_a_launch(B, ctx):
     y = m.forward(ctx, x)
     for k in range(0, rows, len(part)):  # a row's result does not depend on where it stands
         assert np.array_equal(y[k:k + len(part)], want[:min(len(part), rows - k)]), k
+
+
+def test_mlp_gradients_of_long_batches(B, ctx):
+    """262144 rows: sums of a batch in FP32 from end to end would be off by some
+    5e-7. Biases: 16 rows in FP32, then FP64, a few 2^-24. Weights: 32 steps of 32
+    rows, then 64 such sums, each a random walk of 2^-25; what layers 1 and 2 add
+    to it are gradients that round to the other BF16 neighbour."""
+    dims, batch = (4, 16, 16), 262144
+    rng = np.random.default_rng(3)
+    offs, npar = M.layout(*dims)
+    p = (rng.normal(size=npar) / 4.0).astype(np.float32)
+    x = rng.normal(size=(batch, dims[0])).astype(np.float32)
+    t = (rng.normal(size=(batch, dims[2])) + 0.3).astype(np.float32)
+    print(f"mlp {dims} batch {batch}", flush=True)
+    m = B.Mlp(*dims)
+    m.set_params(p)
+    m.backward(ctx, x, t)
+    g = m.grads().astype(np.float64)
+    _, go = M.loss_grad(p.astype(np.float64), x.astype(np.float64), t.astype(np.float64), *dims, bf16=True)
+    for name, (o, shp), tol in zip(["W1", "b1", "W2", "b2", "W3", "b3"], offs, [1e-6, 2e-7, 5e-7, 2e-7, 4e-7, 2e-7]):
+        k = int(np.prod(shp))
+        e = relerr(g[o:o + k], go[o:o + k])
+        print(f"{name} {e:.1e}", flush=True)
+        assert e < tol, name
