@@ -215,7 +215,8 @@ void launch_spmv(const DevBsr& A, const double* x, double* y, const double* bsub
 
 // Triangular sweep y = T^-1 x for the given precision of vectors (TX). With
 // sync == nullptr: one launch per dependency level; otherwise one sync-free
-// launch using `sync`. x and y must not alias.
+// launch using `sync` (or by levels where those are the faster, or a column's
+// rows do not fit a launch). x and y must not alias.
 void launch_sweep(const DevTri& T, const void* x, void* y, int vec_prec, int nrhs, hipStream_t s,
                   const int* skip = nullptr, SweepSync* sync = nullptr, RowGate gate = RowGate());
 

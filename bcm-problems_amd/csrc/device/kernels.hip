@@ -663,7 +663,7 @@ __global__ __launch_bounds__(256) void k_sweep_level(int nrows, const int* __res
 // sorted by dependency level, which interleaves independent chains (e.g. the
 // cells of a block-diagonal union); the positions of the second sweep follow
 // those of the first. A workgroup draws one ticket when it starts and its
-// kSweepWaves waves process kSweepWaves consecutive positions, one each.
+// waves (kSweepWaves, or twice as many) process consecutive positions, one each.
 // Tickets are drawn in position order by workgroups that already run, so the
 // smallest unfinished position always belongs to a running wave whose
 // dependencies are complete: the sweep ends whatever else occupies the GPU and
@@ -742,7 +742,7 @@ struct SweepDir {
 
 // A sweep launch: `phases` sweeps (1 or 2) over npos = nsup * ng positions
 // each; position p is block row p / ng (in the order of its direction) and
-// column p % ng. Phase 0 reads x (doubles if x64, else
+// column p % ng, or group of NR columns. Phase 0 reads x (doubles if x64, else
 // vector values) and writes y0; phase 1 reads y0 and writes y1, and out (as
 // doubles) if given.
 template <class TX>
@@ -1137,7 +1137,7 @@ __global__ __launch_bounds__(64 * W) void k_sweep_free_cx(SweepJob<double> jb) {
 // Four lanes share a row of the block (lane = 4 r + g, g taking the columns g, g
 // + 4, ...), so that a row's sum is two swaps within registers. With the layout
 // of k_sweep_free, whose sums cross the wave through LDS, both sweeps of 64 x 64
-// heat, block 9, took 264 us (now 244), of 20 x 19 x 18 x block 12 167 (120), of
+// heat, block 9, took 264 us (with this one 244), of 20 x 19 x 18 x block 12 167 (120), of
 // 16^3 x block 16 120 (105).
 
 template <class T> __device__ __forceinline__ T ld_wg(const T* p) {

@@ -230,8 +230,10 @@ int bcm_context_sync(bcm_context c);
 /* Triangular sweep schedule: 0 = one launch per dependency level;
  * 1 = one sync-free launch per sweep, or per pair of sweeps (default): waves
  * take the rows in dependency-level order and wait (bounded) on the values of
- * the rows they depend on; 2 = as 1 over the natural sweep order. The schedules agree to rounding: per row they add
- * the same products, grouped differently across lanes for some block sizes. */
+ * the rows they depend on (blocks above 16 with levels as wide as to be bound
+ * by memory: as 0); 2 = as 1 over the natural sweep order. The schedules agree to
+ * rounding: per row they add the same products, grouped differently across lanes
+ * for some block sizes. */
 int bcm_context_set_sweep_mode(bcm_context c, int mode);
 /* Resident waves per CU asked of the sync-free sweeps (1..64). Accepted and
  * without effect: a sweep's waves take their rows as they start, so it needs no
