@@ -933,7 +933,7 @@ BatchTune batch_tune(Batch& bt, Context& ctx, const SolveOptions& opt, int nrhs,
     t.sweep_mode = 0;
     stage1.push_back(t);
     t.sweep_mode = 1;
-    for (int order = 0; order <= 1; ++order) {
+    for (int order = 0; order <= 1 && sweep_free_taken(bt.img[opt.prec].fwd, nrhs); ++order) {
       t.level_order = order;
       stage1.push_back(t);
     }

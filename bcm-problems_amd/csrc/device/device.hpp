@@ -213,10 +213,13 @@ void launch_spmv(const DevBsr& A, const double* x, double* y, const double* bsub
                  double* dot_out, const double* wdot, RedWork& rw, hipStream_t s, const int* skip = nullptr,
                  RowGate gate = RowGate());
 
+// Whether sweeps of nrhs columns over T given a SweepSync take the sync-free
+// kernels; else they go level by level all the same.
+bool sweep_free_taken(const DevTri& T, int nrhs);
+
 // Triangular sweep y = T^-1 x for the given precision of vectors (TX). With
 // sync == nullptr: one launch per dependency level; otherwise one sync-free
-// launch using `sync` (or by levels where those are the faster, or a column's
-// rows do not fit a launch). x and y must not alias.
+// launch using `sync` (sweep_free_taken). x and y must not alias.
 void launch_sweep(const DevTri& T, const void* x, void* y, int vec_prec, int nrhs, hipStream_t s,
                   const int* skip = nullptr, SweepSync* sync = nullptr, RowGate gate = RowGate());
 

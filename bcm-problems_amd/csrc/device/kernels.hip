@@ -2634,14 +2634,13 @@ static int64_t sweep_width(const DevTri& T, int64_t ncol) { return T.levels > 0 
 constexpr int64_t kLaunchThreads = (1LL << 32) - 1;                      // most threads of a launch
 constexpr int64_t kMostPositions = kLaunchThreads / 64 - 2 * kSweepWaves;  // one wave each
 
-// Whether nrhs columns of a factor's sweeps, both in one launch, take the
-// sync-free kernels: where a column's positions fit a launch, any block partition
-// has its column list, and with large blocks levels are not as wide as to be
-// bound by memory alone, where one launch per level, all columns of a row on one
-// wave, reads the least. (Cells of block 24, six columns, FP32, ms for 55 steps,
+// Where a column's positions fit a launch, any block partition has its column
+// list, and with large blocks levels are not as wide as to be bound by memory
+// alone, where one launch per level, all columns of a row on one wave, reads the
+// least. (Cells of block 24, six columns, FP32, ms for 55 steps,
 // sync-free and by levels: 16 cells, 5760 rows and columns a level, 45.6 and 45.5; 40
 // cells 93 and 70.)
-static bool sweep_listed(const DevTri& T, int nrhs) {
+bool sweep_free_taken(const DevTri& T, int nrhs) {
   if (T.b > kStripBlock && !T.cplx && sweep_width(T, nrhs) > 6144) return false;
   return 2LL * T.nsup <= kMostPositions && (T.b || T.cptr.p);
 }
@@ -2916,7 +2915,7 @@ void launch_sweep(const DevTri& T, const void* x, void* y, int vec_prec, int nrh
                   const int* skip, SweepSync* sync, RowGate gate) {
   if (x == y) throw Error(kErrArg, "triangular sweep: input and output must not alias");
   if (T.b == 0 && gate.active) throw Error(kErrArg, "row-gated sweeps need a uniform tuned block size");
-  if (!sweep_listed(T, nrhs)) sync = nullptr;  // level by level
+  if (!sweep_free_taken(T, nrhs)) sync = nullptr;  // level by level
   if (T.b == 0 && !sync) {
     launch_sweep_var(T, x, y, vec_prec, nrhs, s, skip);
     return;
@@ -2930,7 +2929,7 @@ void launch_sweep_pair(const DevTri& T1, const DevTri& T2, const double* r, doub
   const char *rb = reinterpret_cast<const char*>(r), *zb = reinterpret_cast<const char*>(z);
   const bool apart = rb + vb <= zb || zb + vb <= rb;
   // In one launch z is filled before r is read and written while it still is.
-  if (sync && sweep_listed(T1, nrhs) && sweep_listed(T2, nrhs) && T1.b == T2.b && T1.nsup == T2.nsup && T1.cplx == T2.cplx && T1.prec == T2.prec &&
+  if (sync && sweep_free_taken(T1, nrhs) && sweep_free_taken(T2, nrhs) && T1.b == T2.b && T1.nsup == T2.nsup && T1.cplx == T2.cplx && T1.prec == T2.prec &&
       apart) {
     void* y1 = vec_prec == kF64 ? static_cast<void*>(z) : w1;
     double* out = vec_prec == kF64 ? nullptr : z;

@@ -217,6 +217,27 @@ def test_batch_autotune_and_errors(B, ctx, batch, cells):
         batch.solve(ctx, db, dx, B.default_opts(kind=B.BLOCKPCG), 2)
 
 
+def test_batch_of_wide_levels_goes_by_levels(B, O, ctx):
+    """20 cells of 10^3 x 6 columns: 7500 rows and columns an average level, which
+    both schedules process level by level; the tuner then tries no other."""
+    c = cell(B, O, 10, 7)
+    bt = B.Batch([(c["mo"], c["f"])] * 20, prec_mask=0b011)
+    db = B.DeviceArray.from_host(bt.gather([c["b"]] * 20))
+    print(f"wide batch n={bt.n}", flush=True)
+    for precision in (B.F64, B.F32):
+        opts = B.default_opts(kind=B.BLOCKPCG, eps=1e-10, precision=precision)
+        out = []
+        for mode in (0, 1):
+            bt.set_tune(sweep_mode=mode, graph=0, check_every=4, waves_per_cu=8, level_order=1)
+            dx = B.DeviceArray((bt.n, 6))
+            dx.zero()
+            st, its, rr = bt.solve(ctx, db, dx, opts, 6)
+            assert st.converged == st.pairs
+            out.append(dx.host())
+        assert np.array_equal(out[0], out[1])
+        assert bt.autotune(ctx, db, opts, 6).sweep_mode == 0
+
+
 def test_batch_galerkin_start(B, ctx, batch, cells, oracle_sol):
     """Start flag 2: each cell's six guesses X become X C with
     (X^T A X) C = X^T B. With niter = 0 the solve returns the start: it equals
