@@ -806,7 +806,8 @@ __device__ __forceinline__ bool wait_over(int polls, uint64_t& since, uint64_t b
 }
 
 // Stages nd (<= KM) dependency blocks of a row (block rows cols[0..nd) of y,
-// NR columns of leading dimension n) into s[((1 + k) * B + c) * NR + q], and with row >= 0 the row's right-hand side into block 0 of s: x (already a
+// NR columns of leading dimension n) into s[((1 + k) * B + c) * NR + q], and
+// with row >= 0 the row's right-hand side into block 0 of s: x (already a
 // complete vector; doubles if x64) or, when xw is given, the row of xw, waited
 // for like a dependency. Blocks nd .. npad-1 are zero-filled. Each value is
 // loaded once, by one of the 64 lanes, and the lanes re-poll the values still
@@ -2737,8 +2738,8 @@ static void sweep_launch(void (*kern)(SweepJob<TX>), const SweepLaunch& l, int f
     jb.y1 = l.T2 ? static_cast<TX*>(l.y1) + o : nullptr;
     jb.out = l.out ? l.out + o : nullptr;
     const int64_t ny = (int64_t)T.n * jb.ng * nr;
-    hipLaunchKernelGGL((k_sweep_fill<TX>), dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((ny + 255) / 256, 2048))),
-                       dim3(256), 0, l.s, ny, jb.y0, jb.y1, jb.ctl, l.skip);
+    const int fill = (int)std::max<int64_t>(1, std::min<int64_t>((ny + 255) / 256, 2048));
+    hipLaunchKernelGGL((k_sweep_fill<TX>), dim3(fill), dim3(256), 0, l.s, ny, jb.y0, jb.y1, jb.ctl, l.skip);
     if (strip) {
       jb.npos = T.strips * jb.ng;
       const int rows = std::max(T.strip_rows_max, l.T2 ? l.T2->strip_rows_max : 0);
@@ -2929,8 +2930,8 @@ void launch_sweep_pair(const DevTri& T1, const DevTri& T2, const double* r, doub
   const char *rb = reinterpret_cast<const char*>(r), *zb = reinterpret_cast<const char*>(z);
   const bool apart = rb + vb <= zb || zb + vb <= rb;
   // In one launch z is filled before r is read and written while it still is.
-  if (sync && sweep_free_taken(T1, nrhs) && sweep_free_taken(T2, nrhs) && T1.b == T2.b && T1.nsup == T2.nsup && T1.cplx == T2.cplx && T1.prec == T2.prec &&
-      apart) {
+  if (sync && sweep_free_taken(T1, nrhs) && sweep_free_taken(T2, nrhs) && T1.b == T2.b && T1.nsup == T2.nsup &&
+      T1.cplx == T2.cplx && T1.prec == T2.prec && apart) {
     void* y1 = vec_prec == kF64 ? static_cast<void*>(z) : w1;
     double* out = vec_prec == kF64 ? nullptr : z;
     sweep_dispatch({&T1, &T2, r, kF64, w0, y1, out, s, skip, sync}, vec_prec, nrhs, RowGate());
